@@ -108,6 +108,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
 
     if (hipStreamSynchronize(L->stream) != hipSuccess) rc = fail(LCEQ_ERR_HIP, "init sync failed");
   }
+  transfer_user(1);
   if (rc != LCEQ_OK) {
     lceq_destroy(L);
     return rc;
@@ -129,6 +130,7 @@ extern "C" int lceq_destroy(lceq_lattice* L) {
   }
   if (L->stream) (void)hipStreamDestroy(L->stream);
   delete L;
+  transfer_user(-1);
   return LCEQ_OK;
 }
 
@@ -517,33 +519,17 @@ static int ensure_scratch(lceq_lattice* L, size_t bytes) {
 static int put_field(lceq_lattice* L, double* dev, const double* host, int64_t ld, int ncomp,
                      int nclass) {
   NEEDL(L);
-  const Geom& g = L->g;
-  if (!host || ld < g.n) return fail(LCEQ_ERR_ARG, "bad host array or ld < N");
-  std::vector<double> st((size_t)nclass * ncomp * g.npad, 0.0);
-  for (int cls = 0; cls < nclass; ++cls)
-    for (int s = 0; s < g.n; ++s)
-      for (int c = 0; c < ncomp; ++c)
-        st[field_offset(ncomp, cls, c, s, g.npad)] = host[((size_t)cls * ld + s) * ncomp + c];
-  HIPCHK(hipMemcpyAsync(dev, st.data(), st.size() * sizeof(double), hipMemcpyHostToDevice,
-                        L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
-  return LCEQ_OK;
+  if (!host || ld < L->g.n) return fail(LCEQ_ERR_ARG, "bad host array or ld < N");
+  return transfer_field(L->stream, L->device, L->g, dev, const_cast<double*>(host), ld, ncomp,
+                        nclass, false);
 }
 
 static int get_field(lceq_lattice* L, const double* dev, double* host, int64_t ld, int ncomp,
                      int nclass) {
   NEEDL(L);
-  const Geom& g = L->g;
-  if (!host || ld < g.n) return fail(LCEQ_ERR_ARG, "bad host array or ld < N");
-  std::vector<double> st((size_t)nclass * ncomp * g.npad);
-  HIPCHK(hipMemcpyAsync(st.data(), dev, st.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
-  for (int cls = 0; cls < nclass; ++cls)
-    for (int s = 0; s < g.n; ++s)
-      for (int c = 0; c < ncomp; ++c)
-        host[((size_t)cls * ld + s) * ncomp + c] = st[field_offset(ncomp, cls, c, s, g.npad)];
-  return LCEQ_OK;
+  if (!host || ld < L->g.n) return fail(LCEQ_ERR_ARG, "bad host array or ld < N");
+  return transfer_field(L->stream, L->device, L->g, const_cast<double*>(dev), host, ld, ncomp,
+                        nclass, true);
 }
 
 extern "C" int lceq_put_links(lceq_lattice* L, const double* u, int64_t ld) {

@@ -272,6 +272,7 @@ struct ReplicaGroup {
 
 struct lceq_batch {
   int nrep;
+  int device;
   std::vector<Replica> reps;  // host copy of the device table
   std::vector<int64_t> field_off;
   Replica* d_reps;
@@ -425,7 +426,9 @@ extern "C" int lceq_batch_create(int nrep, const int* dims, lceq_batch** out) {
     if (rc) return;
     if (hipMalloc(p, bytes) != hipSuccess) rc = bfail(LCEQ_ERR_HIP, "hipMalloc(%zu) failed", bytes);
   };
-  if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess)
+  transfer_user(1);
+  if (hipGetDevice(&B->device) != hipSuccess) rc = bfail(LCEQ_ERR_HIP, "no HIP device");
+  if (!rc && hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess)
     rc = bfail(LCEQ_ERR_HIP, "hipStreamCreate failed");
   alloc((void**)&B->pool, pool * sizeof(double));
   alloc((void**)&B->parts, parts * sizeof(double));
@@ -476,6 +479,7 @@ extern "C" int lceq_batch_destroy(lceq_batch* B) {
     if (p) (void)hipFree(p);
   if (B->stream) (void)hipStreamDestroy(B->stream);
   delete B;
+  transfer_user(-1);
   return LCEQ_OK;
 }
 
@@ -529,27 +533,10 @@ static int batch_field(lceq_batch* B, int r, double* host, const double* hin, in
   if (!B || r < 0 || r >= B->nrep) return bfail(LCEQ_ERR_ARG, "bad replica index");
   const Replica& R = B->reps[r];
   if (ld < R.g.n) return bfail(LCEQ_ERR_ARG, "ld < N");
-  int ncomp = links ? 4 : 3, nclass = links ? 6 : 2;
-  double* dev = links ? R.U : R.A;
-  std::vector<double> st((size_t)nclass * ncomp * R.g.npad, 0.0);
-  if (hin) {
-    for (int cls = 0; cls < nclass; ++cls)
-      for (int s = 0; s < R.g.n; ++s)
-        for (int c = 0; c < ncomp; ++c)
-          st[field_offset(ncomp, cls, c, s, R.g.npad)] = hin[((size_t)cls * ld + s) * ncomp + c];
-    BHIP(hipMemcpyAsync(dev, st.data(), st.size() * sizeof(double), hipMemcpyHostToDevice,
-                        B->stream));
-    BHIP(hipStreamSynchronize(B->stream));
-  } else {
-    BHIP(hipMemcpyAsync(st.data(), dev, st.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        B->stream));
-    BHIP(hipStreamSynchronize(B->stream));
-    for (int cls = 0; cls < nclass; ++cls)
-      for (int s = 0; s < R.g.n; ++s)
-        for (int c = 0; c < ncomp; ++c)
-          host[((size_t)cls * ld + s) * ncomp + c] = st[field_offset(ncomp, cls, c, s, R.g.npad)];
-  }
-  return LCEQ_OK;
+  if (!host && !hin) return bfail(LCEQ_ERR_ARG, "null field array");
+  return transfer_field(B->stream, B->device, R.g, links ? R.U : R.A,
+                        hin ? const_cast<double*>(hin) : host, ld, links ? 4 : 3, links ? 6 : 2,
+                        !hin);
 }
 extern "C" int lceq_batch_put_links(lceq_batch* B, int r, const double* u, int64_t ld) {
   return batch_field(B, r, nullptr, u, ld, 1);
@@ -743,11 +730,13 @@ extern "C" int lceq_batch_history(lceq_batch* B, double* out, int n) {
     return bfail(LCEQ_ERR_ARG, "bad history request");
   BHIP(hipStreamSynchronize(B->stream));
   size_t row = (size_t)B->nrep * LCEQ_OBS_N;
-  std::vector<double> h((size_t)B->hist_cap * row);
-  BHIP(hipMemcpy(h.data(), B->hist, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < n; ++k) {
-    uint64_t sw = B->sweeps_done - n + k;
-    memcpy(out + k * row, h.data() + (sw % B->hist_cap) * row, row * sizeof(double));
+  // the rows asked for, in one or two runs of the ring
+  for (int k = 0; k < n;) {
+    size_t at = (size_t)((B->sweeps_done - n + k) % (uint64_t)B->hist_cap);
+    int run = std::min(n - k, B->hist_cap - (int)at);
+    BHIP(hipMemcpy(out + k * row, B->hist + at * row, run * row * sizeof(double),
+                   hipMemcpyDeviceToHost));
+    k += run;
   }
   return LCEQ_OK;
 }

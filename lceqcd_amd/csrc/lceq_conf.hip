@@ -13,6 +13,7 @@
 // its values into the first half of each record (real_bytes = 4).
 #include <stdint.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <cmath>
@@ -63,18 +64,23 @@ int field_io(bool write, const ConfGeom& g, double* host, int ncomp, int nclass,
                              what, path, size, g.lx, g.ly, g.lz, (long long)need);
     }
   }
-  std::vector<unsigned char> rec((size_t)recl, 0);
+  // full records (8-byte reals) are the host array itself and follow one
+  // another in the file: read and written in place, without the record buffer
+  std::vector<unsigned char> rec(rb == 8 ? 0 : (size_t)recl, 0);
   for (int cls = 0; cls < nclass && rc == LCEQ_OK; ++cls)
     for (int z = 0; z < g.lz; ++z) {
       double* base = host + ((size_t)cls * g.n + (size_t)z * g.h2) * ncomp;
-      if (write) {
+      if (rb == 8) {
+        if (write && fwrite(base, 1, (size_t)recl, f) != (size_t)recl)
+          rc = lceq::set_error(LCEQ_ERR_IO, "short write to %s", path);
+        if (!write && fread(base, 1, (size_t)recl, f) != (size_t)recl) {
+          rc = lceq::set_error(LCEQ_ERR_IO, "short read from %s", path);
+          break;
+        }
+      } else if (write) {
         for (int64_t i = 0; i < g.h2 * ncomp; ++i) {
-          if (rb == 8) {
-            memcpy(&rec[(size_t)i * 8], &base[i], 8);
-          } else {
-            float v = (float)base[i];
-            memcpy(&rec[(size_t)i * 4], &v, 4);
-          }
+          float v = (float)base[i];
+          memcpy(&rec[(size_t)i * 4], &v, 4);
         }
         if (fwrite(rec.data(), 1, (size_t)recl, f) != (size_t)recl)
           rc = lceq::set_error(LCEQ_ERR_IO, "short write to %s", path);
@@ -85,13 +91,9 @@ int field_io(bool write, const ConfGeom& g, double* host, int ncomp, int nclass,
           break;
         }
         for (int64_t i = 0; i < g.h2 * ncomp; ++i) {
-          if (rb == 8) {
-            memcpy(&base[i], &rec[(size_t)i * 8], 8);
-          } else {
-            float v;
-            memcpy(&v, &rec[(size_t)i * 4], 4);
-            base[i] = v;
-          }
+          float v;
+          memcpy(&v, &rec[(size_t)i * 4], 4);
+          base[i] = v;
         }
       }
     }
@@ -115,6 +117,23 @@ int conf_io(bool write, const int* dims, double* u, double* a, const char* u_pat
   }
   return rc;
 }
+
+// Host arrays of a configuration, not filled first (every value is written
+// by the download or the file)
+struct HostFields {
+  double *u = nullptr, *a = nullptr;
+  bool ok = true;
+  HostFields(int64_t n, bool links, bool higgs) {
+    if (links) ok = (u = (double*)malloc((size_t)24 * n * sizeof(double))) != nullptr;
+    if (ok && higgs) ok = (a = (double*)malloc((size_t)6 * n * sizeof(double))) != nullptr;
+  }
+  ~HostFields() {
+    free(u);
+    free(a);
+  }
+  HostFields(const HostFields&) = delete;
+  HostFields& operator=(const HostFields&) = delete;
+};
 
 // Fortran Iw.m edit of v into out (w characters, at least m digits, w
 // asterisks when the value does not fit).
@@ -150,10 +169,11 @@ extern "C" int lceq_confsave(lceq_lattice* L, const char* u_path, const char* a_
   int rc = lceq_dims(L, dims);
   if (rc) return rc;
   int64_t n = (int64_t)dims[0] * dims[1] * dims[2] / 2;
-  std::vector<double> u(u_path ? (size_t)24 * n : 0), a(a_path ? (size_t)6 * n : 0);
-  if (u_path && (rc = lceq_get_links(L, u.data(), n))) return rc;
-  if (a_path && (rc = lceq_get_higgs(L, a.data(), n))) return rc;
-  return conf_io(true, dims, u.data(), a.data(), u_path, a_path, real_bytes);
+  HostFields h(n, u_path, a_path);
+  if (!h.ok) return lceq::set_error(LCEQ_ERR_ARG, "no host memory for the fields");
+  if (u_path && (rc = lceq_get_links(L, h.u, n))) return rc;
+  if (a_path && (rc = lceq_get_higgs(L, h.a, n))) return rc;
+  return conf_io(true, dims, h.u, h.a, u_path, a_path, real_bytes);
 }
 
 extern "C" int lceq_oldconf(lceq_lattice* L, const char* u_path, const char* a_path,
@@ -163,10 +183,11 @@ extern "C" int lceq_oldconf(lceq_lattice* L, const char* u_path, const char* a_p
   int rc = lceq_dims(L, dims);
   if (rc) return rc;
   int64_t n = (int64_t)dims[0] * dims[1] * dims[2] / 2;
-  std::vector<double> u(u_path ? (size_t)24 * n : 0), a(a_path ? (size_t)6 * n : 0);
-  if ((rc = conf_io(false, dims, u.data(), a.data(), u_path, a_path, real_bytes))) return rc;
-  if (u_path && (rc = lceq_put_links(L, u.data(), n))) return rc;
-  if (a_path && (rc = lceq_put_higgs(L, a.data(), n))) return rc;
+  HostFields h(n, u_path, a_path);
+  if (!h.ok) return lceq::set_error(LCEQ_ERR_ARG, "no host memory for the fields");
+  if ((rc = conf_io(false, dims, h.u, h.a, u_path, a_path, real_bytes))) return rc;
+  if (u_path && (rc = lceq_put_links(L, h.u, n))) return rc;
+  if (a_path && (rc = lceq_put_higgs(L, h.a, n))) return rc;
   return LCEQ_OK;
 }
 

@@ -115,6 +115,15 @@ inline void prof_count(lceq_lattice* L, int kc) {
   if (L->prof_class == kc && (L->prof_n & 1)) ++L->prof_launches;
 }
 
+// Field transfers (lceq_transfer.hip): the nclass classes of a link (ncomp 4)
+// or Higgs (ncomp 3) field of geometry g between `dev` and the caller's host
+// array in the reference layout with leading dimension ld, ordered after the
+// work queued on `stream`; complete on return.
+int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, double* host,
+                   int64_t ld, int ncomp, int nclass, bool get);
+// a lattice or batch that transfers fields exists (+1) or is gone (-1)
+void transfer_user(int change);
+
 // launchers (lceq_kernels.hip); all enqueue on L->stream, no host sync.
 // Link launches use reduction slots 0-5 ((eo, mu) order), Higgs launches
 // slots 6-7 (eo); with reduce = 0 a launch writes no partial sums.
