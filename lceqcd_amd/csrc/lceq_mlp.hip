@@ -97,130 +97,313 @@ __global__ __launch_bounds__(256) void k_mlp_record(Geom g, const double* __rest
 
 // --------------------------------------------------------------- training
 
-constexpr int TR_TB = 32;  // samples per block, one per lane
+constexpr int TR_SAMPLES = 32;  // samples per block: one partial gradient and loss each
+constexpr int TR_TB = 512;
 
-// Activations of the block's samples, [unit][sample] so that each lane walks
-// its own column and the parameter-gradient sums walk contiguous rows
-struct TrainLds {
-  float x[NIN][TR_TB];
-  float h1[NH][TR_TB], d1[NH][TR_TB], h2[NH][TR_TB], d2[NH][TR_TB];
-  float dout[NOUT][TR_TB];
-  float loss[TR_TB];
+// Rows of a block's samples are padded to 36 floats, rows of W2 to 68: the 16
+// rows x 4 columns of an MFMA operand then fall on 64 banks.  x and dout are
+// padded to whole K steps of 4: row NIN of x is ones (its products with a
+// layer's deltas are the bias gradients), the others zero.
+constexpr int XROWS = 12, DROWS = 8;
+struct alignas(16) TrainLds {
+  float x[XROWS][36], y[3][36];
+  float h1[NH][36], d1[NH][36], h2[NH][36], d2[NH][36];
+  float o[NOUT][36], dout[DROWS][36];
+  float w1[NIN][NH], w2[NH][68], w3[NH][NOUT];
+  float b1[NH], b2[NH], b3[8];
+  float loss[36];
 };
+static_assert(sizeof(TrainLds) <= 64 * 1024, "static LDS of one block");
 
 __device__ __forceinline__ float dsilu(float z) {
   float sg = 1.0f / (1.0f + expf(-z));
   return sg * (1.0f + z * (1.0f - sg));
 }
 
-// Gradient of the mean negative log-likelihood of one block of samples
-// (records idx[b]) with respect to all parameters; one partial gradient and
-// one partial loss per block.  Weights are read from global memory: every
-// lane reads the same address at the same time.
-__global__ __launch_bounds__(32) void k_mlp_grad(const float* __restrict__ w,
-                                                 const float* __restrict__ norm,
-                                                 const float* __restrict__ data,
-                                                 const int* __restrict__ idx, int batch,
-                                                 float* __restrict__ gpart,
-                                                 float* __restrict__ lpart) {
+// Record b of a mini-batch of the epoch's permutation i -> (mult i + offs)
+// mod n: (base + mult b) mod n, base that of the batch's first record; mult
+// and base below n < 2^32, b < 2^31.  The quotient mult b / n, below 2^31, is
+// within one of its estimate in double precision.
+struct TrainBatch {
+  uint64_t mult, base, n;
+  double rn;  // 1 / n
+};
+__device__ __forceinline__ size_t train_record(const TrainBatch& t, int b) {
+  uint64_t a = t.mult * (uint64_t)b;
+  int64_t n = (int64_t)t.n, r = (int64_t)(a - (uint64_t)((double)a * t.rn) * t.n);
+  r += r < 0 ? n : 0;
+  r -= r >= n ? n : 0;
+  r += (int64_t)t.base;
+  return (size_t)(r >= n ? r - n : r);
+}
+
+// D = C + A B with fp32 operands and accumulation: lane l holds A[l % 16][l /
+// 16] (16 x 4), B[l / 16][l % 16] (4 x 16) and D's column l % 16, rows 4 (l /
+// 16) .. + 3.  The four products enter one after the other, each by a fused
+// multiply-add (checked on the device bit for bit), so a chain of them is the
+// sum in index order.
+__device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Gradient of the mean negative log-likelihood of one block of samples with
+// respect to all parameters; one partial gradient and one partial loss per
+// block.  A step of 4096 records is 128 blocks and 0.13 GFLOP: what bounds it
+// is one block's latency.  The weights and records are loaded at once into
+// LDS, and every product of the forward and backward pass and of the
+// gradients runs on fp32 MFMA tiles of 16 x 16 (eight waves: 4 unit tiles x 2
+// sample tiles), which take one LDS word per operand and lane where register
+// tiles on the vector unit waited for LDS reads.  Per 4096 records: 194 us
+// with one lane per sample and the weights read from global memory, 13.9 us
+// with 2 x 4 register tiles from LDS, 10.1 us as below; the sums run in the
+// same order in all three.
+__global__ __launch_bounds__(TR_TB) void k_mlp_grad(const float* __restrict__ w,
+                                                    const float* __restrict__ norm,
+                                                    const float* __restrict__ data, TrainBatch tb,
+                                                    int batch, float* __restrict__ gpart,
+                                                    float* __restrict__ lpart) {
   __shared__ TrainLds T;
-  int t = threadIdx.x;
-  int b = blockIdx.x * TR_TB + t;
-  bool on = b < batch;
-  const float* rec = data + (size_t)idx[on ? b : 0] * NREC;
-  for (int k = 0; k < NIN; ++k) T.x[k][t] = (rec[k] - norm[k]) * norm[NIN + k];
-  // forward; d1, d2 hold silu'(z) until the backward pass scales them
-  for (int j = 0; j < NH; ++j) {
-    float a = w[OFF_B1 + j];
-    for (int k = 0; k < NIN; ++k) a += T.x[k][t] * w[OFF_W1 + k * NH + j];
-    T.h1[j][t] = silu(a);
-    T.d1[j][t] = dsilu(a);
-  }
-  for (int j = 0; j < NH; ++j) {
-    float a = w[OFF_B2 + j];
-    for (int k = 0; k < NH; ++k) a += T.h1[k][t] * w[OFF_W2 + k * NH + j];
-    T.h2[j][t] = silu(a);
-    T.d2[j][t] = dsilu(a);
-  }
-  float o[NOUT];
-  for (int j = 0; j < NOUT; ++j) {
-    float a = w[OFF_B3 + j];
-    for (int k = 0; k < NH; ++k) a += T.h2[k][t] * w[OFF_W3 + k * NOUT + j];
-    o[j] = a;
-  }
-  // loss sum_i [s_i + (y_i - mu_i)^2 exp(-2 s_i) / 2] and its gradient
-  float scale = on ? 1.0f / (float)batch : 0.0f, loss = 0.0f;
-  for (int i = 0; i < 3; ++i) {
-    float sv = fminf(fmaxf(o[3 + i], S_MIN), S_MAX);
-    float inv = expf(-sv), r = (rec[NIN + i] - o[i]) * inv;
-    loss += sv + 0.5f * r * r;
-    T.dout[i][t] = -r * inv * scale;
-    bool clamped = o[3 + i] < S_MIN || o[3 + i] > S_MAX;
-    T.dout[3 + i][t] = clamped ? 0.0f : (1.0f - r * r) * scale;
-  }
-  T.loss[t] = on ? loss : 0.0f;
-  // backward through the hidden layers
-  for (int k = 0; k < NH; ++k) {
-    float a = 0.0f;
-    for (int j = 0; j < NOUT; ++j) a += w[OFF_W3 + k * NOUT + j] * T.dout[j][t];
-    T.d2[k][t] *= a;
-  }
-  for (int k = 0; k < NH; ++k) {
-    float a = 0.0f;
-    for (int j = 0; j < NH; ++j) a += w[OFF_W2 + k * NH + j] * T.d2[j][t];
-    T.d1[k][t] *= a;
+  const int tid = threadIdx.x, first = blockIdx.x * TR_SAMPLES;
+  // records (32 x 13 values) and weights: every load issued before the first
+  // is stored, so the block waits for memory once
+  {
+    constexpr int W4 = NH * NH / 4 / TR_TB;  // 16-byte pieces of W2 per thread
+    static_assert(TR_SAMPLES * NREC <= TR_TB && NH * NOUT <= TR_TB && NIN * NH <= 2 * TR_TB, "");
+    const floatx4* w2 = reinterpret_cast<const floatx4*>(w + OFF_W2);
+    floatx4 c[W4];
+    float c1[2], c3, cb = 0.0f;
+    int i = min(tid, TR_SAMPLES * NREC - 1), t = i / NREC, k = i - t * NREC;
+    float v = data[train_record(tb, first + t) * NREC + k];
+    float mean = norm[min(k, NIN - 1)], inv = norm[NIN + min(k, NIN - 1)];
+#pragma unroll
+    for (int u = 0; u < W4; ++u) c[u] = w2[tid + u * TR_TB];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) c1[u] = w[OFF_W1 + min(tid + u * TR_TB, NIN * NH - 1)];
+    c3 = w[OFF_W3 + min(tid, NH * NOUT - 1)];
+    if (tid < NH)
+      cb = w[OFF_B1 + tid];
+    else if (tid < 2 * NH)
+      cb = w[OFF_B2 + tid - NH];
+    else if (tid < 2 * NH + NOUT)
+      cb = w[OFF_B3 + tid - 2 * NH];
+    __builtin_amdgcn_sched_barrier(0);
+    if (tid < TR_SAMPLES) {
+      T.x[NIN][tid] = 1.0f;
+      T.x[NIN + 1][tid] = 0.0f;
+      T.dout[NOUT][tid] = T.dout[NOUT + 1][tid] = 0.0f;
+    }
+    if (k < NIN)
+      T.x[k][t] = (v - mean) * inv;
+    else
+      T.y[k - NIN][t] = v;
+#pragma unroll
+    for (int u = 0; u < W4; ++u) {
+      int j = 4 * (tid + u * TR_TB);
+      *reinterpret_cast<floatx4*>(&T.w2[j / NH][j % NH]) = c[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (tid + u * TR_TB < NIN * NH) (&T.w1[0][0])[tid + u * TR_TB] = c1[u];
+    if (tid < NH * NOUT) (&T.w3[0][0])[tid] = c3;
+    if (tid < NH)
+      T.b1[tid] = cb;
+    else if (tid < 2 * NH)
+      T.b2[tid - NH] = cb;
+    else if (tid < 2 * NH + NOUT)
+      T.b3[tid - 2 * NH] = cb;
   }
   __syncthreads();
-  // parameter gradients: sums over the block's samples in fixed order
-  float* gp = gpart + (size_t)blockIdx.x * NPARAM;
-  for (int i = t; i < NPARAM; i += TR_TB) {
-    const float *u, *v;
-    if (i < OFF_B1) {
-      u = T.x[i / NH];
-      v = T.d1[i % NH];
-    } else if (i < OFF_W2) {
-      u = nullptr;
-      v = T.d1[i - OFF_B1];
-    } else if (i < OFF_B2) {
-      u = T.h1[(i - OFF_W2) / NH];
-      v = T.d2[(i - OFF_W2) % NH];
-    } else if (i < OFF_W3) {
-      u = nullptr;
-      v = T.d2[i - OFF_B2];
-    } else if (i < OFF_B3) {
-      u = T.h2[(i - OFF_W3) / NOUT];
-      v = T.dout[(i - OFF_W3) % NOUT];
-    } else {
-      u = nullptr;
-      v = T.dout[i - OFF_B3];
+
+  // wave: unit tile ut, sample tile st; lane: operand row or column c, K
+  // element kq of a step; its results are sample sc, units ur .. ur + 3
+  const int lane = tid & 63, wv = tid >> 6, c = lane & 15, kq = lane >> 4;
+  const int ut = 16 * (wv & 3), st = 16 * (wv >> 2), sc = st + c, ur = ut + 4 * kq;
+  // forward; d1, d2 hold silu'(z) until the backward pass scales them
+  {
+    floatx4 z = *reinterpret_cast<const floatx4*>(&T.b1[ur]);
+#pragma unroll
+    for (int k = 0; k < XROWS; k += 4) {
+      float a = k + kq < NIN ? T.w1[min(k + kq, NIN - 1)][ut + c] : 0.0f;
+      z = mfma4(a, T.x[k + kq][sc], z);
     }
-    float a = 0.0f;
-    if (u)
-      for (int q = 0; q < TR_TB; ++q) a += u[q] * v[q];
-    else
-      for (int q = 0; q < TR_TB; ++q) a += v[q];
-    gp[i] = a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      T.h1[ur + i][sc] = silu(z[i]);
+      T.d1[ur + i][sc] = dsilu(z[i]);
+    }
   }
-  if (t == 0) {
-    float l = 0.0f;
-    for (int q = 0; q < TR_TB; ++q) l += T.loss[q];
-    lpart[blockIdx.x] = l;
+  __syncthreads();
+  {
+    floatx4 z = *reinterpret_cast<const floatx4*>(&T.b2[ur]);
+#pragma unroll
+    for (int k = 0; k < NH; k += 4) z = mfma4(T.w2[k + kq][ut + c], T.h1[k + kq][sc], z);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      T.h2[ur + i][sc] = silu(z[i]);
+      T.d2[ur + i][sc] = dsilu(z[i]);
+    }
+  }
+  __syncthreads();
+  if ((wv & 3) == 0) {  // one wave per sample tile; rows NOUT and up are not used
+    const int j = min(c, NOUT - 1);
+    floatx4 z;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = T.b3[min(4 * kq + i, NOUT - 1)];
+#pragma unroll
+    for (int k = 0; k < NH; k += 4) z = mfma4(T.w3[k + kq][j], T.h2[k + kq][sc], z);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * kq + i < NOUT) T.o[4 * kq + i][sc] = z[i];
+  }
+  __syncthreads();
+  // loss sum_i [s_i + (y_i - mu_i)^2 exp(-2 s_i) / 2] and its gradient
+  if (tid < TR_SAMPLES) {
+    float scale = 1.0f / (float)batch, loss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      float os = T.o[3 + i][tid], sv = fminf(fmaxf(os, S_MIN), S_MAX);
+      float inv = expf(-sv), r = (T.y[i][tid] - T.o[i][tid]) * inv;
+      loss += sv + 0.5f * r * r;
+      T.dout[i][tid] = -r * inv * scale;
+      bool clamped = os < S_MIN || os > S_MAX;
+      T.dout[3 + i][tid] = clamped ? 0.0f : (1.0f - r * r) * scale;
+    }
+    T.loss[tid] = loss;
+  }
+  __syncthreads();
+  // backward through the hidden layers
+  {
+    floatx4 z = {};
+#pragma unroll
+    for (int j = 0; j < DROWS; j += 4) {
+      float a = j + kq < NOUT ? T.w3[ut + c][min(j + kq, NOUT - 1)] : 0.0f;
+      z = mfma4(a, T.dout[j + kq][sc], z);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T.d2[ur + i][sc] *= z[i];
+  }
+  __syncthreads();
+  {
+    floatx4 z = {};
+#pragma unroll
+    for (int j = 0; j < NH; j += 4) z = mfma4(T.w2[ut + c][j + kq], T.d2[j + kq][sc], z);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T.d1[ur + i][sc] *= z[i];
+  }
+  __syncthreads();
+  // parameter gradients, sums over the block's samples: rows ut .. + 15 of W2
+  // by two column tiles, and one tile each of W1 with the biases of layer 1
+  // (waves 0-3), of layer 2's biases (the same waves), of W3 (waves 4-7) and,
+  // wave 4, of layer 3's biases and the loss
+  float* gp = gpart + (size_t)blockIdx.x * NPARAM;
+  const float* xr = T.x[min(c, XROWS - 1)];
+  const bool low = wv < 4;
+  const float* dr = T.dout[min(c, DROWS - 1)];
+  const float* lr = c == NOUT ? T.loss : dr;
+  floatx4 g2[2] = {}, ga = {}, gb = {};
+#pragma unroll
+  for (int s = 0; s < TR_SAMPLES; s += 4) {
+    float h = T.h1[ut + c][s + kq];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) g2[u] = mfma4(h, T.d2[2 * st + 16 * u + c][s + kq], g2[u]);
+    if (low) {
+      float x = xr[s + kq];
+      ga = mfma4(x, T.d1[ut + c][s + kq], ga);
+      gb = mfma4(x, T.d2[ut + c][s + kq], gb);
+    } else {
+      ga = mfma4(T.h2[ut + c][s + kq], dr[s + kq], ga);
+      gb = mfma4(xr[s + kq], lr[s + kq], gb);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) gp[OFF_W2 + (ur + i) * NH + 2 * st + 16 * u + c] = g2[u][i];
+    const int row = 4 * kq + i;
+    if (low) {
+      if (row < NIN) gp[OFF_W1 + row * NH + ut + c] = ga[i];
+      if (row == NIN) {
+        gp[OFF_B1 + ut + c] = ga[i];
+        gp[OFF_B2 + ut + c] = gb[i];
+      }
+    } else {
+      if (c < NOUT) gp[OFF_W3 + (ur + i) * NOUT + c] = ga[i];
+      if (wv == 4 && row == NIN) {
+        if (c < NOUT) gp[OFF_B3 + c] = gb[i];
+        if (c == NOUT) lpart[blockIdx.x] = gb[i];
+      }
+    }
   }
 }
 
-// Sum the block gradients (fixed order) and take one Adam step
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ params, float* __restrict__ m,
-                                                  float* __restrict__ v,
-                                                  const float* __restrict__ gpart, int nblk,
-                                                  float lr, float c1, float c2) {
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= NPARAM) return;
-  float g = 0.0f;
-  for (int b = 0; b < nblk; ++b) g += gpart[(size_t)b * NPARAM + i];
-  float mi = 0.9f * m[i] + 0.1f * g, vi = 0.999f * v[i] + 0.001f * g * g;
+// Sum the block gradients in order and take one Adam step, 64 parameters per
+// block.  Latency again (2.7 MB for 128 blocks, written by other compute
+// units): eight waves bring 128 partials of each parameter to LDS at once, and
+// the first wave adds them in order.  31.6 us with one thread per parameter
+// and a load waited for at a time, 8.3 us with 64 loads in flight per thread,
+// 3.6 us as below.
+constexpr int ADAM_P = 64, ADAM_TB = 512, ADAM_FLIGHT = 128;
+__global__ __launch_bounds__(ADAM_TB) void k_mlp_adam(float* __restrict__ params,
+                                                      float* __restrict__ m, float* __restrict__ v,
+                                                      const float* __restrict__ gpart, int nblk,
+                                                      float lr, float c1, float c2) {
+  __shared__ float part[ADAM_FLIGHT][ADAM_P];
+  constexpr int WAVES = ADAM_TB / 64, EACH = ADAM_FLIGHT / WAVES;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int i = blockIdx.x * ADAM_P + lane, il = min(i, NPARAM - 1);
+  float mo = 0.0f, vo = 0.0f, po = 0.0f, g = 0.0f;
+  if (wv == 0) {
+    mo = m[il];
+    vo = v[il];
+    po = params[il];
+  }
+  for (int b0 = 0; b0 < nblk; b0 += ADAM_FLIGHT) {
+    float y[EACH];
+#pragma unroll
+    for (int u = 0; u < EACH; ++u)
+      y[u] = gpart[(size_t)min(b0 + wv * EACH + u, nblk - 1) * NPARAM + il];
+    if (b0) __syncthreads();  // the previous partials are added
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) part[wv * EACH + u][lane] = y[u];
+    __syncthreads();
+    if (wv == 0) {
+      const int k = min(ADAM_FLIGHT, nblk - b0);
+#pragma unroll 16
+      for (int u = 0; u < k; ++u) g += part[u][lane];
+    }
+  }
+  if (wv != 0 || i >= NPARAM) return;
+  float mi = 0.9f * mo + 0.1f * g, vi = 0.999f * vo + 0.001f * g * g;
   m[i] = mi;
   v[i] = vi;
-  params[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
+  params[i] = po - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
+}
+
+// Sums and sums of squares of the NIN inputs over the records, in double: one
+// row of 2 NIN partial sums per block
+constexpr int NORM_BLOCKS = 1024;
+__global__ __launch_bounds__(256) void k_mlp_norm(const float* __restrict__ data, int64_t nrec,
+                                                  double* __restrict__ part) {
+  __shared__ double red[4][2 * NIN];
+  double s[2 * NIN] = {};
+  for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < nrec; r += (int64_t)gridDim.x * 256)
+#pragma unroll
+    for (int k = 0; k < NIN; ++k) {
+      double x = data[(size_t)r * NREC + k];
+      s[k] += x;
+      s[NIN + k] += x * x;
+    }
+#pragma unroll
+  for (int k = 0; k < 2 * NIN; ++k) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 * NIN) {
+    int k = threadIdx.x;
+    part[(size_t)blockIdx.x * 2 * NIN + k] = ((red[0][k] + red[1][k]) + red[2][k]) + red[3][k];
+  }
 }
 
 uint64_t splitmix(uint64_t& x) {
@@ -244,9 +427,7 @@ struct lceq_mlp {
   hipStream_t stream;
   std::vector<float> host;  // NSTATE: params, feature mean, inverse scale
   float *params, *adam_m, *adam_v, *norm, *gpart, *lpart;
-  int gpart_blocks;
-  int* idx;
-  int idx_cap;
+  int64_t gpart_blocks, lpart_cap;  // lpart: [steps of one download][blocks]
   MlpPack* pack;
   int sites_per_wave;  // learned Higgs launch: 0 = by lattice size, 32 or 64
   float* data;  // NREC floats per record
@@ -348,8 +529,7 @@ extern "C" int lceq_mlp_create(uint64_t seed, lceq_mlp** out) {
 
 extern "C" int lceq_mlp_destroy(lceq_mlp* M) {
   if (!M) return LCEQ_OK;
-  void* bufs[] = {M->params, M->adam_m, M->adam_v, M->norm, M->gpart, M->lpart, M->idx, M->pack,
-                  M->data};
+  void* bufs[] = {M->params, M->adam_m, M->adam_v, M->norm, M->gpart, M->lpart, M->pack, M->data};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   if (M->stream) (void)hipStreamDestroy(M->stream);
@@ -462,16 +642,25 @@ extern "C" int lceq_mlp_collect(lceq_lattice* L, lceq_mlp* M, int nsteps, int st
 }
 
 // Feature normalisation from the collected records (mean, 1/std; constant
-// features get scale 1)
+// features get scale 1): the sums on the device, where the records are
 static int mlp_fit_norm(lceq_mlp* M) {
-  std::vector<float> d((size_t)M->nrec * NREC);
-  MHIP(hipMemcpy(d.data(), M->data, d.size() * sizeof(float), hipMemcpyDeviceToHost));
+  int nb = (int)std::min<int64_t>(NORM_BLOCKS, (M->nrec + 255) / 256);
+  double* part = nullptr;
+  std::vector<double> h((size_t)nb * 2 * NIN);
+  MHIP(hipMalloc((void**)&part, h.size() * sizeof(double)));
+  hipLaunchKernelGGL(k_mlp_norm, dim3(nb), dim3(256), 0, M->stream, M->data, M->nrec, part);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(h.data(), part, h.size() * sizeof(double), hipMemcpyDeviceToHost, M->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(M->stream);
+  (void)hipFree(part);
+  if (e != hipSuccess)
+    return mfail(LCEQ_ERR_HIP, "summing the training records: %s", hipGetErrorString(e));
   for (int k = 0; k < NIN; ++k) {
     double s = 0.0, s2 = 0.0;
-    for (int64_t i = 0; i < M->nrec; ++i) {
-      double v = d[(size_t)i * NREC + k];
-      s += v;
-      s2 += v * v;
+    for (int b = 0; b < nb; ++b) {
+      s += h[(size_t)b * 2 * NIN + k];
+      s2 += h[(size_t)b * 2 * NIN + NIN + k];
     }
     double mean = s / (double)M->nrec, var = s2 / (double)M->nrec - mean * mean;
     double sd = var > 1e-12 ? std::sqrt(var) : 0.0;
@@ -484,32 +673,38 @@ static int mlp_fit_norm(lceq_mlp* M) {
 // Adam on the collected records: `steps` mini-batches of `batch` records,
 // each batch a stretch of a seeded affine permutation of the records.
 // loss (optional, steps values) receives the mean negative log-likelihood
-// per step (up to the constant 3/2 log 2 pi).
+// per step (up to the constant 3/2 log 2 pi).  The steps are queued without
+// waiting: the kernels form the record indices themselves, and the blocks'
+// losses are downloaded LOSS_STEPS steps at a time.
+constexpr int LOSS_STEPS = 512;
+
 extern "C" int lceq_mlp_train(lceq_mlp* M, int steps, int batch, double lr, uint64_t seed,
                               int fit_norm, double* loss) {
-  if (!M || steps < 0 || batch < TR_TB || batch % TR_TB)
-    return mfail(LCEQ_ERR_ARG, "batch must be a positive multiple of %d", TR_TB);
+  if (!M || steps < 0 || batch < TR_SAMPLES || batch % TR_SAMPLES)
+    return mfail(LCEQ_ERR_ARG, "batch must be a positive multiple of %d", TR_SAMPLES);
   if (M->nrec < batch) return mfail(LCEQ_ERR_ARG, "only %lld records", (long long)M->nrec);
+  if (M->nrec > (int64_t)UINT32_MAX)  // the permutation's products are 64-bit
+    return mfail(LCEQ_ERR_ARG, "%lld records are more than 2^32 - 1", (long long)M->nrec);
   int rc;
   if (fit_norm) {
     if ((rc = mlp_fit_norm(M))) return rc;
     if ((rc = mlp_upload(M))) return rc;
   }
-  int nblk = batch / TR_TB;
+  const int nblk = batch / TR_SAMPLES;
+  const int rows = loss ? std::max(1, std::min(steps, LOSS_STEPS)) : 1;
   if (nblk > M->gpart_blocks) {
     if (M->gpart) MHIP(hipFree(M->gpart));
-    if (M->lpart) MHIP(hipFree(M->lpart));
     M->gpart = nullptr;
-    M->lpart = nullptr;
+    M->gpart_blocks = 0;
     MHIP(hipMalloc((void**)&M->gpart, (size_t)nblk * NPARAM * sizeof(float)));
-    MHIP(hipMalloc((void**)&M->lpart, (size_t)nblk * sizeof(float)));
     M->gpart_blocks = nblk;
   }
-  if (batch > M->idx_cap) {
-    if (M->idx) MHIP(hipFree(M->idx));
-    M->idx = nullptr;
-    MHIP(hipMalloc((void**)&M->idx, (size_t)batch * sizeof(int)));
-    M->idx_cap = batch;
+  if ((int64_t)rows * nblk > M->lpart_cap) {
+    if (M->lpart) MHIP(hipFree(M->lpart));
+    M->lpart = nullptr;
+    M->lpart_cap = 0;
+    MHIP(hipMalloc((void**)&M->lpart, (size_t)rows * nblk * sizeof(float)));
+    M->lpart_cap = (int64_t)rows * nblk;
   }
   if (M->adam_t == 0) {
     MHIP(hipMemsetAsync(M->adam_m, 0, NPARAM * sizeof(float), M->stream));
@@ -518,8 +713,7 @@ extern "C" int lceq_mlp_train(lceq_mlp* M, int steps, int batch, double lr, uint
   const int64_t N = M->nrec;
   uint64_t st = seed;
   int64_t mult = 1, offs = 0, pos = N;
-  std::vector<int> hidx(batch);
-  std::vector<float> lp(nblk);
+  std::vector<float> lp(loss ? (size_t)rows * nblk : 0);
   for (int it = 0; it < steps; ++it) {
     if (pos + batch > N) {  // new epoch: a fresh affine permutation i -> (mult i + offs) mod N
       do {
@@ -528,24 +722,27 @@ extern "C" int lceq_mlp_train(lceq_mlp* M, int steps, int batch, double lr, uint
       offs = (int64_t)(splitmix(st) % (uint64_t)N);
       pos = 0;
     }
-    for (int b = 0; b < batch; ++b)
-      hidx[b] = (int)(((unsigned __int128)(mult) * (unsigned __int128)(pos + b) + offs) % N);
+    TrainBatch tb{(uint64_t)(mult % N), ((uint64_t)mult * (uint64_t)pos % (uint64_t)N + offs) % N,
+                  (uint64_t)N, 1.0 / (double)N};
     pos += batch;
-    MHIP(hipMemcpyAsync(M->idx, hidx.data(), batch * sizeof(int), hipMemcpyHostToDevice, M->stream));
+    const int row = it % rows;
     hipLaunchKernelGGL(k_mlp_grad, dim3(nblk), dim3(TR_TB), 0, M->stream, M->params, M->norm,
-                       M->data, M->idx, batch, M->gpart, M->lpart);
+                       M->data, tb, batch, M->gpart, M->lpart + (size_t)row * nblk);
     ++M->adam_t;
     float c1 = 1.0f - std::pow(0.9f, (float)M->adam_t), c2 = 1.0f - std::pow(0.999f, (float)M->adam_t);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, M->stream, M->params,
-                       M->adam_m, M->adam_v, M->gpart, nblk, (float)lr, c1, c2);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((NPARAM + ADAM_P - 1) / ADAM_P), dim3(ADAM_TB), 0,
+                       M->stream, M->params, M->adam_m, M->adam_v, M->gpart, nblk, (float)lr, c1,
+                       c2);
     if ((rc = check_launch())) return rc;
-    if (loss) {
-      MHIP(hipMemcpyAsync(lp.data(), M->lpart, nblk * sizeof(float), hipMemcpyDeviceToHost,
-                          M->stream));
+    if (loss && (row == rows - 1 || it == steps - 1)) {
+      MHIP(hipMemcpyAsync(lp.data(), M->lpart, (size_t)(row + 1) * nblk * sizeof(float),
+                          hipMemcpyDeviceToHost, M->stream));
       MHIP(hipStreamSynchronize(M->stream));
-      double l = 0.0;
-      for (int b = 0; b < nblk; ++b) l += lp[b];
-      loss[it] = l / batch;
+      for (int r = 0; r <= row; ++r) {
+        double l = 0.0;
+        for (int b = 0; b < nblk; ++b) l += lp[(size_t)r * nblk + b];
+        loss[it - row + r] = l / batch;
+      }
     }
   }
   MHIP(hipMemcpyAsync(M->host.data(), M->params, NPARAM * sizeof(float), hipMemcpyDeviceToHost,
