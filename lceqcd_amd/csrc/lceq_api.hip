@@ -90,6 +90,10 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
 
   alloc(&L->obs, LCEQ_OBS_N);
+  if (rc == LCEQ_OK &&
+      hipHostMalloc((void**)&L->pin, (LCEQ_OBS_N + LCEQ_PIN_DOUBLES) * sizeof(double),
+                    hipHostMallocDefault) != hipSuccess)
+    rc = fail(LCEQ_ERR_HIP, "hipHostMalloc failed");
   alloc(&L->slices, 14 * (size_t)lz * corr_split(L->g));
   alloc(&L->corr, 5 * (size_t)lz + 8);
   L->hist_cap = 4096;
@@ -124,6 +128,7 @@ extern "C" int lceq_destroy(lceq_lattice* L) {
                     L->slices, L->corr, L->hist, L->scratch, L->fed};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
+  if (L->pin) (void)hipHostFree(L->pin);
   if (L->prof_ev) {
     for (int i = 0; i < L->prof_cap; ++i) (void)hipEventDestroy(L->prof_ev[i]);
     delete[] L->prof_ev;
@@ -589,15 +594,25 @@ extern "C" int lceq_hotstart(lceq_lattice* L, uint64_t seed, double sigma) {
   return check_launch();
 }
 
-int read_obs(lceq_lattice* L, double* host) {
-  HIPCHK(hipMemcpyAsync(host, L->obs, LCEQ_OBS_N * sizeof(double), hipMemcpyDeviceToHost,
-                        L->stream));
+int read_small(lceq_lattice* L, const double* dev, size_t n, double* host) {
+  if (n > LCEQ_PIN_DOUBLES) {
+    HIPCHK(hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipStreamSynchronize(L->stream));
+    return LCEQ_OK;
+  }
+  launch_export(L, dev, n);
+  int rc = check_launch();
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(L->stream));
+  memcpy(host, L->pin + LCEQ_OBS_N, n * sizeof(double));
   return LCEQ_OK;
 }
 
-int write_obs(lceq_lattice* L, int index, double value) {
-  HIPCHK(hipMemcpyAsync(L->obs + index, &value, sizeof(double), hipMemcpyHostToDevice, L->stream));
+int read_obs(lceq_lattice* L, double* host) { return read_small(L, L->obs, LCEQ_OBS_N, host); }
+
+int finish_obs(lceq_lattice* L) {
+  int rc = check_launch();
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(L->stream));
   return LCEQ_OK;
 }
@@ -665,11 +680,10 @@ static int link_call(lceq_lattice* L, int kp, int measflag, double* accept) {
   NEEDL(L);
   int rc = link_sweep(L, kp, measflag, 0, 1);
   if (rc) return rc;
-  launch_finalize(L, kp ? 1 : 2, measflag, 0, 0, nullptr);
+  launch_finalize(L, kp ? 1 : 2, measflag, 0, 0, nullptr, accept != nullptr);
   if (accept) {
-    double o[LCEQ_OBS_N];
-    if ((rc = read_obs(L, o))) return rc;
-    *accept = o[OBS_ACC_LINK];
+    if ((rc = finish_obs(L))) return rc;
+    *accept = L->pin[OBS_ACC_LINK];
   }
   return LCEQ_OK;
 }
@@ -722,14 +736,13 @@ static int higgs_sweep(lceq_lattice* L, int kind, int measflag) {
 extern "C" int lceq_ahiggs1(lceq_lattice* L, double* delta, int measflag, double* accept) {
   NEEDL(L);
   if (!delta) return fail(LCEQ_ERR_ARG, "delta is required");
-  int rc = write_obs(L, OBS_DELTA, *delta);
+  launch_set_obs(L, OBS_DELTA, *delta);
+  int rc = higgs_sweep(L, 1, measflag);
   if (rc) return rc;
-  if ((rc = higgs_sweep(L, 1, measflag))) return rc;
-  launch_finalize(L, 0, 0, 1, measflag, nullptr);
-  double o[LCEQ_OBS_N];
-  if ((rc = read_obs(L, o))) return rc;
-  *delta = o[OBS_DELTA];
-  if (accept) *accept = o[OBS_ACC_HIGGS];
+  launch_finalize(L, 0, 0, 1, measflag, nullptr, true);
+  if ((rc = finish_obs(L))) return rc;
+  *delta = L->pin[OBS_DELTA];
+  if (accept) *accept = L->pin[OBS_ACC_HIGGS];
   return LCEQ_OK;
 }
 
@@ -737,11 +750,11 @@ static int higgs_call(lceq_lattice* L, int kind, int measflag, double* accept) {
   NEEDL(L);
   int rc = higgs_sweep(L, kind, measflag);
   if (rc) return rc;
-  launch_finalize(L, 0, 0, kind, measflag, nullptr);
-  if (accept && measflag == 1) {
-    double o[LCEQ_OBS_N];
-    if ((rc = read_obs(L, o))) return rc;
-    *accept = o[OBS_ACC_HIGGS];
+  const bool read = accept && measflag == 1;
+  launch_finalize(L, 0, 0, kind, measflag, nullptr, read);
+  if (read) {
+    if ((rc = finish_obs(L))) return rc;
+    *accept = L->pin[OBS_ACC_HIGGS];
   }
   return LCEQ_OK;
 }
@@ -766,9 +779,7 @@ extern "C" int lceq_check_fields(lceq_lattice* L, double tol, double* max_dev,
   launch_check_fields(L, L->scratch);
   if ((rc = check_launch())) return rc;
   std::vector<double> h(2 * (size_t)nb);
-  HIPCHK(hipMemcpyAsync(h.data(), L->scratch, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
+  if ((rc = read_small(L, L->scratch, h.size(), h.data()))) return rc;
   double dev = 0.0, bad = 0.0;
   for (int b = 0; b < nb; ++b) {
     dev = std::max(dev, h[2 * b]);
@@ -948,10 +959,10 @@ extern "C" int lceq_sweep(lceq_lattice* L, int schedule, int nsweep, int n_or, d
   if (nsweep < 0 || n_or < 0) return fail(LCEQ_ERR_ARG, "nsweep, n_or must be >= 0");
   if (schedule != LCEQ_SWEEP_KP_OR_METRO && schedule != LCEQ_SWEEP_REFERENCE)
     return fail(LCEQ_ERR_ARG, "unknown schedule %d", schedule);
-  int rc;
+  int rc = LCEQ_OK;
   if (schedule == LCEQ_SWEEP_KP_OR_METRO) {
     if (!delta) return fail(LCEQ_ERR_ARG, "delta is required for schedule 0");
-    if ((rc = write_obs(L, OBS_DELTA, *delta))) return rc;
+    launch_set_obs(L, OBS_DELTA, *delta);
   }
   if (measflag && L->hist_rows + nsweep > L->hist_cap)
     return fail(LCEQ_ERR_ARG, "history full (%d rows); call lceq_history", L->hist_cap);
@@ -971,21 +982,21 @@ extern "C" int lceq_sweep(lceq_lattice* L, int schedule, int nsweep, int n_or, d
       prof_end(L, KC_LINK_OR);
       if (rc) return rc;
       if ((rc = higgs_sweep(L, 1, measflag))) return rc;
-      launch_finalize(L, measflag ? (n_or ? 2 : 1) : 0, measflag, 1, measflag, row);
+      launch_finalize(L, measflag ? (n_or ? 2 : 1) : 0, measflag, 1, measflag, row,
+                      it == nsweep - 1);
     } else {  // f/main.f:38-41
       if ((rc = higgs_sweep(L, 2, measflag))) return rc;
-      if (measflag) launch_finalize(L, 0, 0, 2, 1, nullptr);
+      if (measflag) launch_finalize(L, 0, 0, 2, 1, nullptr, false);
       if ((rc = higgs_sweep(L, 3, measflag))) return rc;
       if ((rc = link_sweep(L, 1, measflag, 0, measflag))) return rc;
-      if (measflag) launch_finalize(L, 1, 1, 3, 1, row);
+      if (measflag) launch_finalize(L, 1, 1, 3, 1, row, false);
       launch_renorm(L, L->U);
     }
   }
   if ((rc = check_launch())) return rc;
   if (schedule == LCEQ_SWEEP_KP_OR_METRO) {
-    HIPCHK(hipMemcpyAsync(delta, L->obs + OBS_DELTA, sizeof(double), hipMemcpyDeviceToHost,
-                          L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
+    if ((rc = finish_obs(L))) return rc;
+    if (nsweep > 0) *delta = L->pin[OBS_DELTA];
   }
   return LCEQ_OK;
 }
@@ -995,10 +1006,9 @@ extern "C" int lceq_history(lceq_lattice* L, double* out, int n) {
   if (n < 0 || n > L->hist_rows) return fail(LCEQ_ERR_ARG, "only %d rows recorded", L->hist_rows);
   if (n > 0) {
     if (!out) return fail(LCEQ_ERR_ARG, "null output");
-    HIPCHK(hipMemcpyAsync(out, L->hist + (size_t)(L->hist_rows - n) * LCEQ_OBS_N,
-                          (size_t)n * LCEQ_OBS_N * sizeof(double), hipMemcpyDeviceToHost,
-                          L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
+    int rc = read_small(L, L->hist + (size_t)(L->hist_rows - n) * LCEQ_OBS_N,
+                        (size_t)n * LCEQ_OBS_N, out);
+    if (rc) return rc;
   }
   L->hist_rows = 0;
   return LCEQ_OK;

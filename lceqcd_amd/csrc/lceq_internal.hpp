@@ -30,6 +30,9 @@ enum {
   LCEQ_OBS_N = 16
 };
 
+// doubles of lceq_lattice::pin after the observables (64 KiB in all)
+#define LCEQ_PIN_DOUBLES (8192 - LCEQ_OBS_N)
+
 struct lceq_lattice {
   lceq::Geom g;
   int vol;
@@ -40,6 +43,9 @@ struct lceq_lattice {
   double *partials;  // [LCEQ_NSLOT][LCEQ_NQ][pstride]
   int pstride;       // >= number of 64-site blocks (the smallest launch shape)
   double *obs;       // [LCEQ_OBS_N]
+  // pinned host memory that kernels write results to: the observables, then
+  // PIN_DOUBLES values of any other small result
+  double *pin;
   double *hist;      // [hist_cap][LCEQ_OBS_N] per-sweep records
   int hist_cap;
   int hist_rows;     // rows recorded since the last lceq_history
@@ -133,9 +139,14 @@ void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int reno
 // 0 none, 1 KP (agauge), 2 overrelaxation; higgs_kind 0 none, 1-3 ahiggs1-3;
 // with hist_row the observables are also copied into that history row.
 // higgs_nb: block partials of the Higgs slots when their launch used another
-// shape than the lattice's (0: the lattice's shape)
+// shape than the lattice's (0: the lattice's shape).  to_host: the
+// observables also go to L->pin, for finish_obs
 void launch_finalize(lceq_lattice* L, int link_kind, int link_meas, int higgs_kind,
-                     int higgs_meas, double* hist_row, int higgs_nb = 0);
+                     int higgs_meas, double* hist_row, bool to_host, int higgs_nb = 0);
+// obs[index] = value, and n doubles (at most LCEQ_PIN_DOUBLES) of device
+// memory to L->pin + LCEQ_OBS_N
+void launch_set_obs(lceq_lattice* L, int index, double value);
+void launch_export(lceq_lattice* L, const double* dev, size_t n);
 void launch_staples(lceq_lattice* L, int eo, int mu);
 void launch_force(lceq_lattice* L, int eo);
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
@@ -167,8 +178,11 @@ void launch_testconf(lceq_lattice* L);
 // helpers of the C ABI layer (lceq_api.hip) shared with the other entry files
 int check_launch();
 uint64_t next_pass(lceq_lattice* L);
+// n doubles of device memory to the host, after the work queued so far
+int read_small(lceq_lattice* L, const double* dev, size_t n, double* host);
 int read_obs(lceq_lattice* L, double* host);
-int write_obs(lceq_lattice* L, int index, double value);
+// waits for a launch_finalize with to_host; its observables are in L->pin
+int finish_obs(lceq_lattice* L);
 // one full link sweep (six (eo, mu) launches) of the KP heatbath or the
 // overrelaxation, partials in slots 0-5 when reduce is set
 int link_sweep(lceq_lattice* L, int kp, int measflag, int renorm_on_write, int reduce);

@@ -151,6 +151,7 @@ struct FinalizeArgs {
   double vol;
   double* obs;
   double* hist_row;
+  double* host;  // pinned copy of the observables, or null
 };
 
 // One 1024-thread block sums every partial the closing routines wrote: six
@@ -247,12 +248,36 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs p) {
     double o = ob[threadIdx.x];
     p.obs[threadIdx.x] = o;
     if (p.hist_row) p.hist_row[threadIdx.x] = o;
+    if (p.host) p.host[threadIdx.x] = o;
   }
 }
 
+__global__ __launch_bounds__(64) void k_set_obs(double* __restrict__ obs, int index, double value) {
+  if (threadIdx.x == 0) obs[index] = value;
+}
+
+void launch_set_obs(lceq_lattice* L, int index, double value) {
+  hipLaunchKernelGGL(k_set_obs, dim3(1), dim3(64), 0, L->stream, L->obs, index, value);
+}
+
+// Small results reach the host by stores to pinned memory: a copy command to
+// pageable memory and its wait took 40 us (the seven averages of a lattice),
+// this kernel and its wait 14
+__global__ __launch_bounds__(TB) void k_export(const double* __restrict__ dev,
+                                               double* __restrict__ host, unsigned n) {
+  unsigned i = blockIdx.x * TB + threadIdx.x;
+  if (i < n) host[i] = dev[i];
+}
+
+void launch_export(lceq_lattice* L, const double* dev, size_t n) {
+  hipLaunchKernelGGL(k_export, dim3(blocks_for((int)n)), dim3(TB), 0, L->stream, dev,
+                     L->pin + LCEQ_OBS_N, (unsigned)n);
+}
+
 void launch_finalize(lceq_lattice* L, int link_kind, int link_meas, int higgs_kind,
-                     int higgs_meas, double* hist_row, int higgs_nb) {
+                     int higgs_meas, double* hist_row, bool to_host, int higgs_nb) {
   FinalizeArgs a;
+  a.host = to_host ? L->pin : nullptr;
   a.part = L->partials;
   a.pstride = L->pstride;
   a.nb_link = shape_blocks(L);

@@ -834,11 +834,10 @@ extern "C" int lceq_higgs_mlp(lceq_lattice* L, lceq_mlp* M, double* accept) {
   if (!L || !M) return mfail(LCEQ_ERR_ARG, "null argument");
   int rc = mlp_higgs_sweep(L, M);
   if (rc) return rc;
-  launch_finalize(L, 0, 0, 2, 1, nullptr, mlp_blocks(L, M));
+  launch_finalize(L, 0, 0, 2, 1, nullptr, accept != nullptr, mlp_blocks(L, M));
   if (accept) {
-    double o[LCEQ_OBS_N];
-    if ((rc = read_obs(L, o))) return rc;
-    *accept = o[OBS_ACC_HIGGS];
+    if ((rc = finish_obs(L))) return rc;
+    *accept = L->pin[OBS_ACC_HIGGS];
   }
   return LCEQ_OK;
 }
@@ -860,7 +859,8 @@ extern "C" int lceq_sweep_mlp(lceq_lattice* L, lceq_mlp* M, int nsweep, int n_or
       if ((rc = link_sweep(L, 0, m, 1, m))) return rc;
     }
     if ((rc = mlp_higgs_sweep(L, M))) return rc;
-    launch_finalize(L, measflag ? (n_or ? 2 : 1) : 0, measflag, 2, 1, row, mlp_blocks(L, M));
+    launch_finalize(L, measflag ? (n_or ? 2 : 1) : 0, measflag, 2, 1, row, false,
+                    mlp_blocks(L, M));
   }
   return check_launch();
 }
