@@ -857,52 +857,59 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   return LCEQ_OK;
 }
 
-static int run_corr(lceq_lattice* L, std::vector<double>& c) {
-  launch_slices(L);
-  launch_corr(L);
+// Measurement meas of launch_corr; *c points at its results (the layout of
+// L->corr) in pinned memory, or in `store` on lattices too long for it
+static int run_corr(lceq_lattice* L, int meas, const double** c, std::vector<double>& store) {
+  size_t n = 5 * (size_t)L->g.lz + 5;
+  double* host = n <= LCEQ_PIN_DOUBLES ? L->pin + LCEQ_OBS_N : nullptr;
+  launch_corr(L, meas, host);
   int rc = check_launch();
   if (rc) return rc;
-  c.resize(5 * (size_t)L->g.lz + 5);
-  HIPCHK(hipMemcpyAsync(c.data(), L->corr, c.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        L->stream));
+  *c = host;
+  if (!host) {
+    store.resize(n);
+    *c = store.data();
+    HIPCHK(hipMemcpyAsync(store.data(), L->corr, n * sizeof(double), hipMemcpyDeviceToHost,
+                          L->stream));
+  }
   HIPCHK(hipStreamSynchronize(L->stream));
   return LCEQ_OK;
 }
 
 extern "C" int lceq_correlator(lceq_lattice* L, double* corr_a, double* corr_u, double* corr_3) {
   NEEDL(L);
-  std::vector<double> c;
-  int rc = run_corr(L, c);
+  std::vector<double> store;
+  const double* c;
+  int rc = run_corr(L, 0, &c, store);
   if (rc) return rc;
   int lz = L->g.lz;
-  if (corr_a) memcpy(corr_a, c.data(), lz * sizeof(double));
-  if (corr_u) memcpy(corr_u, c.data() + lz, lz * sizeof(double));
-  if (corr_3) memcpy(corr_3, c.data() + 2 * lz, lz * sizeof(double));
-  HIPCHK(hipMemcpyAsync(L->obs + OBS_A0F, c.data() + 5 * lz + 2, 3 * sizeof(double),
-                        hipMemcpyHostToDevice, L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
+  if (corr_a) memcpy(corr_a, c, lz * sizeof(double));
+  if (corr_u) memcpy(corr_u, c + lz, lz * sizeof(double));
+  if (corr_3) memcpy(corr_3, c + 2 * (size_t)lz, lz * sizeof(double));
   return LCEQ_OK;
 }
 
 extern "C" int lceq_scalarcorr(lceq_lattice* L, double* mean, double* corr) {
   NEEDL(L);
-  std::vector<double> c;
-  int rc = run_corr(L, c);
+  std::vector<double> store;
+  const double* c;
+  int rc = run_corr(L, 1, &c, store);
   if (rc) return rc;
-  int lz = L->g.lz;
+  size_t lz = L->g.lz;
   if (mean) *mean = c[5 * lz];
-  if (corr) memcpy(corr, c.data() + 3 * lz, lz * sizeof(double));
+  if (corr) memcpy(corr, c + 3 * lz, lz * sizeof(double));
   return LCEQ_OK;
 }
 
 extern "C" int lceq_polyakov(lceq_lattice* L, double* mean_sq, double* corr) {
   NEEDL(L);
-  std::vector<double> c;
-  int rc = run_corr(L, c);
+  std::vector<double> store;
+  const double* c;
+  int rc = run_corr(L, 2, &c, store);
   if (rc) return rc;
-  int lz = L->g.lz;
+  size_t lz = L->g.lz;
   if (mean_sq) *mean_sq = c[5 * lz + 1];
-  if (corr) memcpy(corr, c.data() + 4 * lz, lz * sizeof(double));
+  if (corr) memcpy(corr, c + 4 * lz, lz * sizeof(double));
   return LCEQ_OK;
 }
 

@@ -161,8 +161,10 @@ void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarde
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter = 0);
 // blocks per z slice of the slice sums (the slices buffer holds 14 lz split)
 int corr_split(const Geom& g);
-void launch_slices(lceq_lattice* L);
-void launch_corr(lceq_lattice* L);
+// the slice sums and correlators of measurement meas (0 correlator, which
+// also sets a0f in the observables, 1 scalarcorr, 2 polyakov) into L->corr
+// and, where host is not null, the pinned copy there
+void launch_corr(lceq_lattice* L, int meas, double* host);
 void launch_heat_kpi(lceq_lattice* L, int n, const double* b, const double* a0_old, double* v,
                      const double* fed, uint64_t pass);
 void launch_gauss(lceq_lattice* L, int n, const double* r, double* x, const double* fed,

@@ -640,145 +640,180 @@ void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter) {
 // slices[(q*lz + z)*split + j]):
 //   0-2 a_f(1..3); 3+3*mu: Im alpha_mu, 4+3*mu: Im beta_mu, 5+3*mu: -Re beta_mu
 //   (the (Im a, -i b) projection of u_f); 12 rho(a); 13 cos(4|a|).
+// A measurement sums only what it uses: MEAS 0 (correlator) 0-11 from u_f and
+// a_f, 1 (scalarcorr) 12 and 2 (polyakov) 13 from a, 24 of 144 bytes a site.
+template <int MEAS>
 __global__ __launch_bounds__(256) void k_slices(Geom g, int split,
                                                 const double* __restrict__ Uf,
                                                 const double* __restrict__ Af,
                                                 const double* __restrict__ A,
                                                 double* __restrict__ slices) {
-  __shared__ double red[4][14];
+  constexpr int Q0 = MEAS == 0 ? 0 : 11 + MEAS, NQ = MEAS == 0 ? 12 : 1;
+  __shared__ double red[4][NQ];
   int z = blockIdx.x, j = blockIdx.y;
   int nz = 2 * g.h2, chunk = (nz + split - 1) / split;
   int i0 = j * chunk, i1 = min(nz, i0 + chunk);
-  double acc[14];
+  double acc[NQ];
 #pragma unroll
-  for (int q = 0; q < 14; ++q) acc[q] = 0.0;
+  for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
   for (int i = i0 + threadIdx.x; i < i1; i += TB) {
     int p = i >= g.h2, s = z * g.h2 + (i - p * g.h2);
-    vec3 af = ld_higgs(Af, g, p, s), a = ld_higgs(A, g, p, s);
+    if constexpr (MEAS == 0) {
+      vec3 af = ld_higgs(Af, g, p, s);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) acc[k] += af.x[k];
+      for (int k = 0; k < 3; ++k) acc[k] += af.x[k];
 #pragma unroll
-    for (int mu = 0; mu < 3; ++mu) {
-      su2 u = ld_link(Uf, g, mu, p, s);
-      acc[3 + 3 * mu] += u.a.im;
-      acc[4 + 3 * mu] += u.b.im;
-      acc[5 + 3 * mu] -= u.b.re;
+      for (int mu = 0; mu < 3; ++mu) {
+        su2 u = ld_link(Uf, g, mu, p, s);
+        acc[3 + 3 * mu] += u.a.im;
+        acc[4 + 3 * mu] += u.b.im;
+        acc[5 + 3 * mu] -= u.b.re;
+      }
+    } else {
+      vec3 a = ld_higgs(A, g, p, s);
+      double rho = a.x[0] * a.x[0] + a.x[1] * a.x[1] + a.x[2] * a.x[2];
+      acc[0] += MEAS == 1 ? rho : cos(4.0 * sqrt(rho));
     }
-    double rho = a.x[0] * a.x[0] + a.x[1] * a.x[1] + a.x[2] * a.x[2];
-    acc[12] += rho;
-    acc[13] += cos(4.0 * sqrt(rho));
   }
 #pragma unroll
-  for (int q = 0; q < 14; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     double t = acc[q];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][q] = t;
   }
   __syncthreads();
-  if (threadIdx.x < 14) {
+  if (threadIdx.x < NQ) {
     int q = threadIdx.x;
-    slices[(q * g.lz + z) * split + j] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
+    slices[((Q0 + q) * g.lz + z) * split + j] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
   }
 }
 
 // Periodic z-correlators on the slice means (f/correlator.f:139-164,
-// f/scalarcorr.f:96-104, f/polyakov.f:97-107).  corr layout:
-// [0,lz) C_a, [lz,2lz) C_u, [2lz,3lz) C_3, [3lz,4lz) rho, [4lz,5lz) Polyakov,
-// then mean(rho), mean(P)^2, a0f(1..3).  The slice partials are summed in a
-// fixed order into slice means, held in LDS (dynamic, 14 lz doubles) when
-// LDS is set, else in `slices` itself.
-constexpr int CORR_TB = 1024;    // threads of the one k_corr block
+// f/scalarcorr.f:96-104, f/polyakov.f:97-107).  corr layout: [0,lz) C_a,
+// [lz,2lz) C_u, [2lz,3lz) C_3, [3lz,4lz) rho, [4lz,5lz) Polyakov, then
+// mean(rho), mean(P)^2, a0f(1..3); a copy goes to pinned host memory where it
+// fits (host), and a0f to the observables.
+// A block sums the slice partials of its correlator's quantities in a fixed
+// order into slice means, in LDS (dynamic, 6 lz doubles; LDS = false: read
+// from `slices`, with split = 1, each time).  What bounds it is latency: a
+// correlator is lz dependent additions in x0 order.  The three correlators of
+// u_f and a_f take one block each per CORR_Z separations, whose threads form
+// the products of CORR_X slices with their partners for one thread per
+// separation to add; rho and Polyakov are one multiply-add a slice, a thread
+// per separation.  At lz = 128, 19.5 us for correlator with a thread per
+// separation that also forms the products, 7.0 us as here.
+constexpr int CORR_TB = 256;
 constexpr int CORR_MAX_SPLIT = 16;
+constexpr int CORR_Z = 16, CORR_X = 128;
 
 template <bool LDS>
-__global__ __launch_bounds__(CORR_TB) void k_corr(Geom g, int split, double* __restrict__ slices,
-                                                  double* __restrict__ corr) {
+__global__ __launch_bounds__(CORR_TB) void k_corr(Geom g, int split, int meas,
+                                                  const double* __restrict__ slices,
+                                                  double* __restrict__ corr,
+                                                  double* __restrict__ host,
+                                                  double* __restrict__ obs) {
   extern __shared__ double lds_slices[];
-  int lz = g.lz;
-  double area = (double)(g.lx * g.ly);
-  double* as = LDS ? lds_slices : slices;
-  // in place (LDS = false) is safe: element i reads only its own partials,
-  // and split = 1 then (see corr_split), so slices[i * split] = slices[i].
-  // All partials of an element are loaded before they are added (in order).
-  for (int i = threadIdx.x; i < 14 * lz; i += CORR_TB) {
-    double y[CORR_MAX_SPLIT];
+  __shared__ double prod[CORR_Z][CORR_X + 1];
+  const int lz = g.lz, tid = threadIdx.x;
+  const double area = (double)(g.lx * g.ly);
+  const int kind = meas == 0 ? (int)blockIdx.y : 2 + meas;
+  const int zper = meas == 0 ? CORR_Z : CORR_TB;
+  const int z0 = (int)blockIdx.x * zper;
+  const int q0 = kind < 2 ? 3 * kind : kind == 2 ? 9 : 9 + kind;  // first quantity
+  const int nq = kind >= 3 ? 1 : kind == 1 ? 6 : 3;
+  const double* part = slices + (size_t)q0 * lz * split;
+  // all partials of an element are loaded before they are added (in order)
+  if (LDS) {
+    for (int i = tid; i < nq * lz; i += CORR_TB) {
+      double y[CORR_MAX_SPLIT];
 #pragma unroll
-    for (int j = 0; j < CORR_MAX_SPLIT; ++j) y[j] = j < split ? slices[i * split + j] : 0.0;
-    double v = 0.0;
+      for (int j = 0; j < CORR_MAX_SPLIT; ++j) y[j] = j < split ? part[i * split + j] : 0.0;
+      double v = 0.0;
 #pragma unroll
-    for (int j = 0; j < CORR_MAX_SPLIT; ++j)
-      if (j < split) v += y[j];
-    as[i] = v / area;
-  }
-  __syncthreads();
-  // one thread per (correlator, separation); each sum runs over x0 in order
-  for (int task = threadIdx.x; task < 5 * lz; task += CORR_TB) {
-    int kind = task / lz, z = task - kind * lz;
-    double c = 0.0;
-    // one loop per kind, unrolled so that the LDS reads of several x0 are in
-    // flight together; the additions stay in x0 order
-    if (kind == 0) {
-#pragma unroll 8
-      for (int x0 = 0; x0 < lz; ++x0) {
-        int x1 = x0 + z < lz ? x0 + z : x0 + z - lz;
-        double d = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) d = d + as[k * lz + x0] * as[k * lz + x1];
-        c = c + d;
-      }
-    } else if (kind == 1) {  // Re[A1 A1' + A2 conj(A2')] for mu = 1,2, A1 real
-#pragma unroll 8
-      for (int x0 = 0; x0 < lz; ++x0) {
-        int x1 = x0 + z < lz ? x0 + z : x0 + z - lz;
-        double t = 0.0;
-#pragma unroll
-        for (int mu = 0; mu < 2; ++mu) {
-          double a1 = as[(3 + 3 * mu) * lz + x0], a1p = as[(3 + 3 * mu) * lz + x1];
-          double br = as[(4 + 3 * mu) * lz + x0], bi = as[(5 + 3 * mu) * lz + x0];
-          double brp = as[(4 + 3 * mu) * lz + x1], bip = as[(5 + 3 * mu) * lz + x1];
-          t = t + a1 * a1p;
-          t = t + (br * brp + bi * bip);
-        }
-        c = c + t;
-      }
-    } else if (kind == 2) {  // mu = 3
-#pragma unroll 8
-      for (int x0 = 0; x0 < lz; ++x0) {
-        int x1 = x0 + z < lz ? x0 + z : x0 + z - lz;
-        double a1 = as[9 * lz + x0], a1p = as[9 * lz + x1];
-        double br = as[10 * lz + x0], bi = as[11 * lz + x0];
-        double brp = as[10 * lz + x1], bip = as[11 * lz + x1];
-        c = c + (a1 * a1p + (br * brp + bi * bip));
-      }
-    } else {  // rho, Polyakov
-      const double* q = as + (kind == 3 ? 12 : 13) * lz;
-#pragma unroll 8
-      for (int x0 = 0; x0 < lz; ++x0) {
-        int x1 = x0 + z < lz ? x0 + z : x0 + z - lz;
-        c = c + q[x0] * q[x1];
-      }
+      for (int j = 0; j < CORR_MAX_SPLIT; ++j)
+        if (j < split) v += y[j];
+      lds_slices[i] = v / area;
     }
-    corr[kind * lz + z] = kind == 1 ? c / (lz * 2) : c / lz;
+    __syncthreads();
   }
-  // the means, one quantity per thread, summed over z in order
-  if (threadIdx.x < 5) {
-    const int qs[5] = {12, 13, 0, 1, 2};
-    int q = qs[threadIdx.x];
-    double m = 0.0;
-#pragma unroll 8
-    for (int z = 0; z < lz; ++z) m += as[q * lz + z];
-    m = m / lz;
+  auto mean = [&](int q, int x) {
+    return LDS ? lds_slices[q * lz + x] : (0.0 + part[(size_t)q * lz + x]) / area;
+  };
+  auto put = [&](int i, double v) {
+    corr[i] = v;
+    if (host) host[i] = v;
+  };
+  auto product = [&](int x0, int x1) {
+    if (kind == 0) {
+      double d = 0.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d = d + mean(k, x0) * mean(k, x1);
+      return d;
+    }
+    if (kind == 1) {  // Re[A1 A1' + A2 conj(A2')] for mu = 1,2, A1 real
+      double t = 0.0;
+#pragma unroll
+      for (int mu = 0; mu < 2; ++mu) {
+        double a1 = mean(3 * mu, x0), a1p = mean(3 * mu, x1);
+        double br = mean(1 + 3 * mu, x0), bi = mean(2 + 3 * mu, x0);
+        double brp = mean(1 + 3 * mu, x1), bip = mean(2 + 3 * mu, x1);
+        t = t + a1 * a1p;
+        t = t + (br * brp + bi * bip);
+      }
+      return t;
+    }
+    // mu = 3
+    return mean(0, x0) * mean(0, x1) + (mean(1, x0) * mean(1, x1) + mean(2, x0) * mean(2, x1));
+  };
+  // the means, one quantity per thread, summed over z in order, by the last
+  // wave of the first block while the first wave adds products
+  auto means = [&]() {
+    const int m = tid - (CORR_TB - 64);
+    if (z0 != 0 || m < 0 || m >= (kind == 0 ? 3 : kind >= 3 ? 1 : 0)) return;
+    double v = 0.0;
+#pragma unroll 16
+    for (int z = 0; z < lz; ++z) v += mean(m, z);
+    v = v / lz;
     // mean(rho), mean(P)^2, a0f(1..3) = mean over sites = mean of slice means
-    corr[5 * lz + threadIdx.x] = threadIdx.x == 1 ? m * m : m;
+    put(5 * lz + (kind == 0 ? 2 + m : kind - 3), kind == 4 ? v * v : v);
+    if (kind == 0) obs[OBS_A0F + m] = v;
+  };
+  const int zt = z0 + tid;
+  const bool adds = tid < zper && zt < lz;
+  double c = 0.0;
+  if (kind >= 3) {  // rho, Polyakov: one multiply-add per slice
+    means();
+    if (adds) {
+#pragma unroll 16
+      for (int x0 = 0; x0 < lz; ++x0) c = c + mean(0, x0) * mean(0, x0 + zt < lz ? x0 + zt : x0 + zt - lz);
+    }
+  } else {
+    for (int xb = 0; xb < lz; xb += CORR_X) {
+      const int nx = min(CORR_X, lz - xb);
+      for (int i = tid; i < CORR_Z * CORR_X; i += CORR_TB) {
+        int zi = i / CORR_X, xi = i % CORR_X, z = z0 + zi, x0 = xb + xi;
+        if (xi < nx && z < lz) prod[zi][xi] = product(x0, x0 + z < lz ? x0 + z : x0 + z - lz);
+      }
+      __syncthreads();
+      if (xb == 0) means();
+      if (adds) {
+#pragma unroll 16
+        for (int xi = 0; xi < nx; ++xi) c = c + prod[tid][xi];
+      }
+      __syncthreads();
+    }
   }
+  if (adds) put(kind * lz + zt, kind == 1 ? c / (lz * 2) : c / lz);
 }
 
-// slice means in LDS up to this many bytes (one block, 64 KB per workgroup)
-constexpr size_t CORR_LDS_MAX = 64 * 1024;
+// slice means in LDS up to this many bytes (64 KB per workgroup, of which the
+// products take 16.1)
+constexpr size_t CORR_LDS_MAX = 47 * 1024;
+constexpr int CORR_LDS_Q = 6;  // most quantities of one correlator
 
 int corr_split(const Geom& g) {
-  if (14 * (size_t)g.lz * sizeof(double) > CORR_LDS_MAX) return 1;
+  if (CORR_LDS_Q * (size_t)g.lz * sizeof(double) > CORR_LDS_MAX) return 1;
   int nz = 2 * g.h2;
   // 512 sites per block, at most CORR_MAX_SPLIT blocks per slice.  One site
   // per thread (twice the blocks) was measured slower: 64^3 slice sums
@@ -787,20 +822,25 @@ int corr_split(const Geom& g) {
   return std::max(1, std::min(CORR_MAX_SPLIT, (nz + 2 * TB - 1) / (2 * TB)));
 }
 
-void launch_slices(lceq_lattice* L) {
-  int split = corr_split(L->g);
-  hipLaunchKernelGGL(k_slices, dim3(L->g.lz, split), dim3(TB), 0, L->stream, L->g, split, L->Uf,
-                     L->Af, L->A, L->slices);
-}
-void launch_corr(lceq_lattice* L) {
-  int split = corr_split(L->g);
-  size_t lds = 14 * (size_t)L->g.lz * sizeof(double);
-  if (lds <= CORR_LDS_MAX)
-    hipLaunchKernelGGL(k_corr<true>, dim3(1), dim3(CORR_TB), lds, L->stream, L->g, split,
-                       L->slices, L->corr);
+void launch_corr(lceq_lattice* L, int meas, double* host) {
+  const Geom& g = L->g;
+  int split = corr_split(g);
+  dim3 grid(g.lz, split);
+  if (meas == 0)
+    hipLaunchKernelGGL(k_slices<0>, grid, dim3(TB), 0, L->stream, g, split, L->Uf, L->Af, L->A, L->slices);
+  else if (meas == 1)
+    hipLaunchKernelGGL(k_slices<1>, grid, dim3(TB), 0, L->stream, g, split, L->Uf, L->Af, L->A, L->slices);
   else
-    hipLaunchKernelGGL(k_corr<false>, dim3(1), dim3(CORR_TB), 0, L->stream, L->g, split,
-                       L->slices, L->corr);
+    hipLaunchKernelGGL(k_slices<2>, grid, dim3(TB), 0, L->stream, g, split, L->Uf, L->Af, L->A, L->slices);
+  size_t lds = CORR_LDS_Q * (size_t)g.lz * sizeof(double);
+  const int zper = meas == 0 ? CORR_Z : CORR_TB;
+  dim3 kinds((g.lz + zper - 1) / zper, meas == 0 ? 3 : 1);
+  if (lds <= CORR_LDS_MAX)
+    hipLaunchKernelGGL(k_corr<true>, kinds, dim3(CORR_TB), lds, L->stream, g, split, meas,
+                       L->slices, L->corr, host, L->obs);
+  else
+    hipLaunchKernelGGL(k_corr<false>, kinds, dim3(CORR_TB), 0, L->stream, g, split, meas,
+                       L->slices, L->corr, host, L->obs);
 }
 
 // ============================================ array-level entry points
