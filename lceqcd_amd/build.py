@@ -25,6 +25,9 @@ FLAGS = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17",
     # keep the compiler away from packed FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # leading kernel arguments in scalar registers at wave start (at most 14
+    # dwords): no memory round trip ahead of a launch's first loads
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall", "-Wno-unknown-warning-option",
 ]
 # a * b + c inside one expression may become one fused multiply-add

@@ -179,8 +179,11 @@ __device__ __forceinline__ int div_small(int s, int d, float rd) {
   return q;
 }
 
+// Site s of parity p: half of x, the index offsets h1 y and h2 z of its row,
+// and whether x is odd
 struct Coord {
-  int x, y, z;
+  int xh, yo, zo;
+  bool odd;
 };
 
 // Site order of an update launch.  sy = 0: the site index order (position P
@@ -207,14 +210,14 @@ __host__ __device__ inline SiteOrder site_order(const Geom& g, int sy) {
 
 __device__ __forceinline__ Coord site_coord(const Geom& g, int p, int s) {
   int z = div_small(s, g.h2, g.rh2);
-  int r = s - z * g.h2;
+  int zo = z * g.h2;
+  int r = s - zo;
   int y = div_small(r, g.h1, g.rh1);
-  int xh = r - y * g.h1;
-  return Coord{2 * xh + ((p + y + z) & 1), y, z};
+  int yo = y * g.h1;
+  return Coord{r - yo, yo, zo, (bool)((p + y + z) & 1)};
 }
-// the site at position P of the order o (P < N)
-__device__ __forceinline__ unsigned order_site(const Geom& g, const SiteOrder& o, unsigned P) {
-  if (!o.sy) return P;
+// the site at position P of the order o (P < N) of sy > 0 strip rows
+__device__ __forceinline__ unsigned strip_site(const Geom& g, const SiteOrder& o, unsigned P) {
   int r = div_small((int)P, g.h1, g.rh1);  // row in the order
   int k = (int)P - r * g.h1;
   int strip = div_small(r, o.rows, o.rrows);
@@ -234,13 +237,12 @@ struct Steps {
 };
 __device__ __forceinline__ Steps site_steps(const Geom& g, Coord c) {
   Steps t;
-  bool odd = c.x & 1;
-  t.p[0] = odd ? (c.x == g.lx - 1 ? 1 - g.h1 : 1) : 0;
-  t.m[0] = odd ? 0 : (c.x == 0 ? g.h1 - 1 : -1);
-  t.p[1] = c.y == g.ly - 1 ? -g.wy : g.h1;
-  t.m[1] = c.y == 0 ? g.wy : -g.h1;
-  t.p[2] = c.z == g.lz - 1 ? -g.wz : g.h2;
-  t.m[2] = c.z == 0 ? g.wz : -g.h2;
+  t.p[0] = c.odd ? (c.xh == g.h1 - 1 ? 1 - g.h1 : 1) : 0;
+  t.m[0] = c.odd ? 0 : (c.xh == 0 ? g.h1 - 1 : -1);
+  t.p[1] = c.yo == g.wy ? -g.wy : g.h1;
+  t.m[1] = c.yo == 0 ? g.wy : -g.h1;
+  t.p[2] = c.zo == g.wz ? -g.wz : g.h2;
+  t.m[2] = c.zo == 0 ? g.wz : -g.h2;
   return t;
 }
 // component d (0..2, a run-time value) of a step vector

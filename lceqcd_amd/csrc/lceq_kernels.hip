@@ -32,13 +32,59 @@ __device__ double block_sum_range(const double* __restrict__ x, int n) {
 
 // ================================================================ links
 
+// What a wave needs before it can issue its operand loads, as leading
+// arguments: the compiler's kernel-argument preload (build.py) has them in
+// scalar registers when the wave starts, 14 dwords, all there is room for.
+// Loaded from the argument segment they put one memory round trip ahead of
+// the gathers of every launch: 64^3 production sweep 172 -> 163.5 us,
+// reference sweep 91.4 -> 86.1 us, one gauge-fixing iteration 20.4 -> 19.2 us;
+// from 96^3 on 1%.  Pairs of 32-bit values share an argument.  (The same in
+// four vector-typed arguments cost 1.5% on lattices beyond the Infinity Cache.)
+#define HEAD_PARAMS                                                                           \
+  double *hU, double *hA, uint64_t hn, uint64_t hb, uint64_t hh, uint64_t hw, uint64_t hr
+#define HEAD_OF head_of(hU, hA, hn, hb, hh, hw, hr)
+enum { HEAD_EO = 1, HEAD_XCD = 2, HEAD_STRIPS = 4 };
+
+struct Head {
+  double *U, *A;
+  Geom g;  // without the extents
+  int nb, flags;
+};
+__device__ __forceinline__ int half0(uint64_t v) { return (int)(uint32_t)v; }
+__device__ __forceinline__ int half1(uint64_t v) { return (int)(uint32_t)(v >> 32); }
+__device__ __forceinline__ Head head_of(double* U, double* A, uint64_t hn, uint64_t hb,
+                                        uint64_t hh, uint64_t hw, uint64_t hr) {
+  Geom g{0, 0, 0, half0(hh), half1(hh), half0(hn), half1(hn),
+         __builtin_bit_cast(float, half0(hr)), __builtin_bit_cast(float, half1(hr)),
+         half0(hw), half1(hw)};
+  return Head{U, A, g, half0(hb), half1(hb)};
+}
+
+struct HeadArgs {
+  double *U, *A;
+  uint64_t n, b, h, w, r;
+};
+static uint64_t halves(int a, int b) {
+  return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
+}
+static HeadArgs head_args(const lceq_lattice* L, double* U, double* A, int nb, int eo) {
+  const Geom& g = L->g;
+  int flags = (eo ? HEAD_EO : 0) | (L->xcd ? HEAD_XCD : 0) | (L->strip ? HEAD_STRIPS : 0);
+  return HeadArgs{U, A, halves(g.n, g.npad), halves(nb, flags), halves(g.h1, g.h2),
+                  halves(g.wy, g.wz), halves(__builtin_bit_cast(int, g.rh1),
+                                             __builtin_bit_cast(int, g.rh2))};
+}
+
+// The rest of a link launch's arguments
 struct LinkArgs {
-  LinkSite site;
-  int reduce;
-  double* part;  // partial sums of this launch's slot: [LCEQ_NQ][pstride]
-  int pstride, nb, xcd;
   SiteOrder order;
-  int early;  // the schedule of link_update_site's EARLY (early_schedule)
+  double beta, beta_a;
+  const double* fed;
+  Philox key;
+  uint64_t pass;
+  int measflag, renorm, reduce;
+  int pstride;
+  double* part;  // partial sums of this launch's slot: [LCEQ_NQ][pstride]
 };
 
 // Schedule of the update launches (link_update_site, higgs_update_site):
@@ -59,85 +105,97 @@ __device__ __forceinline__ int shape_block(int nb, int xcd) {
 
 // One site per thread, TBX sites per block
 template <bool KP, bool FED, int TBX, int MU, bool EARLY>
-__global__ __launch_bounds__(TBX) void k_link(LinkArgs a) {
-  int blk = shape_block(a.nb, a.xcd);
+__global__ __launch_bounds__(TBX) void k_link(HEAD_PARAMS, LinkArgs a) {
+  const Head h = HEAD_OF;
+  int blk = shape_block(h.nb, h.flags & HEAD_XCD);
   unsigned P = (unsigned)(blk * TBX + threadIdx.x);
   double red[3] = {0.0, 0.0, 0.0};
-  if (P < (unsigned)a.site.g.n) {
-    LinkSite p = a.site;
+  if (P < (unsigned)h.g.n) {
+    LinkSite p;
+    p.g = h.g;
+    p.U = h.U;
+    p.A = h.A;
+    p.eo = h.flags & HEAD_EO;
     p.mu = MU;
-    link_update_site<KP, FED, EARLY>(p, order_site(p.g, a.order, P), red);
+    p.beta = a.beta;
+    p.beta_a = a.beta_a;
+    p.fed = a.fed;
+    p.key = a.key;
+    p.pass = a.pass;
+    p.measflag = a.measflag;
+    p.renorm = a.renorm;
+    unsigned s = h.flags & HEAD_STRIPS ? strip_site(p.g, a.order, P) : P;
+    link_update_site<KP, FED, EARLY>(p, s, red);
   }
   if (a.reduce) block_sum_store<3, TBX / 64>(red, a.part, a.pstride, blk);
 }
 
 int shape_blocks(const lceq_lattice* L) { return (L->g.n + L->tb - 1) / L->tb; }
 
+template <bool KP, bool FED, int MU, bool EARLY, int TBX>
+static void link_launch(lceq_lattice* L, int eo, const LinkArgs& a) {
+  int nb = shape_blocks(L);
+  HeadArgs h = head_args(L, L->U, L->A, nb, eo);
+  hipLaunchKernelGGL((k_link<KP, FED, TBX, MU, EARLY>), dim3(nb), dim3(TBX), 0, L->stream, h.U, h.A,
+                     h.n, h.b, h.h, h.w, h.r, a);
+}
+
 template <bool KP, bool FED, int MU, bool EARLY>
-static void link_dispatch_tb(lceq_lattice* L, const LinkArgs& a) {
-  dim3 grid(a.nb);
+static void link_dispatch_tb(lceq_lattice* L, int eo, const LinkArgs& a) {
   switch (L->tb) {
-    case 64: hipLaunchKernelGGL((k_link<KP, FED, 64, MU, EARLY>), grid, dim3(64), 0, L->stream, a); break;
-    case 128: hipLaunchKernelGGL((k_link<KP, FED, 128, MU, EARLY>), grid, dim3(128), 0, L->stream, a); break;
-    case 512: hipLaunchKernelGGL((k_link<KP, FED, 512, MU, EARLY>), grid, dim3(512), 0, L->stream, a); break;
-    default: hipLaunchKernelGGL((k_link<KP, FED, 256, MU, EARLY>), grid, dim3(256), 0, L->stream, a); break;
+    case 64: link_launch<KP, FED, MU, EARLY, 64>(L, eo, a); break;
+    case 128: link_launch<KP, FED, MU, EARLY, 128>(L, eo, a); break;
+    case 512: link_launch<KP, FED, MU, EARLY, 512>(L, eo, a); break;
+    default: link_launch<KP, FED, MU, EARLY, 256>(L, eo, a); break;
   }
 }
 
 template <bool KP, bool FED, int MU>
-static void link_dispatch_mu(lceq_lattice* L, const LinkArgs& a) {
-  if (a.early)
-    link_dispatch_tb<KP, FED, MU, true>(L, a);
+static void link_dispatch_mu(lceq_lattice* L, int eo, const LinkArgs& a) {
+  if (early_schedule(L))
+    link_dispatch_tb<KP, FED, MU, true>(L, eo, a);
   else
-    link_dispatch_tb<KP, FED, MU, false>(L, a);
+    link_dispatch_tb<KP, FED, MU, false>(L, eo, a);
 }
 
 // The direction is a template argument: the neighbour steps and link offsets
 // of the staple are then fixed at compile time.
 template <bool KP, bool FED>
-static void link_dispatch(lceq_lattice* L, const LinkArgs& a) {
-  switch (a.site.mu) {
-    case 0: link_dispatch_mu<KP, FED, 0>(L, a); break;
-    case 1: link_dispatch_mu<KP, FED, 1>(L, a); break;
-    default: link_dispatch_mu<KP, FED, 2>(L, a); break;
+static void link_dispatch(lceq_lattice* L, int eo, int mu, const LinkArgs& a) {
+  switch (mu) {
+    case 0: link_dispatch_mu<KP, FED, 0>(L, eo, a); break;
+    case 1: link_dispatch_mu<KP, FED, 1>(L, eo, a); break;
+    default: link_dispatch_mu<KP, FED, 2>(L, eo, a); break;
   }
 }
 
 void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int renorm_on_write,
                  const double* fed, uint64_t pass, int reduce) {
   LinkArgs a;
-  a.site.g = L->g;
-  a.site.U = L->U;
-  a.site.A = L->A;
-  a.site.eo = eo;
-  a.site.mu = mu;
-  a.site.beta = L->beta;
-  a.site.beta_a = L->beta_a;
-  a.site.fed = fed;
-  a.site.key = Philox{(uint32_t)L->seed, (uint32_t)(L->seed >> 32)};
-  a.site.pass = pass;
-  a.site.measflag = measflag;
-  a.site.renorm = renorm_on_write;
-  a.reduce = reduce;
-  a.part = L->partials + (size_t)(eo * 3 + mu) * LCEQ_NQ * L->pstride;
-  a.pstride = L->pstride;
-  a.nb = shape_blocks(L);
-  a.xcd = L->xcd;
   a.order = site_order(L->g, L->strip);
-  a.early = early_schedule(L) ? 1 : 0;
+  a.beta = L->beta;
+  a.beta_a = L->beta_a;
+  a.fed = fed;
+  a.key = Philox{(uint32_t)L->seed, (uint32_t)(L->seed >> 32)};
+  a.pass = pass;
+  a.measflag = measflag;
+  a.renorm = renorm_on_write;
+  a.reduce = reduce;
+  a.pstride = L->pstride;
+  a.part = L->partials + (size_t)(eo * 3 + mu) * LCEQ_NQ * L->pstride;
   int kc = kp ? KC_LINK_KP : KC_LINK_OR;
   prof_begin(L, kc);
   prof_count(L, kc);
   if (kp) {
     if (fed)
-      link_dispatch<true, true>(L, a);
+      link_dispatch<true, true>(L, eo, mu, a);
     else
-      link_dispatch<true, false>(L, a);
+      link_dispatch<true, false>(L, eo, mu, a);
   } else {
     if (fed)
-      link_dispatch<false, true>(L, a);
+      link_dispatch<false, true>(L, eo, mu, a);
     else
-      link_dispatch<false, false>(L, a);
+      link_dispatch<false, false>(L, eo, mu, a);
   }
   prof_end(L, kc);
 }
@@ -322,73 +380,94 @@ void launch_force(lceq_lattice* L, int eo) {
 }
 
 struct HiggsArgs {
-  HiggsSite site;
-  double* part;
-  int pstride, nb, xcd;
   SiteOrder order;
-  int early;  // as LinkArgs::early
+  int imode, measflag;
+  double beta_a, beta_2, beta_4;
+  const double* delta;
+  const double* fed;
+  Philox key;
+  uint64_t pass;
+  double* part;
+  int pstride;
 };
 
 template <int KIND, bool FED, int TBX, bool EARLY>
-__global__ __launch_bounds__(TBX) void k_higgs(HiggsArgs a) {
-  int blk = shape_block(a.nb, a.xcd);
+__global__ __launch_bounds__(TBX) void k_higgs(HEAD_PARAMS, HiggsArgs a) {
+  const Head h = HEAD_OF;
+  int blk = shape_block(h.nb, h.flags & HEAD_XCD);
   unsigned P = (unsigned)(blk * TBX + threadIdx.x);
   double red[4] = {0.0, 0.0, 0.0, 0.0};
-  if (P < (unsigned)a.site.g.n)
-    higgs_update_site<KIND, FED, EARLY>(a.site, order_site(a.site.g, a.order, P), red);
+  if (P < (unsigned)h.g.n) {
+    HiggsSite p;
+    p.g = h.g;
+    p.U = h.U;
+    p.A = h.A;
+    p.eo = h.flags & HEAD_EO;
+    p.imode = a.imode;
+    p.beta_a = a.beta_a;
+    p.beta_2 = a.beta_2;
+    p.beta_4 = a.beta_4;
+    p.delta = a.delta;
+    p.fed = a.fed;
+    p.key = a.key;
+    p.pass = a.pass;
+    p.measflag = a.measflag;
+    unsigned s = h.flags & HEAD_STRIPS ? strip_site(p.g, a.order, P) : P;
+    higgs_update_site<KIND, FED, EARLY>(p, s, red);
+  }
   block_sum_store<4, TBX / 64>(red, a.part, a.pstride, blk);
 }
 
+template <int KIND, bool FED, bool EARLY, int TBX>
+static void higgs_launch(lceq_lattice* L, int eo, const HiggsArgs& a) {
+  int nb = shape_blocks(L);
+  HeadArgs h = head_args(L, L->U, L->A, nb, eo);
+  hipLaunchKernelGGL((k_higgs<KIND, FED, TBX, EARLY>), dim3(nb), dim3(TBX), 0, L->stream, h.U, h.A,
+                     h.n, h.b, h.h, h.w, h.r, a);
+}
+
 template <int KIND, bool FED, bool EARLY>
-static void higgs_dispatch_tb(lceq_lattice* L, const HiggsArgs& a) {
-  dim3 grid(a.nb);
+static void higgs_dispatch_tb(lceq_lattice* L, int eo, const HiggsArgs& a) {
   switch (L->tb) {
-    case 64: hipLaunchKernelGGL((k_higgs<KIND, FED, 64, EARLY>), grid, dim3(64), 0, L->stream, a); break;
-    case 128: hipLaunchKernelGGL((k_higgs<KIND, FED, 128, EARLY>), grid, dim3(128), 0, L->stream, a); break;
-    case 512: hipLaunchKernelGGL((k_higgs<KIND, FED, 512, EARLY>), grid, dim3(512), 0, L->stream, a); break;
-    default: hipLaunchKernelGGL((k_higgs<KIND, FED, 256, EARLY>), grid, dim3(256), 0, L->stream, a); break;
+    case 64: higgs_launch<KIND, FED, EARLY, 64>(L, eo, a); break;
+    case 128: higgs_launch<KIND, FED, EARLY, 128>(L, eo, a); break;
+    case 512: higgs_launch<KIND, FED, EARLY, 512>(L, eo, a); break;
+    default: higgs_launch<KIND, FED, EARLY, 256>(L, eo, a); break;
   }
 }
 
 // the early issue exists for ahiggs1 only (EARLY = KIND == 1 there)
 template <int KIND, bool FED>
-static void higgs_dispatch(lceq_lattice* L, const HiggsArgs& a) {
-  if (a.early)
-    higgs_dispatch_tb<KIND, FED, KIND == 1>(L, a);
+static void higgs_dispatch(lceq_lattice* L, int eo, const HiggsArgs& a) {
+  if (early_schedule(L))
+    higgs_dispatch_tb<KIND, FED, KIND == 1>(L, eo, a);
   else
-    higgs_dispatch_tb<KIND, FED, false>(L, a);
+    higgs_dispatch_tb<KIND, FED, false>(L, eo, a);
 }
 
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
                   uint64_t pass) {
   HiggsArgs a;
-  a.site.g = L->g;
-  a.site.U = L->U;
-  a.site.A = L->A;
-  a.site.eo = eo;
-  a.site.imode = L->imode;
-  a.site.beta_a = L->beta_a;
-  a.site.beta_2 = L->beta_2;
-  a.site.beta_4 = L->beta_4;
-  a.site.delta = L->obs + OBS_DELTA;
-  a.site.fed = fed;
-  a.site.key = Philox{(uint32_t)L->seed, (uint32_t)(L->seed >> 32)};
-  a.site.pass = pass;
-  a.site.measflag = measflag;
+  a.order = site_order(L->g, L->strip);
+  a.imode = L->imode;
+  a.measflag = measflag;
+  a.beta_a = L->beta_a;
+  a.beta_2 = L->beta_2;
+  a.beta_4 = L->beta_4;
+  a.delta = L->obs + OBS_DELTA;
+  a.fed = fed;
+  a.key = Philox{(uint32_t)L->seed, (uint32_t)(L->seed >> 32)};
+  a.pass = pass;
   a.part = L->partials + (size_t)(6 + eo) * LCEQ_NQ * L->pstride;
   a.pstride = L->pstride;
-  a.nb = shape_blocks(L);
-  a.xcd = L->xcd;
-  a.order = site_order(L->g, L->strip);
-  a.early = early_schedule(L) ? 1 : 0;
   prof_begin(L, KC_HIGGS);
   prof_count(L, KC_HIGGS);
   if (kind == 1) {
-    if (fed) higgs_dispatch<1, true>(L, a); else higgs_dispatch<1, false>(L, a);
+    if (fed) higgs_dispatch<1, true>(L, eo, a); else higgs_dispatch<1, false>(L, eo, a);
   } else if (kind == 2) {
-    if (fed) higgs_dispatch<2, true>(L, a); else higgs_dispatch<2, false>(L, a);
+    if (fed) higgs_dispatch<2, true>(L, eo, a); else higgs_dispatch<2, false>(L, eo, a);
   } else {
-    if (fed) higgs_dispatch<3, true>(L, a); else higgs_dispatch<3, false>(L, a);
+    if (fed) higgs_dispatch<3, true>(L, eo, a); else higgs_dispatch<3, false>(L, eo, a);
   }
   prof_end(L, KC_HIGGS);
 }
@@ -459,14 +538,11 @@ void launch_check_fields(lceq_lattice* L, double* part) {
 // ========================================================= gauge fixing
 
 struct GfArgs {
-  Geom g;
-  double* Uf;
-  double* Af;
-  int eo, compute_da, renorm, guarded;
+  int compute_da, renorm, guarded;
   double lambda, alpha;
   double* obs;  // OBS_GF_DONE read when guarded; the convergence test writes
   double* part;
-  int pstride, nb;
+  int pstride;
   // convergence test of the previous iteration at the start of this launch
   // (landau_gauge iterations after the first of a batch): `iter` iterations
   // are complete, their last da is in `part`
@@ -514,12 +590,14 @@ __device__ __forceinline__ bool gfix_stop(double da, double iter, double limit_o
 // first repeats the convergence test of the previous iteration (the same
 // sum in the same order, so all blocks agree) and the launch returns when
 // the loop has ended; the operand loads are issued before the test.
-__global__ __launch_bounds__(256) void k_gfix(GfArgs p) {
-  const Geom& g = p.g;
-  int blk = xcd_block(p.nb);
+__global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
+  const Head h = HEAD_OF;
+  const Geom& g = h.g;
+  double *Uf = h.U, *Af = h.A;
+  int blk = xcd_block(h.nb);
   int s = blk * TB + threadIdx.x;
   bool act = s < g.n;
-  int eo = p.eo, oe = eo ^ 1;
+  int eo = h.flags & HEAD_EO, oe = eo ^ 1;
   su2 ux[3], uy[3];
   int sy[3];
   vec3 af;
@@ -528,16 +606,16 @@ __global__ __launch_bounds__(256) void k_gfix(GfArgs p) {
 #pragma unroll
     for (int mu = 0; mu < 3; ++mu) {
       sy[mu] = s + st.m[mu];
-      ux[mu] = ld_link(p.Uf, g, mu, eo, s);
-      uy[mu] = ld_link(p.Uf, g, mu, oe, sy[mu]);
+      ux[mu] = ld_link(Uf, g, mu, eo, s);
+      uy[mu] = ld_link(Uf, g, mu, oe, sy[mu]);
     }
-    af = ld_higgs(p.Af, g, eo, s);
+    af = ld_higgs(Af, g, eo, s);
   }
   // uniform over the grid; tested after the operand loads are issued, so that
   // its round trip overlaps theirs
   if (p.guarded && p.obs[OBS_GF_DONE] != 0.0) return;
   if (p.check) {
-    double da = gfix_da(p.part, p.nb, (double)g.n);
+    double da = gfix_da(p.part, h.nb, (double)g.n);
     if (gfix_stop(da, p.iter, p.limit_or, p.max_iter, p.obs, blk == 0 && threadIdx.x == 0))
       return;  // block-uniform
   }
@@ -569,7 +647,7 @@ __global__ __launch_bounds__(256) void k_gfix(GfArgs p) {
       o.a = c_mk(cos(tho), -t2);
       o.b = c_mk(-(f * o.b.re), -(f * o.b.im));
     }
-    st_higgs(p.Af, g, eo, s, adj_rot<false>(o, af));  // g X(a_f) g^+, :243-252
+    st_higgs(Af, g, eo, s, adj_rot<false>(o, af));  // g X(a_f) g^+, :243-252
 #pragma unroll
     for (int mu = 0; mu < 3; ++mu) {  // :256-324
       su2 nx = m_nn(o, ux[mu]);
@@ -578,8 +656,8 @@ __global__ __launch_bounds__(256) void k_gfix(GfArgs p) {
         nx = normalized(nx);
         ny = normalized(ny);
       }
-      st_link(p.Uf, g, mu, eo, s, nx);
-      st_link(p.Uf, g, mu, oe, sy[mu], ny);
+      st_link(Uf, g, mu, eo, s, nx);
+      st_link(Uf, g, mu, oe, sy[mu], ny);
     }
   }
   if (p.compute_da) block_sum_store<1>(red, p.part, p.pstride, blk);
@@ -603,10 +681,6 @@ __global__ __launch_bounds__(256) void k_gfix_finalize(const double* __restrict_
 void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check,
                  int iter) {
   GfArgs a;
-  a.g = L->g;
-  a.Uf = L->Uf;
-  a.Af = L->Af;
-  a.eo = eo;
   a.compute_da = compute_da;
   a.renorm = renorm;
   a.guarded = guarded;
@@ -615,14 +689,16 @@ void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarde
   a.obs = L->obs;
   a.part = L->partials;
   a.pstride = L->pstride;
-  a.nb = blocks_for(L->g.n);
   a.check = check;
   a.iter = (double)iter;
   a.limit_or = L->limit_or;
   a.max_iter = (double)L->max_iter;
   prof_begin(L, KC_GFIX);
   prof_count(L, KC_GFIX);
-  hipLaunchKernelGGL(k_gfix, dim3(a.nb), dim3(TB), 0, L->stream, a);
+  int nb = blocks_for(L->g.n);
+  HeadArgs h = head_args(L, L->Uf, L->Af, nb, eo);
+  hipLaunchKernelGGL(k_gfix, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A,
+                     h.n, h.b, h.h, h.w, h.r, a);
   prof_end(L, KC_GFIX);
 }
 
