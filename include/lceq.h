@@ -89,11 +89,11 @@ int lceq_get_shape(lceq_lattice *L, int *threads_per_block, int *xcd_order);
  * sweep, shapes (64,128,256,512) x (launch order, XCD order).  Philox only. */
 int lceq_autotune(lceq_lattice *L, int n_or, int trials, double *ms);
 /* site order of the link and Higgs updates (no counterpart in the
- * reference): strip_rows = 0 takes the sites in index order; a power of two
- * >= 2 dividing ly (with ly * lz < 2^22) takes the rows (y, z) of a parity
- * in strips of that many y rows, each strip advancing through z, so that the
- * z neighbours of the sites in flight stay in the L2 of a lattice larger than
- * the Infinity Cache.
+ * reference): a power of two >= 2 dividing ly (with ly * lz < 2^22) takes the
+ * rows (y, z) of a parity in strips of that many y rows, each strip advancing
+ * through z, so that the z neighbours of the sites in flight stay in the L2;
+ * strip_rows = 0 leaves the order to the library: index order, and strips
+ * where a z plane is large (8192 sites of a parity or more).
  * Fields do not depend on the order; plaquette and Higgs sums are added in an
  * order-dependent way.  Default 0. */
 int lceq_set_site_order(lceq_lattice *L, int strip_rows);

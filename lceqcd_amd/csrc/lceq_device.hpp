@@ -195,15 +195,16 @@ struct Coord {
 // XCD reuse them from its L2 on lattices too large for the Infinity Cache.
 struct SiteOrder {
   int sy, lsy;  // strip height and its log2
-  int rows;     // sy * lz: rows per strip
+  int rows;     // sy * planes: rows per strip
   float rrows;  // 1 / rows
 };
-__host__ __device__ inline SiteOrder site_order(const Geom& g, int sy) {
+// (over lz planes)
+__host__ __device__ inline SiteOrder site_order(int lz, int sy) {
   SiteOrder o;
   o.sy = sy;
   o.lsy = 0;
   while ((1 << o.lsy) < sy) ++o.lsy;
-  o.rows = sy * g.lz;
+  o.rows = sy * lz;
   o.rrows = sy ? 1.0f / (float)o.rows : 0.0f;
   return o;
 }

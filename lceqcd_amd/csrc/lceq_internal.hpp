@@ -63,7 +63,8 @@ struct lceq_lattice {
   // launch shape of the link and Higgs updates: threads (= sites) per block
   // 64/128/256/512 and the XCD-aware block order (partials sized for 64)
   int tb, xcd;
-  // site order of those launches: strips of `strip` y rows (0: index order)
+  // site order of those launches: strips of `strip` y rows (0: by the
+  // lattice's shape, strip_rows)
   int strip;
   uint64_t seed, pass;
   // timing of one kernel class (bench instrumentation): one event pair per
@@ -98,6 +99,8 @@ inline const char* geom_reject(int lx, int ly, int lz) {
 enum KernelClass { KC_NONE = 0, KC_LINK_KP = 1, KC_LINK_OR = 2, KC_HIGGS = 3, KC_GFIX = 4 };
 
 int blocks_for(int n);
+// the strip rows of the update launches' site order (0: index order)
+int strip_rows(const lceq_lattice* L);
 // blocks of the link and Higgs update launches at the lattice's launch shape
 int shape_blocks(const lceq_lattice* L);
 
@@ -133,8 +136,13 @@ void transfer_user(int change);
 // launchers (lceq_kernels.hip); all enqueue on L->stream, no host sync.
 // Link launches use reduction slots 0-5 ((eo, mu) order), Higgs launches
 // slots 6-7 (eo); with reduce = 0 a launch writes no partial sums.
+// range (Philox; Higgs: ahiggs1 only): the launch covers these sites alone,
+// whole z planes; with partial sums its start is a multiple of the block size.
+struct SiteRange {
+  int p0, len;  // sites p0 .. p0 + len - 1, modulo the parity's n
+};
 void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int renorm_on_write,
-                 const double* fed, uint64_t pass, int reduce);
+                 const double* fed, uint64_t pass, int reduce, const SiteRange* range = nullptr);
 // One-block reduction of the partial sums into the observables: link_kind
 // 0 none, 1 KP (agauge), 2 overrelaxation; higgs_kind 0 none, 1-3 ahiggs1-3;
 // with hist_row the observables are also copied into that history row.
@@ -150,7 +158,7 @@ void launch_export(lceq_lattice* L, const double* dev, size_t n);
 void launch_staples(lceq_lattice* L, int eo, int mu);
 void launch_force(lceq_lattice* L, int eo);
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
-                  uint64_t pass);
+                  uint64_t pass, const SiteRange* range = nullptr);
 void launch_renorm(lceq_lattice* L, double* U);
 // per-block (unitarity deviation, non-finite count) of U and A into part[2 nb]
 void launch_check_fields(lceq_lattice* L, double* part);

@@ -43,7 +43,7 @@ __device__ double block_sum_range(const double* __restrict__ x, int n) {
 #define HEAD_PARAMS                                                                           \
   double *hU, double *hA, uint64_t hn, uint64_t hb, uint64_t hh, uint64_t hw, uint64_t hr
 #define HEAD_OF head_of(hU, hA, hn, hb, hh, hw, hr)
-enum { HEAD_EO = 1, HEAD_XCD = 2, HEAD_STRIPS = 4 };
+enum { HEAD_EO = 1, HEAD_XCD = 2, HEAD_STRIPS = 4, HEAD_WRAP = 8 };
 
 struct Head {
   double *U, *A;
@@ -67,10 +67,15 @@ struct HeadArgs {
 static uint64_t halves(int a, int b) {
   return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
 }
-static HeadArgs head_args(const lceq_lattice* L, double* U, double* A, int nb, int eo) {
+// r: the launch covers a range of the sites only; its head then carries the
+// range's length and start in place of n and the number of blocks
+static HeadArgs head_args(const lceq_lattice* L, double* U, double* A, int nb, int eo,
+                          const SiteRange* r = nullptr) {
   const Geom& g = L->g;
-  int flags = (eo ? HEAD_EO : 0) | (L->xcd ? HEAD_XCD : 0) | (L->strip ? HEAD_STRIPS : 0);
-  return HeadArgs{U, A, halves(g.n, g.npad), halves(nb, flags), halves(g.h1, g.h2),
+  int flags = (eo ? HEAD_EO : 0) | (L->xcd ? HEAD_XCD : 0) | (strip_rows(L) ? HEAD_STRIPS : 0);
+  if (r && (int64_t)r->p0 + r->len > g.n) flags |= HEAD_WRAP;
+  return HeadArgs{U, A, halves(r ? r->len : g.n, g.npad), halves(r ? r->p0 : nb, flags),
+                  halves(g.h1, g.h2),
                   halves(g.wy, g.wz), halves(__builtin_bit_cast(int, g.rh1),
                                              __builtin_bit_cast(int, g.rh2))};
 }
@@ -84,6 +89,7 @@ struct LinkArgs {
   uint64_t pass;
   int measflag, renorm, reduce;
   int pstride;
+  int n, nb;     // sites of the parity and blocks of the slot (RANGE)
   double* part;  // partial sums of this launch's slot: [LCEQ_NQ][pstride]
 };
 
@@ -96,6 +102,26 @@ static bool early_schedule(const lceq_lattice* L) {
   return L->g.n >= 32768 && 30.0 * 8.0 * (double)L->g.npad <= 256.0 * 1024.0 * 1024.0;
 }
 
+// The strip rows of the launches: the caller's, or by the lattice's shape.  In
+// index order a site's z neighbours are a plane away; from 8192 sites a plane
+// and parity on (4 MB of fields, one XCD's L2) they have left the L2 when the
+// next plane reads them, and strips keep them.  Production sweeps in ns per
+// site, index order against strips: 128x128x100 0.672 0.645, 144x144x96 0.711
+// 0.642, 160x160x80 0.784 0.636, 192x192x48 0.882 0.648, 256x256x32 0.897
+// 0.636; 112^3 0.654 0.660 and 64^3 0.640 0.663 the other way.  Strips of 1024
+// to 2047 sites a plane: 512 cost up to 15% (128x128x64 0.790 against 0.697).
+// Where no power of two of rows gives that, strips of two rows, which pay from
+// 12800 sites a plane on (200x200x40 0.890 0.677).
+int strip_rows(const lceq_lattice* L) {
+  const Geom& g = L->g;
+  if (L->strip) return L->strip;
+  if (g.h2 < 8192 || (int64_t)g.ly * g.lz >= (int64_t)1 << 22) return 0;
+  int sy = 2;
+  while ((int64_t)sy * g.h1 < 1024) sy *= 2;
+  if (sy * g.h1 < 2048 && g.ly % sy == 0) return sy;
+  return g.h2 >= 12800 ? 2 : 0;
+}
+
 // Block index in the launch's block order: XCD-aware (contiguous sites per
 // XCD) or the launch order
 __device__ __forceinline__ int shape_block(int nb, int xcd) {
@@ -103,11 +129,23 @@ __device__ __forceinline__ int shape_block(int nb, int xcd) {
   return xcd ? b : (int)blockIdx.x;
 }
 
+// Site and slot block of a launch over a range of the sites, which may run on
+// past the last site to the first: s counts from the range's start
+__device__ __forceinline__ unsigned range_site(const Head& h, unsigned s, int n) {
+  s += (unsigned)h.nb;
+  return h.flags & HEAD_WRAP && s >= (unsigned)n ? s - (unsigned)n : s;
+}
+template <int TBX>
+__device__ __forceinline__ int range_block(const Head& h, int blk, int nb) {
+  blk += h.nb / TBX;
+  return blk >= nb ? blk - nb : blk;
+}
+
 // One site per thread, TBX sites per block
-template <bool KP, bool FED, int TBX, int MU, bool EARLY>
+template <bool KP, bool FED, int TBX, int MU, bool EARLY, bool RANGE>
 __global__ __launch_bounds__(TBX) void k_link(HEAD_PARAMS, LinkArgs a) {
   const Head h = HEAD_OF;
-  int blk = shape_block(h.nb, h.flags & HEAD_XCD);
+  int blk = shape_block(RANGE ? (h.g.n + TBX - 1) / TBX : h.nb, h.flags & HEAD_XCD);
   unsigned P = (unsigned)(blk * TBX + threadIdx.x);
   double red[3] = {0.0, 0.0, 0.0};
   if (P < (unsigned)h.g.n) {
@@ -125,54 +163,63 @@ __global__ __launch_bounds__(TBX) void k_link(HEAD_PARAMS, LinkArgs a) {
     p.measflag = a.measflag;
     p.renorm = a.renorm;
     unsigned s = h.flags & HEAD_STRIPS ? strip_site(p.g, a.order, P) : P;
+    if (RANGE) s = range_site(h, s, a.n);
     link_update_site<KP, FED, EARLY>(p, s, red);
   }
-  if (a.reduce) block_sum_store<3, TBX / 64>(red, a.part, a.pstride, blk);
+  if (a.reduce)
+    block_sum_store<3, TBX / 64>(red, a.part, a.pstride,
+                                 RANGE ? range_block<TBX>(h, blk, a.nb) : blk);
 }
 
 int shape_blocks(const lceq_lattice* L) { return (L->g.n + L->tb - 1) / L->tb; }
 
-template <bool KP, bool FED, int MU, bool EARLY, int TBX>
-static void link_launch(lceq_lattice* L, int eo, const LinkArgs& a) {
-  int nb = shape_blocks(L);
-  HeadArgs h = head_args(L, L->U, L->A, nb, eo);
-  hipLaunchKernelGGL((k_link<KP, FED, TBX, MU, EARLY>), dim3(nb), dim3(TBX), 0, L->stream, h.U, h.A,
-                     h.n, h.b, h.h, h.w, h.r, a);
+template <bool KP, bool FED, int MU, bool EARLY, bool RANGE, int TBX>
+static void link_launch(lceq_lattice* L, int eo, const LinkArgs& a, const SiteRange* r) {
+  int nb = RANGE ? (r->len + TBX - 1) / TBX : shape_blocks(L);
+  HeadArgs h = head_args(L, L->U, L->A, nb, eo, r);
+  hipLaunchKernelGGL((k_link<KP, FED, TBX, MU, EARLY, RANGE>), dim3(nb), dim3(TBX), 0, L->stream,
+                     h.U, h.A, h.n, h.b, h.h, h.w, h.r, a);
 }
 
-template <bool KP, bool FED, int MU, bool EARLY>
-static void link_dispatch_tb(lceq_lattice* L, int eo, const LinkArgs& a) {
+template <bool KP, bool FED, int MU, bool EARLY, bool RANGE>
+static void link_dispatch_tb(lceq_lattice* L, int eo, const LinkArgs& a, const SiteRange* r) {
   switch (L->tb) {
-    case 64: link_launch<KP, FED, MU, EARLY, 64>(L, eo, a); break;
-    case 128: link_launch<KP, FED, MU, EARLY, 128>(L, eo, a); break;
-    case 512: link_launch<KP, FED, MU, EARLY, 512>(L, eo, a); break;
-    default: link_launch<KP, FED, MU, EARLY, 256>(L, eo, a); break;
+    case 64: link_launch<KP, FED, MU, EARLY, RANGE, 64>(L, eo, a, r); break;
+    case 128: link_launch<KP, FED, MU, EARLY, RANGE, 128>(L, eo, a, r); break;
+    case 512: link_launch<KP, FED, MU, EARLY, RANGE, 512>(L, eo, a, r); break;
+    default: link_launch<KP, FED, MU, EARLY, RANGE, 256>(L, eo, a, r); break;
   }
 }
 
 template <bool KP, bool FED, int MU>
-static void link_dispatch_mu(lceq_lattice* L, int eo, const LinkArgs& a) {
+static void link_dispatch_mu(lceq_lattice* L, int eo, const LinkArgs& a, const SiteRange* r) {
+  if constexpr (!FED) {
+    if (r) return link_dispatch_tb<KP, FED, MU, true, true>(L, eo, a, r);
+  }
   if (early_schedule(L))
-    link_dispatch_tb<KP, FED, MU, true>(L, eo, a);
+    link_dispatch_tb<KP, FED, MU, true, false>(L, eo, a, nullptr);
   else
-    link_dispatch_tb<KP, FED, MU, false>(L, eo, a);
+    link_dispatch_tb<KP, FED, MU, false, false>(L, eo, a, nullptr);
 }
 
 // The direction is a template argument: the neighbour steps and link offsets
 // of the staple are then fixed at compile time.
 template <bool KP, bool FED>
-static void link_dispatch(lceq_lattice* L, int eo, int mu, const LinkArgs& a) {
+static void link_dispatch(lceq_lattice* L, int eo, int mu, const LinkArgs& a,
+                          const SiteRange* r) {
   switch (mu) {
-    case 0: link_dispatch_mu<KP, FED, 0>(L, eo, a); break;
-    case 1: link_dispatch_mu<KP, FED, 1>(L, eo, a); break;
-    default: link_dispatch_mu<KP, FED, 2>(L, eo, a); break;
+    case 0: link_dispatch_mu<KP, FED, 0>(L, eo, a, r); break;
+    case 1: link_dispatch_mu<KP, FED, 1>(L, eo, a, r); break;
+    default: link_dispatch_mu<KP, FED, 2>(L, eo, a, r); break;
   }
 }
 
 void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int renorm_on_write,
-                 const double* fed, uint64_t pass, int reduce) {
+                 const double* fed, uint64_t pass, int reduce, const SiteRange* range) {
   LinkArgs a;
-  a.order = site_order(L->g, L->strip);
+  a.n = L->g.n;
+  a.nb = shape_blocks(L);
+  a.order = site_order(range ? range->len / L->g.h2 : L->g.lz, strip_rows(L));
   a.beta = L->beta;
   a.beta_a = L->beta_a;
   a.fed = fed;
@@ -188,14 +235,14 @@ void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int reno
   prof_count(L, kc);
   if (kp) {
     if (fed)
-      link_dispatch<true, true>(L, eo, mu, a);
+      link_dispatch<true, true>(L, eo, mu, a, range);
     else
-      link_dispatch<true, false>(L, eo, mu, a);
+      link_dispatch<true, false>(L, eo, mu, a, range);
   } else {
     if (fed)
-      link_dispatch<false, true>(L, eo, mu, a);
+      link_dispatch<false, true>(L, eo, mu, a, range);
     else
-      link_dispatch<false, false>(L, eo, mu, a);
+      link_dispatch<false, false>(L, eo, mu, a, range);
   }
   prof_end(L, kc);
 }
@@ -389,12 +436,13 @@ struct HiggsArgs {
   uint64_t pass;
   double* part;
   int pstride;
+  int n, nb;  // as LinkArgs
 };
 
-template <int KIND, bool FED, int TBX, bool EARLY>
+template <int KIND, bool FED, int TBX, bool EARLY, bool RANGE>
 __global__ __launch_bounds__(TBX) void k_higgs(HEAD_PARAMS, HiggsArgs a) {
   const Head h = HEAD_OF;
-  int blk = shape_block(h.nb, h.flags & HEAD_XCD);
+  int blk = shape_block(RANGE ? (h.g.n + TBX - 1) / TBX : h.nb, h.flags & HEAD_XCD);
   unsigned P = (unsigned)(blk * TBX + threadIdx.x);
   double red[4] = {0.0, 0.0, 0.0, 0.0};
   if (P < (unsigned)h.g.n) {
@@ -413,42 +461,50 @@ __global__ __launch_bounds__(TBX) void k_higgs(HEAD_PARAMS, HiggsArgs a) {
     p.pass = a.pass;
     p.measflag = a.measflag;
     unsigned s = h.flags & HEAD_STRIPS ? strip_site(p.g, a.order, P) : P;
+    if (RANGE) s = range_site(h, s, a.n);
     higgs_update_site<KIND, FED, EARLY>(p, s, red);
   }
-  block_sum_store<4, TBX / 64>(red, a.part, a.pstride, blk);
+  block_sum_store<4, TBX / 64>(red, a.part, a.pstride,
+                               RANGE ? range_block<TBX>(h, blk, a.nb) : blk);
 }
 
-template <int KIND, bool FED, bool EARLY, int TBX>
-static void higgs_launch(lceq_lattice* L, int eo, const HiggsArgs& a) {
-  int nb = shape_blocks(L);
-  HeadArgs h = head_args(L, L->U, L->A, nb, eo);
-  hipLaunchKernelGGL((k_higgs<KIND, FED, TBX, EARLY>), dim3(nb), dim3(TBX), 0, L->stream, h.U, h.A,
-                     h.n, h.b, h.h, h.w, h.r, a);
+template <int KIND, bool FED, bool EARLY, bool RANGE, int TBX>
+static void higgs_launch(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
+  int nb = RANGE ? (r->len + TBX - 1) / TBX : shape_blocks(L);
+  HeadArgs h = head_args(L, L->U, L->A, nb, eo, r);
+  hipLaunchKernelGGL((k_higgs<KIND, FED, TBX, EARLY, RANGE>), dim3(nb), dim3(TBX), 0, L->stream,
+                     h.U, h.A, h.n, h.b, h.h, h.w, h.r, a);
 }
 
-template <int KIND, bool FED, bool EARLY>
-static void higgs_dispatch_tb(lceq_lattice* L, int eo, const HiggsArgs& a) {
+template <int KIND, bool FED, bool EARLY, bool RANGE>
+static void higgs_dispatch_tb(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
   switch (L->tb) {
-    case 64: higgs_launch<KIND, FED, EARLY, 64>(L, eo, a); break;
-    case 128: higgs_launch<KIND, FED, EARLY, 128>(L, eo, a); break;
-    case 512: higgs_launch<KIND, FED, EARLY, 512>(L, eo, a); break;
-    default: higgs_launch<KIND, FED, EARLY, 256>(L, eo, a); break;
+    case 64: higgs_launch<KIND, FED, EARLY, RANGE, 64>(L, eo, a, r); break;
+    case 128: higgs_launch<KIND, FED, EARLY, RANGE, 128>(L, eo, a, r); break;
+    case 512: higgs_launch<KIND, FED, EARLY, RANGE, 512>(L, eo, a, r); break;
+    default: higgs_launch<KIND, FED, EARLY, RANGE, 256>(L, eo, a, r); break;
   }
 }
 
-// the early issue exists for ahiggs1 only (EARLY = KIND == 1 there)
+// the early issue exists for ahiggs1 only (EARLY = KIND == 1 there), and so do
+// launches over a range
 template <int KIND, bool FED>
-static void higgs_dispatch(lceq_lattice* L, int eo, const HiggsArgs& a) {
+static void higgs_dispatch(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
+  if constexpr (KIND == 1 && !FED) {
+    if (r) return higgs_dispatch_tb<KIND, FED, true, true>(L, eo, a, r);
+  }
   if (early_schedule(L))
-    higgs_dispatch_tb<KIND, FED, KIND == 1>(L, eo, a);
+    higgs_dispatch_tb<KIND, FED, KIND == 1, false>(L, eo, a, nullptr);
   else
-    higgs_dispatch_tb<KIND, FED, false>(L, eo, a);
+    higgs_dispatch_tb<KIND, FED, false, false>(L, eo, a, nullptr);
 }
 
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
-                  uint64_t pass) {
+                  uint64_t pass, const SiteRange* range) {
   HiggsArgs a;
-  a.order = site_order(L->g, L->strip);
+  a.n = L->g.n;
+  a.nb = shape_blocks(L);
+  a.order = site_order(range ? range->len / L->g.h2 : L->g.lz, strip_rows(L));
   a.imode = L->imode;
   a.measflag = measflag;
   a.beta_a = L->beta_a;
@@ -463,11 +519,11 @@ void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double*
   prof_begin(L, KC_HIGGS);
   prof_count(L, KC_HIGGS);
   if (kind == 1) {
-    if (fed) higgs_dispatch<1, true>(L, eo, a); else higgs_dispatch<1, false>(L, eo, a);
+    if (fed) higgs_dispatch<1, true>(L, eo, a, range); else higgs_dispatch<1, false>(L, eo, a, range);
   } else if (kind == 2) {
-    if (fed) higgs_dispatch<2, true>(L, eo, a); else higgs_dispatch<2, false>(L, eo, a);
+    if (fed) higgs_dispatch<2, true>(L, eo, a, range); else higgs_dispatch<2, false>(L, eo, a, range);
   } else {
-    if (fed) higgs_dispatch<3, true>(L, eo, a); else higgs_dispatch<3, false>(L, eo, a);
+    if (fed) higgs_dispatch<3, true>(L, eo, a, range); else higgs_dispatch<3, false>(L, eo, a, range);
   }
   prof_end(L, KC_HIGGS);
 }

@@ -138,8 +138,9 @@ class Lattice:
 
     # -------------------------------------------------------------- uniforms
     def set_site_order(self, strip_rows=0):
-        """Site order of the link and Higgs updates: 0 (index order) or strips
-        of ``strip_rows`` y rows advancing through z (same fields)."""
+        """Site order of the link and Higgs updates: 0 (the library's: index
+        order, strips on lattices with large planes) or strips of
+        ``strip_rows`` y rows advancing through z (same fields)."""
         self._check(self._L.lceq_set_site_order(self.h, int(strip_rows)))
 
     def get_site_order(self):
