@@ -719,16 +719,19 @@ extern "C" int lceq_gauss(lceq_lattice* L, double* x, const double* r, int nh) {
   return LCEQ_OK;
 }
 
-// both parities of one Higgs routine (kind 1/2/3 = ahiggs1/2/3); partial
-// sums land in slots 6-7 for launch_finalize
-static int higgs_sweep(lceq_lattice* L, int kind, int measflag) {
+// both parities of one Higgs routine (kind 1/2/3 = ahiggs1/2/3); with reduce
+// partial sums land in slots 6-7 for launch_finalize; renorm as launch_higgs,
+// in the first parity's launch
+static int higgs_sweep(lceq_lattice* L, int kind, int measflag, int reduce = 1,
+                       bool renorm = false) {
   int64_t per = (kind == 1 ? 4 : kind == 2 ? 7 : 1) * (int64_t)L->g.n;
   const double* fed0;
   int rc = take_uniforms(L, 2 * per, &fed0);
   if (rc) return rc;
   prof_begin(L, KC_HIGGS);
   for (int eo = 0; eo < 2; ++eo)
-    launch_higgs(L, kind, eo, measflag, fed0 ? fed0 + eo * per : nullptr, next_pass(L));
+    launch_higgs(L, kind, eo, measflag, fed0 ? fed0 + eo * per : nullptr, next_pass(L), reduce,
+                 renorm && eo == 0);
   prof_end(L, KC_HIGGS);
   return check_launch();
 }
@@ -1027,7 +1030,7 @@ struct SweepPass {
 
 static void launch_pass(lceq_lattice* L, const SweepPass& q, const SiteRange* r) {
   if (q.higgs)
-    launch_higgs(L, 1, q.eo, q.meas, nullptr, q.pass, r);
+    launch_higgs(L, 1, q.eo, q.meas, nullptr, q.pass, q.reduce, false, r);
   else
     launch_link(L, q.kp, q.eo, q.mu, q.meas, 1, nullptr, q.pass, q.reduce, r);
 }
@@ -1101,12 +1104,15 @@ extern "C" int lceq_sweep(lceq_lattice* L, int schedule, int nsweep, int n_or, d
       launch_finalize(L, measflag ? (n_or ? 2 : 1) : 0, measflag, 1, measflag, row,
                       it == nsweep - 1);
     } else {  // f/main.f:38-41
-      if ((rc = higgs_sweep(L, 2, measflag))) return rc;
-      if (measflag) launch_finalize(L, 0, 0, 2, 1, nullptr, false);
-      if ((rc = higgs_sweep(L, 3, measflag))) return rc;
+      // ahiggs2's averages are ahiggs3's a launch later, so it sums nothing.
+      // renorm is carried by the next sweep's first launch, which loads every
+      // link once (64^3: a renorm launch 12.2 us, carried 1.6)
+      const bool carry = L->rng_mode == LCEQ_RNG_PHILOX;
+      if ((rc = higgs_sweep(L, 2, 0, 0, carry && it > 0))) return rc;
+      if ((rc = higgs_sweep(L, 3, measflag, measflag))) return rc;
       if ((rc = link_sweep(L, 1, measflag, 0, measflag))) return rc;
       if (measflag) launch_finalize(L, 1, 1, 3, 1, row, false);
-      launch_renorm(L, L->U);
+      if (!carry || it == nsweep - 1) launch_renorm(L, L->U);
     }
   }
   if ((rc = check_launch())) return rc;

@@ -157,8 +157,11 @@ void launch_set_obs(lceq_lattice* L, int index, double value);
 void launch_export(lceq_lattice* L, const double* dev, size_t n);
 void launch_staples(lceq_lattice* L, int eo, int mu);
 void launch_force(lceq_lattice* L, int eo);
+// renorm (Philox ahiggs2 only): every link is normalised first, as by
+// launch_renorm
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
-                  uint64_t pass, const SiteRange* range = nullptr);
+                  uint64_t pass, int reduce, bool renorm = false,
+                  const SiteRange* range = nullptr);
 void launch_renorm(lceq_lattice* L, double* U);
 // per-block (unitarity deviation, non-finite count) of U and A into part[2 nb]
 void launch_check_fields(lceq_lattice* L, double* part);

@@ -428,7 +428,7 @@ void launch_force(lceq_lattice* L, int eo) {
 
 struct HiggsArgs {
   SiteOrder order;
-  int imode, measflag;
+  int imode, measflag, reduce;
   double beta_a, beta_2, beta_4;
   const double* delta;
   const double* fed;
@@ -439,8 +439,11 @@ struct HiggsArgs {
   int n, nb;  // as LinkArgs
 };
 
-template <int KIND, bool FED, int TBX, bool EARLY, bool RANGE>
+// MODE: the whole lattice, a range of it, or the whole lattice with renorm first
+enum { HIGGS_ALL, HIGGS_RANGE, HIGGS_RENORM };
+template <int KIND, bool FED, int TBX, bool EARLY, int MODE>
 __global__ __launch_bounds__(TBX) void k_higgs(HEAD_PARAMS, HiggsArgs a) {
+  constexpr bool RANGE = MODE == HIGGS_RANGE;
   const Head h = HEAD_OF;
   int blk = shape_block(RANGE ? (h.g.n + TBX - 1) / TBX : h.nb, h.flags & HEAD_XCD);
   unsigned P = (unsigned)(blk * TBX + threadIdx.x);
@@ -462,46 +465,52 @@ __global__ __launch_bounds__(TBX) void k_higgs(HEAD_PARAMS, HiggsArgs a) {
     p.measflag = a.measflag;
     unsigned s = h.flags & HEAD_STRIPS ? strip_site(p.g, a.order, P) : P;
     if (RANGE) s = range_site(h, s, a.n);
-    higgs_update_site<KIND, FED, EARLY>(p, s, red);
+    higgs_update_site<KIND, FED, EARLY, MODE == HIGGS_RENORM>(p, s, red);
   }
-  block_sum_store<4, TBX / 64>(red, a.part, a.pstride,
-                               RANGE ? range_block<TBX>(h, blk, a.nb) : blk);
+  if (a.reduce)
+    block_sum_store<4, TBX / 64>(red, a.part, a.pstride,
+                                 RANGE ? range_block<TBX>(h, blk, a.nb) : blk);
 }
 
-template <int KIND, bool FED, bool EARLY, bool RANGE, int TBX>
+template <int KIND, bool FED, bool EARLY, int MODE, int TBX>
 static void higgs_launch(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
-  int nb = RANGE ? (r->len + TBX - 1) / TBX : shape_blocks(L);
+  int nb = MODE == HIGGS_RANGE ? (r->len + TBX - 1) / TBX : shape_blocks(L);
   HeadArgs h = head_args(L, L->U, L->A, nb, eo, r);
-  hipLaunchKernelGGL((k_higgs<KIND, FED, TBX, EARLY, RANGE>), dim3(nb), dim3(TBX), 0, L->stream,
+  hipLaunchKernelGGL((k_higgs<KIND, FED, TBX, EARLY, MODE>), dim3(nb), dim3(TBX), 0, L->stream,
                      h.U, h.A, h.n, h.b, h.h, h.w, h.r, a);
 }
 
-template <int KIND, bool FED, bool EARLY, bool RANGE>
+template <int KIND, bool FED, bool EARLY, int MODE>
 static void higgs_dispatch_tb(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
   switch (L->tb) {
-    case 64: higgs_launch<KIND, FED, EARLY, RANGE, 64>(L, eo, a, r); break;
-    case 128: higgs_launch<KIND, FED, EARLY, RANGE, 128>(L, eo, a, r); break;
-    case 512: higgs_launch<KIND, FED, EARLY, RANGE, 512>(L, eo, a, r); break;
-    default: higgs_launch<KIND, FED, EARLY, RANGE, 256>(L, eo, a, r); break;
+    case 64: higgs_launch<KIND, FED, EARLY, MODE, 64>(L, eo, a, r); break;
+    case 128: higgs_launch<KIND, FED, EARLY, MODE, 128>(L, eo, a, r); break;
+    case 512: higgs_launch<KIND, FED, EARLY, MODE, 512>(L, eo, a, r); break;
+    default: higgs_launch<KIND, FED, EARLY, MODE, 256>(L, eo, a, r); break;
   }
 }
 
 // the early issue exists for ahiggs1 only (EARLY = KIND == 1 there), and so do
-// launches over a range
+// launches over a range; renorm first exists for ahiggs2
 template <int KIND, bool FED>
-static void higgs_dispatch(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r) {
+static void higgs_dispatch(lceq_lattice* L, int eo, const HiggsArgs& a, const SiteRange* r,
+                           bool renorm) {
   if constexpr (KIND == 1 && !FED) {
-    if (r) return higgs_dispatch_tb<KIND, FED, true, true>(L, eo, a, r);
+    if (r) return higgs_dispatch_tb<KIND, FED, true, HIGGS_RANGE>(L, eo, a, r);
+  }
+  if constexpr (KIND == 2 && !FED) {
+    if (renorm) return higgs_dispatch_tb<KIND, FED, false, HIGGS_RENORM>(L, eo, a, nullptr);
   }
   if (early_schedule(L))
-    higgs_dispatch_tb<KIND, FED, KIND == 1, false>(L, eo, a, nullptr);
+    higgs_dispatch_tb<KIND, FED, KIND == 1, HIGGS_ALL>(L, eo, a, nullptr);
   else
-    higgs_dispatch_tb<KIND, FED, false, false>(L, eo, a, nullptr);
+    higgs_dispatch_tb<KIND, FED, false, HIGGS_ALL>(L, eo, a, nullptr);
 }
 
 void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double* fed,
-                  uint64_t pass, const SiteRange* range) {
+                  uint64_t pass, int reduce, bool renorm, const SiteRange* range) {
   HiggsArgs a;
+  a.reduce = reduce;
   a.n = L->g.n;
   a.nb = shape_blocks(L);
   a.order = site_order(range ? range->len / L->g.h2 : L->g.lz, strip_rows(L));
@@ -519,11 +528,11 @@ void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double*
   prof_begin(L, KC_HIGGS);
   prof_count(L, KC_HIGGS);
   if (kind == 1) {
-    if (fed) higgs_dispatch<1, true>(L, eo, a, range); else higgs_dispatch<1, false>(L, eo, a, range);
+    if (fed) higgs_dispatch<1, true>(L, eo, a, range, renorm); else higgs_dispatch<1, false>(L, eo, a, range, renorm);
   } else if (kind == 2) {
-    if (fed) higgs_dispatch<2, true>(L, eo, a, range); else higgs_dispatch<2, false>(L, eo, a, range);
+    if (fed) higgs_dispatch<2, true>(L, eo, a, range, renorm); else higgs_dispatch<2, false>(L, eo, a, range, renorm);
   } else {
-    if (fed) higgs_dispatch<3, true>(L, eo, a, range); else higgs_dispatch<3, false>(L, eo, a, range);
+    if (fed) higgs_dispatch<3, true>(L, eo, a, range, renorm); else higgs_dispatch<3, false>(L, eo, a, range, renorm);
   }
   prof_end(L, KC_HIGGS);
 }

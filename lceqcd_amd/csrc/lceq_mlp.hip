@@ -630,7 +630,7 @@ extern "C" int lceq_mlp_collect(lceq_lattice* L, lceq_mlp* M, int nsteps, int st
     float* out = base + (size_t)eo * nrec * NREC;
     launch_record(L->stream, L->g, L->U, L->A, eo, stride, nrec, L->beta_a, L->beta_2, L->beta_4,
                   out, 0);
-    for (int h = 0; h < nsteps; ++h) launch_higgs(L, 1, eo, 0, nullptr, next_pass(L));
+    for (int h = 0; h < nsteps; ++h) launch_higgs(L, 1, eo, 0, nullptr, next_pass(L), 0);
     launch_record(L->stream, L->g, L->U, L->A, eo, stride, nrec, L->beta_a, L->beta_2, L->beta_4,
                   out, 1);
   }

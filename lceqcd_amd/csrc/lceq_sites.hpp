@@ -338,7 +338,7 @@ __device__ __forceinline__ vec3 hop_force(const double* __restrict__ U,
 // Per-lattice parameters of one Higgs parity launch
 struct HiggsSite {
   Geom g;
-  const double* U;
+  double* U;  // written with RENORM only
   double* A;
   int eo, imode;
   double beta_a, beta_2, beta_4;
@@ -354,7 +354,10 @@ struct HiggsSite {
 // EARLY (ahiggs1 only): the operands at the site itself go out ahead of the
 // neighbour index arithmetic, as in link_update_site (1.3% off the ahiggs1
 // launch at 64^3; ahiggs2 and ahiggs3 were slower with it).
-template <int KIND, bool FED, bool EARLY = true>
+// RENORM: renorm (f/renorm.f) first.  The links at the site and those that end
+// there are, over the sites of one parity, every link of the lattice once, so
+// the update normalises and stores what it has loaded anyway.
+template <int KIND, bool FED, bool EARLY = true, bool RENORM = false>
 __device__ __forceinline__ void higgs_update_site(const HiggsSite& p, unsigned s, double (&red)[4]) {
   const Geom& g = p.g;
   int eo = p.eo;
@@ -390,6 +393,16 @@ __device__ __forceinline__ void higgs_update_site(const HiggsSite& p, unsigned s
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (RENORM) {
+    Steps st = site_steps(g, site_coord(g, eo, (int)s));
+#pragma unroll
+    for (int mu = 0; mu < 3; ++mu) {
+      k.ux[mu] = normalized(k.ux[mu]);
+      k.uy[mu] = normalized(k.uy[mu]);
+      st_link(p.U, g, mu, eo, s, k.ux[mu]);
+      st_link(p.U, g, mu, eo ^ 1, (unsigned)((int)s + st.m[mu]), k.uy[mu]);
+    }
+  }
   vec3 F = force_sum(k);
   double ro = 0.0, rn = 0.0, boltz, racc;
   if (KIND == 1) {  // f/ahiggs1.f:51-92
