@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <climits>
 #include <string>
 #include <vector>
@@ -806,27 +807,19 @@ extern "C" int lceq_or_gauge_fixing(lceq_lattice* L, double* da1) {
   NEEDL(L);
   launch_gfix(L, 0, 0, 0, 0);
   launch_gfix(L, 1, 1, 0, 0);
-  launch_gfix_finalize(L, 0);
+  launch_gfix_finalize(L, 0, 0, da1 != nullptr);
   int rc = check_launch();
   if (rc) return rc;
   if (da1) {
-    double o[LCEQ_OBS_N];
-    if ((rc = read_obs(L, o))) return rc;
-    *da1 = o[OBS_DA];
+    if ((rc = finish_obs(L))) return rc;
+    *da1 = L->pin[OBS_DA];
   }
   return LCEQ_OK;
 }
 
 extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   NEEDL(L);
-  size_t np = (size_t)L->g.npad;
-  HIPCHK(hipMemcpyAsync(L->Uf, L->U, 24 * np * sizeof(double), hipMemcpyDeviceToDevice, L->stream));
-  HIPCHK(hipMemcpyAsync(L->Af, L->A, 6 * np * sizeof(double), hipMemcpyDeviceToDevice, L->stream));
-  double init[3] = {10000.0, 0.0, 0.0};  // da1 = 10000 (f/landau_gauge.f:28), iter, done
-  HIPCHK(hipMemcpyAsync(L->obs + OBS_DA, init, 2 * sizeof(double), hipMemcpyHostToDevice, L->stream));
-  double z2[2] = {0.0, 0.0};
-  HIPCHK(hipMemcpyAsync(L->obs + OBS_GF_DONE, z2, 2 * sizeof(double), hipMemcpyHostToDevice,
-                        L->stream));
+  launch_gfix_begin(L);
   // Batches of guarded iterations; after convergence (or the cap) the
   // remaining launches of a batch return at once.  Inside a batch the loop
   // condition for the iterations so far is tested by the next iteration's
@@ -836,21 +829,33 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   // of a 352 us iteration at 160^3), so there each iteration is followed by
   // the finalize instead: the same sum in the same order, the same stop.
   const bool test_launch = blocks_for(L->g.n) > 2048;
+  // The iterations left are estimated from the decay of da over the last
+  // batch, which is close to geometric once the fields are smooth; a batch takes
+  // at most 7/8 of them, so that few launches are left over at the end (a
+  // launch after convergence takes about 3 us, up to 256 iterations of them
+  // went unused).
   int batch = 8, done_iter = 0;
-  double o[LCEQ_OBS_N];
+  double last = 0.0;
+  const double* o = L->pin;
   for (;;) {
     for (int k = 0; k < batch; ++k) {
       launch_gfix(L, 0, 0, 0, 1, test_launch ? 0 : k > 0, done_iter);
       launch_gfix(L, 1, 1, 1, 1);
       ++done_iter;
-      if (test_launch) launch_gfix_finalize(L, 1, done_iter);
+      if (test_launch) launch_gfix_finalize(L, 1, done_iter, k == batch - 1);
     }
-    if (!test_launch) launch_gfix_finalize(L, 1, done_iter);
-    int rc = check_launch();
+    if (!test_launch) launch_gfix_finalize(L, 1, done_iter, true);
+    int rc = finish_obs(L);
     if (rc) return rc;
-    if ((rc = read_obs(L, o))) return rc;
     if (o[OBS_GF_DONE] != 0.0) break;
-    if (batch < 256) batch *= 2;
+    int next = std::min(256, 2 * batch);
+    if (last > o[OBS_DA] && L->limit_or > 0.0) {
+      double left = batch * log(o[OBS_DA] / L->limit_or) / log(last / o[OBS_DA]);
+      if (left < 2.0 * next) next = std::max(8, std::min(next, (int)(0.875 * left)));
+    }
+    next = (int)std::min<int64_t>(next, std::max<int64_t>(1, (int64_t)L->max_iter - done_iter));
+    last = o[OBS_DA];
+    batch = next;
   }
   if (da1) *da1 = o[OBS_DA];
   if (iter_or1) *iter_or1 = (int)o[OBS_ITER];

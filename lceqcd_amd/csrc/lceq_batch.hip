@@ -188,8 +188,7 @@ __global__ __launch_bounds__(1024) void k_finalize_batch(const Replica* __restri
 #pragma unroll
         for (int u = 0; u < 8; ++u) t += y[u];
       }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      t = wave_sum(t);
     }
     if (lane == 0) tot[q] = t;
   }

@@ -383,16 +383,45 @@ __device__ __forceinline__ void philox_pair(const Philox& key, uint32_t idx, uin
 // Every thread of the block receives the NQ totals.
 // Deterministic block sum over NW waves (fixed butterfly and combine order);
 // the result is left in every thread.
+// Sum of one value over a wave's 64 lanes, in every lane: partners 32, 16, 8,
+// 4, 2 and 1 lanes away in turn, the additions of a xor butterfly.  The partner's
+// value comes by lane swaps and row moves inside the vector unit (4 cycles)
+// instead of a shuffle through the LDS crossbar (over 100 cycles a step, two
+// words each).  A rotation by 8 within a row of 16 is the partner 8 away; by 4
+// it is the partner 4 away or the one 8 further, which holds the same sum.
+template <int CTRL>
+__device__ __forceinline__ double lane_move(double t) {
+  int2 w = __builtin_bit_cast(int2, t);
+  w.x = __builtin_amdgcn_mov_dpp(w.x, CTRL, 0xf, 0xf, true);
+  w.y = __builtin_amdgcn_mov_dpp(w.y, CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, w);
+}
+__device__ __forceinline__ double wave_sum(double t) {
+  constexpr int ROW_ROR_8 = 0x128, ROW_ROR_4 = 0x124, QUAD_XOR_2 = 0x4e, QUAD_XOR_1 = 0xb1;
+  {  // 32 away: the halves of two copies swapped give lane l both l and l ^ 32
+    uint2 w = __builtin_bit_cast(uint2, t);
+    auto lo = __builtin_amdgcn_permlane32_swap(w.x, w.x, false, false);
+    auto hi = __builtin_amdgcn_permlane32_swap(w.y, w.y, false, false);
+    t = __builtin_bit_cast(double, uint2{lo[0], hi[0]}) + __builtin_bit_cast(double, uint2{lo[1], hi[1]});
+  }
+  {  // 16 away, likewise between the rows of each half
+    uint2 w = __builtin_bit_cast(uint2, t);
+    auto lo = __builtin_amdgcn_permlane16_swap(w.x, w.x, false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap(w.y, w.y, false, false);
+    t = __builtin_bit_cast(double, uint2{lo[0], hi[0]}) + __builtin_bit_cast(double, uint2{lo[1], hi[1]});
+  }
+  t += lane_move<ROW_ROR_8>(t);
+  t += lane_move<ROW_ROR_4>(t);
+  t += lane_move<QUAD_XOR_2>(t);
+  t += lane_move<QUAD_XOR_1>(t);
+  return t;
+}
+
 template <int NQ, int NW = 4>
 __device__ __forceinline__ void block_sum(double (&v)[NQ]) {
   __shared__ double red[NW][NQ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    double t = v[q];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-    v[q] = t;
-  }
+  for (int q = 0; q < NQ; ++q) v[q] = wave_sum(v[q]);
   int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (lane == 0) {
 #pragma unroll
@@ -408,16 +437,23 @@ __device__ __forceinline__ void block_sum(double (&v)[NQ]) {
   }
   __syncthreads();
 }
+// the block's totals to out[q * stride + blk], one thread per quantity
 template <int NQ, int NW = 4>
 __device__ __forceinline__ void block_sum_store(double (&v)[NQ], double* __restrict__ out,
                                                 int stride, int blk) {
-  block_sum<NQ, NW>(v);
+  __shared__ double red[NW][NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) v[q] = wave_sum(v[q]);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) red[threadIdx.x >> 6][q] = v[q];
+  }
+  __syncthreads();
   if (threadIdx.x < NQ) {
     int q = threadIdx.x;
-    double t = v[0];
+    double t = red[0][q];
 #pragma unroll
-    for (int k = 1; k < NQ; ++k)
-      if (q == k) t = v[k];
+    for (int w = 1; w < NW; ++w) t += red[w][q];
     out[(size_t)q * stride + blk] = t;
   }
 }

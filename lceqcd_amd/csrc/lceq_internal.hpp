@@ -169,7 +169,9 @@ void launch_check_fields(lceq_lattice* L, double* part);
 // condition for the `iter` iterations already complete (see k_gfix).
 void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check = 0,
                  int iter = 0);
-void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter = 0);
+void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host);
+// u_f = u, a_f = a, and the loop's observables as before its first iteration
+void launch_gfix_begin(lceq_lattice* L);
 // blocks per z slice of the slice sums (the slices buffer holds 14 lz split)
 int corr_split(const Geom& g);
 // the slice sums and correlators of measurement meas (0 correlator, which

@@ -15,21 +15,6 @@ static constexpr int TB = 256;
 
 int blocks_for(int n) { return (n + TB - 1) / TB; }
 
-// deterministic sum of x[0..n) by one 256-thread block; result in all threads
-__device__ double block_sum_range(const double* __restrict__ x, int n) {
-  __shared__ double red[4];
-  double t = 0.0;
-  for (int i = threadIdx.x; i < n; i += TB) t += x[i];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
-  __syncthreads();
-  double r = ((red[0] + red[1]) + red[2]) + red[3];
-  __syncthreads();
-  return r;
-}
-
 // ================================================================ links
 
 // What a wave needs before it can issue its operand loads, as leading
@@ -301,8 +286,7 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs p) {
   }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t[h] += __shfl_xor(t[h], off, 64);
+    t[h] = wave_sum(t[h]);
     if (lane == 0 && w + 16 * h < NV) tot[w + 16 * h] = t[h];
   }
   if (threadIdx.x < LCEQ_OBS_N) ob[threadIdx.x] = ov;
@@ -618,7 +602,17 @@ struct GfArgs {
 // da1 = (sum of the per-block partials of the eo = 1 half) / N
 // (f/or_gauge_fixing1.f:156-157), summed in a fixed order that does not
 // depend on the caller; every thread of a 256-thread block must call it.
+// The order is that of a block: thread t adds partials t, t + 256, ...; the
+// waves' butterflies; the four waves in turn.  Up to 64 partials, one wave's,
+// every wave does that by itself, so that a launch that tests the loop condition
+// first has no block barriers ahead of its update (32^3: 0.4 us of an iteration;
+// with more partials the waves' repeated loads cost more than the barriers: 64^3
+// 18.9 us an iteration, 20.7 that way).
 __device__ __forceinline__ double gfix_da(const double* __restrict__ part, int nb, double n) {
+  if (nb <= 64) {
+    const int lane = threadIdx.x & 63;
+    return wave_sum(lane < nb ? part[lane] : 0.0) / n;
+  }
   double v[1] = {0.0};
   for (int i0 = threadIdx.x; i0 < nb; i0 += TB * 4) {
     double y[4];
@@ -704,12 +698,13 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
     double ra = fmin(1.0, fmax(-1.0, o.a.re));
     double th = acos(ra);
     if (th != 0.0) {
-      double tho = p.lambda * th;
+      double tho = p.lambda * th, sn, cs;
+      sincos(tho, &sn, &cs);
       // sin(th) for th = acos(ra) in (0, pi] is sqrt((1 - ra)(1 + ra)); the
       // factored form keeps full relative precision as th -> 0
-      double f = sin(tho) * rsqrt((1.0 - ra) * (1.0 + ra));
+      double f = sn * rsqrt((1.0 - ra) * (1.0 + ra));
       double t2 = f * o.a.im;
-      o.a = c_mk(cos(tho), -t2);
+      o.a = c_mk(cs, -t2);
       o.b = c_mk(-(f * o.b.re), -(f * o.b.im));
     }
     st_higgs(Af, g, eo, s, adj_rot<false>(o, af));  // g X(a_f) g^+, :243-252
@@ -730,17 +725,55 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
 
 // da1 after one or_gauge_fixing call (guarded = 0), or the convergence test
 // of a landau_gauge batch's last iteration (guarded = 1, `iter` iterations
-// complete): the loop ends when da1 <= limit_or or at the iteration cap.
+// complete): the loop ends when da1 <= limit_or or at the iteration cap.  With
+// `host` the loop's observables also go to pinned memory there.
 __global__ __launch_bounds__(256) void k_gfix_finalize(const double* __restrict__ part, int nb,
                                                        double n, int guarded, double iter,
                                                        double limit_or, double max_iter,
-                                                       double* __restrict__ obs) {
-  if (guarded && obs[OBS_GF_DONE] != 0.0) return;
-  double da = gfix_da(part, nb, n);
-  if (guarded)
-    gfix_stop(da, iter, limit_or, max_iter, obs, threadIdx.x == 0);
-  else if (threadIdx.x == 0)
-    obs[OBS_DA] = da;
+                                                       double* __restrict__ obs,
+                                                       double* __restrict__ host) {
+  if (!guarded || obs[OBS_GF_DONE] == 0.0) {
+    double da = gfix_da(part, nb, n);
+    if (guarded)
+      gfix_stop(da, iter, limit_or, max_iter, obs, threadIdx.x == 0);
+    else if (threadIdx.x == 0)
+      obs[OBS_DA] = da;
+  }
+  // thread 0 wrote what has changed, so it alone copies
+  if (host && threadIdx.x == 0) {
+    host[OBS_DA] = obs[OBS_DA];
+    host[OBS_ITER] = obs[OBS_ITER];
+    host[OBS_GF_DONE] = obs[OBS_GF_DONE];
+    host[OBS_GF_CAPPED] = obs[OBS_GF_CAPPED];
+  }
+}
+
+// Start of landau_gauge (f/landau_gauge.f:26-52): u -> u_f, a -> a_f, da1 =
+// 10000, no iterations, not converged; one launch for two copies and two
+// uploads (16-byte elements, the arrays are whole 64-site rows of them)
+__global__ __launch_bounds__(TB) void k_gfix_begin(const double2* __restrict__ U,
+                                                   const double2* __restrict__ A,
+                                                   double2* __restrict__ Uf,
+                                                   double2* __restrict__ Af, unsigned nu,
+                                                   unsigned na, double* __restrict__ obs) {
+  unsigned i = blockIdx.x * TB + threadIdx.x;
+  if (i < nu)
+    Uf[i] = U[i];
+  else if (i - nu < na)
+    Af[i - nu] = A[i - nu];
+  if (i == 0) {
+    obs[OBS_DA] = 10000.0;
+    obs[OBS_ITER] = 0.0;
+    obs[OBS_GF_DONE] = 0.0;
+    obs[OBS_GF_CAPPED] = 0.0;
+  }
+}
+
+void launch_gfix_begin(lceq_lattice* L) {
+  unsigned nu = 12 * (unsigned)L->g.npad, na = 3 * (unsigned)L->g.npad;
+  hipLaunchKernelGGL(k_gfix_begin, dim3((nu + na + TB - 1) / TB), dim3(TB), 0, L->stream,
+                     (const double2*)L->U, (const double2*)L->A, (double2*)L->Uf,
+                     (double2*)L->Af, nu, na, L->obs);
 }
 
 void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check,
@@ -767,10 +800,10 @@ void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarde
   prof_end(L, KC_GFIX);
 }
 
-void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter) {
+void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host) {
   hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream, L->partials,
                      blocks_for(L->g.n), (double)L->g.n, guarded, (double)iter, L->limit_or,
-                     (double)L->max_iter, L->obs);
+                     (double)L->max_iter, L->obs, to_host ? L->pin : nullptr);
 }
 
 // ========================================================== correlators
@@ -818,9 +851,7 @@ __global__ __launch_bounds__(256) void k_slices(Geom g, int split,
   }
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    double t = acc[q];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    double t = wave_sum(acc[q]);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][q] = t;
   }
   __syncthreads();
