@@ -587,7 +587,7 @@ void launch_check_fields(lceq_lattice* L, double* part) {
 // ========================================================= gauge fixing
 
 struct GfArgs {
-  int compute_da, renorm, guarded;
+  int guarded;
   double lambda, alpha;
   double* obs;  // OBS_GF_DONE read when guarded; the convergence test writes
   double* part;
@@ -649,6 +649,9 @@ __device__ __forceinline__ bool gfix_stop(double da, double iter, double limit_o
 // first repeats the convergence test of the previous iteration (the same
 // sum in the same order, so all blocks agree) and the launch returns when
 // the loop has ended; the operand loads are issued before the test.
+// DA and RENORM are template arguments: without a branch around each pair, the
+// six normalisations' chains of dependent operations run side by side.
+template <bool DA, bool RENORM>
 __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   const Head h = HEAD_OF;
   const Geom& g = h.g;
@@ -688,7 +691,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
     s2.a = c_add(s2.a, c_scale(p.alpha, uy[2].a));
     s2.b = c_add(s2.b, c_scale(p.alpha, uy[2].b));
     su2 w{c_add(s1.a, c_conj(s2.a)), c_sub(s1.b, s2.b)};  // :145-146
-    if (p.compute_da) {                                    // :153-158
+    if (DA) {                                              // :153-158
       double d = c_sub(s1.a, s2.a).im;
       red[0] = d * d + (w.b.re * w.b.re + w.b.im * w.b.im);
     }
@@ -712,7 +715,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
     for (int mu = 0; mu < 3; ++mu) {  // :256-324
       su2 nx = m_nn(o, ux[mu]);
       su2 ny = m_nd(uy[mu], o);
-      if (p.renorm) {
+      if (RENORM) {
         nx = normalized(nx);
         ny = normalized(ny);
       }
@@ -720,7 +723,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
       st_link(Uf, g, mu, oe, sy[mu], ny);
     }
   }
-  if (p.compute_da) block_sum_store<1>(red, p.part, p.pstride, blk);
+  if (DA) block_sum_store<1>(red, p.part, p.pstride, blk);
 }
 
 // da1 after one or_gauge_fixing call (guarded = 0), or the convergence test
@@ -779,8 +782,6 @@ void launch_gfix_begin(lceq_lattice* L) {
 void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check,
                  int iter) {
   GfArgs a;
-  a.compute_da = compute_da;
-  a.renorm = renorm;
   a.guarded = guarded;
   a.lambda = L->lambda;
   a.alpha = L->alpha;
@@ -795,8 +796,16 @@ void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarde
   prof_count(L, KC_GFIX);
   int nb = blocks_for(L->g.n);
   HeadArgs h = head_args(L, L->Uf, L->Af, nb, eo);
-  hipLaunchKernelGGL(k_gfix, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A,
-                     h.n, h.b, h.h, h.w, h.r, a);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A, h.n, h.b, h.h, h.w, h.r,
+                       a);
+  };
+  if (renorm)
+    launch(k_gfix<true, true>);
+  else if (compute_da)
+    launch(k_gfix<true, false>);
+  else
+    launch(k_gfix<false, false>);
   prof_end(L, KC_GFIX);
 }
 
