@@ -49,82 +49,106 @@ struct Replica {
   double* obs;      // [LCEQ_OBS_N]
 };
 
+// One update block's replica, as far as its operand addresses need it: a block
+// reads its own 64 bytes in one round trip.  (A table of replica numbers and the
+// replica behind it were two, ahead of the operand loads of every block.)
+struct alignas(64) BlockHead {
+  double *U, *A;
+  int n, npad, h1, h2;
+  float rh1, rh2;
+  int wy, wz;
+  int lblk, rep;  // block within the replica, replica
+};
+
 struct BatchCommon {
+  const BlockHead* heads;
   const Replica* reps;
-  const int* blk2rep;
-  int total_nb;           // blocks of this launch (one replica group's)
-  int blk_base;           // global index of the launch's first block
   // device counters: ctr[0] sweeps (history row), ctr[1] the Philox pass
   // of the first launch of the current sweep; launch j of a sweep uses pass
   // ctr[1] + j, as the j-th next_pass() of a single lattice's sweep
   const uint64_t* ctr;
-  int xcd;                // XCD-aware block order (else launch order)
+  double* obs;  // [replica][LCEQ_OBS_N]
+  int total_nb, blk_base;  // blocks of this launch (one replica group's), first block
+  int xcd;                 // XCD-aware block order (else launch order)
 };
 
-__device__ __forceinline__ int batch_block(const BatchCommon& c, int& r, const Replica*& R) {
-  int gblk = c.blk_base + (c.xcd ? xcd_block(c.total_nb) : (int)blockIdx.x);
-  r = c.blk2rep[gblk];
-  R = c.reps + r;
-  return gblk - R->blk0;
+// The update kernels' arguments: what a wave needs before its head load is in
+// scalar registers at its start (the first 14 dwords, see build.py)
+enum { BATCH_EO = 1, BATCH_XCD = 2, BATCH_MEAS = 4, BATCH_REDUCE = 8 };
+#define BATCH_PARAMS                                                                          \
+  const BlockHead *heads, uint64_t blocks, uint64_t flags_pass, const Replica *reps,          \
+      const uint64_t *ctr, double *obs
+
+struct BatchBlock {
+  Geom g;  // without the extents
+  double *U, *A;
+  const Replica* R;
+  int lblk, rep, flags, pass;
+};
+__device__ __forceinline__ BatchBlock batch_block(const BlockHead* heads, uint64_t blocks,
+                                                  uint64_t flags_pass, const Replica* reps) {
+  int nb = (int)(uint32_t)blocks, flags = (int)(uint32_t)flags_pass;
+  int blk = xcd_block(nb);
+  const BlockHead h = heads[(int)(blocks >> 32) + (flags & BATCH_XCD ? blk : (int)blockIdx.x)];
+  return BatchBlock{Geom{0, 0, 0, h.h1, h.h2, h.n, h.npad, h.rh1, h.rh2, h.wy, h.wz}, h.U, h.A,
+                    reps + h.rep, h.lblk, h.rep, flags, (int)(flags_pass >> 32)};
 }
 
-// One (eo, mu) link class of every replica, TBX sites per block
-template <bool KP, int TBX>
-__global__ __launch_bounds__(TBX) void k_link_batch(BatchCommon c, int eo, int mu, int pass_in_sweep,
-                                                    int measflag, int reduce) {
-  int r;
-  const Replica* R;
-  int lblk = batch_block(c, r, R);
-  unsigned s = (unsigned)(lblk * TBX + threadIdx.x);
+// One (eo, MU) link class of every replica, TBX sites per block
+template <bool KP, int TBX, int MU>
+__global__ __launch_bounds__(TBX) void k_link_batch(BATCH_PARAMS) {
+  const BatchBlock b = batch_block(heads, blocks, flags_pass, reps);
+  const Replica* R = b.R;
+  unsigned s = (unsigned)(b.lblk * TBX + threadIdx.x);
+  const int eo = b.flags & BATCH_EO;
   double red[3] = {0.0, 0.0, 0.0};
-  if (s < (unsigned)R->g.n) {
+  if (s < (unsigned)b.g.n) {
     LinkSite p;
-    p.g = R->g;
-    p.U = R->U;
-    p.A = R->A;
+    p.g = b.g;
+    p.U = b.U;
+    p.A = b.A;
     p.eo = eo;
-    p.mu = mu;
+    p.mu = MU;
     p.beta = R->beta;
     p.beta_a = R->beta_a;
     p.fed = nullptr;
     p.key = R->key;
-    p.pass = c.ctr[1] + (uint64_t)pass_in_sweep;
-    p.measflag = measflag;
+    p.pass = ctr[1] + (uint64_t)b.pass;
+    p.measflag = b.flags & BATCH_MEAS ? 1 : 0;
     p.renorm = 1;
     link_update_site<KP, false>(p, s, red);
   }
-  if (reduce)
-    block_sum_store<3, TBX / 64>(red, R->part + (size_t)(eo * 3 + mu) * LCEQ_NQ * R->pstride,
-                                 R->pstride, lblk);
+  if (b.flags & BATCH_REDUCE)
+    block_sum_store<3, TBX / 64>(red, R->part + (size_t)(eo * 3 + MU) * LCEQ_NQ * R->pstride,
+                                 R->pstride, b.lblk);
 }
 
 template <int TBX>
-__global__ __launch_bounds__(TBX) void k_higgs_batch(BatchCommon c, int eo, int pass_in_sweep,
-                                                     int measflag) {
-  int r;
-  const Replica* R;
-  int lblk = batch_block(c, r, R);
-  unsigned s = (unsigned)(lblk * TBX + threadIdx.x);
+__global__ __launch_bounds__(TBX) void k_higgs_batch(BATCH_PARAMS) {
+  const BatchBlock b = batch_block(heads, blocks, flags_pass, reps);
+  const Replica* R = b.R;
+  unsigned s = (unsigned)(b.lblk * TBX + threadIdx.x);
+  const int eo = b.flags & BATCH_EO;
   double red[4] = {0.0, 0.0, 0.0, 0.0};
-  if (s < (unsigned)R->g.n) {
+  if (s < (unsigned)b.g.n) {
     HiggsSite p;
-    p.g = R->g;
-    p.U = R->U;
-    p.A = R->A;
+    p.g = b.g;
+    p.U = b.U;
+    p.A = b.A;
     p.eo = eo;
     p.imode = 0;
     p.beta_a = R->beta_a;
     p.beta_2 = R->beta_2;
     p.beta_4 = R->beta_4;
-    p.delta = R->obs + OBS_DELTA;
+    p.delta = obs + (size_t)b.rep * LCEQ_OBS_N + OBS_DELTA;
     p.fed = nullptr;
     p.key = R->key;
-    p.pass = c.ctr[1] + (uint64_t)pass_in_sweep;
-    p.measflag = measflag;
+    p.pass = ctr[1] + (uint64_t)b.pass;
+    p.measflag = b.flags & BATCH_MEAS ? 1 : 0;
     higgs_update_site<1, false>(p, s, red);
   }
   block_sum_store<4, TBX / 64>(red, R->part + (size_t)(6 + eo) * LCEQ_NQ * R->pstride, R->pstride,
-                               lblk);
+                               b.lblk);
 }
 
 // One Higgs parity of every replica with the learned proposal: the per-site
@@ -275,7 +299,7 @@ struct lceq_batch {
   std::vector<Replica> reps;  // host copy of the device table
   std::vector<int64_t> field_off;
   Replica* d_reps;
-  int* d_blk2rep;
+  BlockHead* d_heads;
   int total_nb;
   int64_t total_sites;
   double *pool, *parts, *obs, *hist;
@@ -353,16 +377,19 @@ static void batch_groups(lceq_batch* B) {
 // of every update launch.  Partial-sum slots are sized for the smallest
 // shape at creation (pstride), so a shape change needs no reallocation.
 static int batch_layout(lceq_batch* B, int tb, int xcd) {
-  std::vector<int> blk2rep;
+  std::vector<BlockHead> heads;
   int nb_total = 0;
   for (int r = 0; r < B->nrep; ++r) {
     Replica& R = B->reps[r];
-    R.nb = (R.g.n + tb - 1) / tb;
+    const Geom& g = R.g;
+    R.nb = (g.n + tb - 1) / tb;
     R.blk0 = nb_total;
-    for (int k = 0; k < R.nb; ++k) blk2rep.push_back(r);
+    for (int k = 0; k < R.nb; ++k)
+      heads.push_back(
+          BlockHead{R.U, R.A, g.n, g.npad, g.h1, g.h2, g.rh1, g.rh2, g.wy, g.wz, k, r});
     nb_total += R.nb;
   }
-  BHIP(hipMemcpyAsync(B->d_blk2rep, blk2rep.data(), blk2rep.size() * sizeof(int),
+  BHIP(hipMemcpyAsync(B->d_heads, heads.data(), heads.size() * sizeof(BlockHead),
                       hipMemcpyHostToDevice, B->stream));
   B->total_nb = nb_total;
   B->tb = tb;
@@ -385,7 +412,7 @@ extern "C" int lceq_batch_create(int nrep, const int* dims, lceq_batch** out) {
   B->field_off.resize(nrep);
   int64_t pool = 0, parts = 0;
   int nb_total = 0;
-  std::vector<int> blk2rep, mblk2rep;
+  std::vector<int> mblk2rep;
   for (int r = 0; r < nrep; ++r) {
     int lx = dims[3 * r], ly = dims[3 * r + 1], lz = dims[3 * r + 2];
     if (const char* why = geom_reject(lx, ly, lz)) {
@@ -407,7 +434,6 @@ extern "C" int lceq_batch_create(int nrep, const int* dims, lceq_batch** out) {
     B->field_off[r] = pool;
     pool += 30 * (int64_t)R.g.npad;  // 24 link + 6 Higgs components
     parts += (int64_t)LCEQ_NSLOT * LCEQ_NQ * R.pstride;
-    for (int k = 0; k < R.nb; ++k) blk2rep.push_back(r);
     nb_total += R.nb;
     R.mnb = (R.g.n + mlp::MLP_TB - 1) / mlp::MLP_TB;
     R.mblk0 = (int)mblk2rep.size();
@@ -434,7 +460,7 @@ extern "C" int lceq_batch_create(int nrep, const int* dims, lceq_batch** out) {
   alloc((void**)&B->obs, (size_t)nrep * LCEQ_OBS_N * sizeof(double));
   alloc((void**)&B->hist, (size_t)B->hist_cap * nrep * LCEQ_OBS_N * sizeof(double));
   alloc((void**)&B->d_reps, nrep * sizeof(Replica));
-  alloc((void**)&B->d_blk2rep, blk2rep.size() * sizeof(int));
+  alloc((void**)&B->d_heads, (size_t)nb_total * sizeof(BlockHead));  // of the smallest shape
   alloc((void**)&B->d_mblk2rep, mblk2rep.size() * sizeof(int));
   alloc((void**)&B->d_ctr, 2 * sizeof(uint64_t));
   if (rc) {
@@ -472,7 +498,7 @@ extern "C" int lceq_batch_destroy(lceq_batch* B) {
   if (!B) return LCEQ_OK;
   if (B->stream) (void)hipStreamSynchronize(B->stream);
   if (B->graph) (void)hipGraphExecDestroy(B->graph);
-  void* bufs[] = {B->pool, B->parts, B->obs, B->hist, B->d_reps, B->d_blk2rep, B->d_mblk2rep,
+  void* bufs[] = {B->pool, B->parts, B->obs, B->hist, B->d_reps, B->d_heads, B->d_mblk2rep,
                   B->d_ctr};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
@@ -550,22 +576,42 @@ extern "C" int lceq_batch_get_higgs(lceq_batch* B, int r, double* a, int64_t ld)
   return batch_field(B, r, a, nullptr, ld, 0);
 }
 
+// the launch arguments of BATCH_PARAMS for the replicas of c
+#define BATCH_ARGS(c, flags, pass)                                                            \
+  (c).heads, halves((c).total_nb, (c).blk_base),                                              \
+      halves((flags) | ((c).xcd ? BATCH_XCD : 0), pass), (c).reps, (c).ctr, (c).obs
+static uint64_t halves(int a, int b) {
+  return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
+}
+
+template <bool KP, int TBX>
+static void enqueue_link(lceq_batch* B, const BatchCommon& c, int flags, int mu, int pass) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(c.total_nb), dim3(TBX), 0, B->stream,
+                       BATCH_ARGS(c, flags, pass));
+  };
+  // the direction at compile time, as for a single lattice
+  if (mu == 0)
+    launch(k_link_batch<KP, TBX, 0>);
+  else if (mu == 1)
+    launch(k_link_batch<KP, TBX, 1>);
+  else
+    launch(k_link_batch<KP, TBX, 2>);
+}
+
 template <int TBX>
 static void enqueue_links(lceq_batch* B, const BatchCommon& c, int n_or, int measflag) {
-  dim3 grid(c.total_nb), blk(TBX);
   int pass = 0;
   for (int k = -1; k < n_or; ++k) {
     int kp = k < 0;
     int m = measflag && (kp ? n_or == 0 : k == n_or - 1);
     for (int eo = 0; eo < 2; ++eo)
-      for (int mu = 0; mu < 3; ++mu) {
+      for (int mu = 0; mu < 3; ++mu, ++pass) {
+        int flags = (eo ? BATCH_EO : 0) | (m ? BATCH_MEAS | BATCH_REDUCE : 0);
         if (kp)
-          hipLaunchKernelGGL((k_link_batch<true, TBX>), grid, blk, 0, B->stream, c, eo, mu, pass,
-                             m, m);
+          enqueue_link<true, TBX>(B, c, flags, mu, pass);
         else
-          hipLaunchKernelGGL((k_link_batch<false, TBX>), grid, blk, 0, B->stream, c, eo, mu, pass,
-                             m, m);
-        ++pass;
+          enqueue_link<false, TBX>(B, c, flags, mu, pass);
       }
   }
 }
@@ -574,17 +620,18 @@ static void enqueue_links(lceq_batch* B, const BatchCommon& c, int n_or, int mea
 template <int TBX>
 static void enqueue_higgs(lceq_batch* B, const BatchCommon& c, int eo, int pass_in_sweep,
                           int measflag) {
-  hipLaunchKernelGGL((k_higgs_batch<TBX>), dim3(c.total_nb), dim3(TBX), 0, B->stream, c, eo,
-                     pass_in_sweep, measflag);
+  int flags = (eo ? BATCH_EO : 0) | (measflag == 1 ? BATCH_MEAS : 0);
+  hipLaunchKernelGGL((k_higgs_batch<TBX>), dim3(c.total_nb), dim3(TBX), 0, B->stream,
+                     BATCH_ARGS(c, flags, pass_in_sweep));
 }
 
 // launches over every replica
 static BatchCommon batch_common(const lceq_batch* B) {
-  return BatchCommon{B->d_reps, B->d_blk2rep, B->total_nb, 0, B->d_ctr, B->xcd};
+  return BatchCommon{B->d_heads, B->d_reps, B->d_ctr, B->obs, B->total_nb, 0, B->xcd};
 }
 // launches over one replica group
 static BatchCommon group_common(const lceq_batch* B, const ReplicaGroup& G) {
-  return BatchCommon{B->d_reps, B->d_blk2rep, G.nb, G.blk0, B->d_ctr, B->xcd};
+  return BatchCommon{B->d_heads, B->d_reps, B->d_ctr, B->obs, G.nb, G.blk0, B->xcd};
 }
 
 // Enqueue one sweep of every replica: for each replica group in turn, 1 KP
