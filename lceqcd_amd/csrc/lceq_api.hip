@@ -88,6 +88,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   alloc(&L->Af, 6 * np);
   alloc(&L->Vst, 24 * np);
   alloc(&L->F, 3 * np);
+  alloc(&L->gf_part, 2 * (size_t)gfix_tiles(g));
   alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
 
   alloc(&L->obs, LCEQ_OBS_N);
@@ -125,7 +126,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
 extern "C" int lceq_destroy(lceq_lattice* L) {
   if (!L) return LCEQ_OK;
   if (L->stream) (void)hipStreamSynchronize(L->stream);
-  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->partials, L->obs,
+  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->Ug, L->gf_part, L->partials, L->obs,
                     L->slices, L->corr, L->hist, L->scratch, L->fed};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
@@ -805,9 +806,9 @@ extern "C" int lceq_u_f_renorm(lceq_lattice* L) {
 
 extern "C" int lceq_or_gauge_fixing(lceq_lattice* L, double* da1) {
   NEEDL(L);
-  launch_gfix(L, 0, 0, 0, 0);
-  launch_gfix(L, 1, 1, 0, 0);
-  launch_gfix_finalize(L, 0, 0, da1 != nullptr);
+  launch_gfix(L, 0, 0, 0);
+  launch_gfix(L, 1, 0, 0);
+  launch_gfix_finalize(L, 0, 0, da1 != nullptr, false);
   int rc = check_launch();
   if (rc) return rc;
   if (da1) {
@@ -819,7 +820,14 @@ extern "C" int lceq_or_gauge_fixing(lceq_lattice* L, double* da1) {
 
 extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   NEEDL(L);
-  launch_gfix_begin(L);
+  // one launch per iteration between two link arrays; without memory for the
+  // second, two launches in place
+  if (!L->Ug && hipMalloc((void**)&L->Ug, 24 * (size_t)L->g.npad * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
+    L->Ug = nullptr;
+  }
+  const bool one = L->Ug != nullptr;
+  launch_gfix_begin(L, !one);
   // Batches of guarded iterations; after convergence (or the cap) the
   // remaining launches of a batch return at once.  Inside a batch the loop
   // condition for the iterations so far is tested by the next iteration's
@@ -828,7 +836,7 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   // partials costs more than a one-block test launch per iteration (26 us
   // of a 352 us iteration at 160^3), so there each iteration is followed by
   // the finalize instead: the same sum in the same order, the same stop.
-  const bool test_launch = blocks_for(L->g.n) > 2048;
+  const bool test_launch = gfix_tiles(L->g) > 2048;
   // The iterations left are estimated from the decay of da over the last
   // batch, which is close to geometric once the fields are smooth; a batch takes
   // at most 7/8 of them, so that few launches are left over at the end (a
@@ -839,12 +847,17 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   const double* o = L->pin;
   for (;;) {
     for (int k = 0; k < batch; ++k) {
-      launch_gfix(L, 0, 0, 0, 1, test_launch ? 0 : k > 0, done_iter);
-      launch_gfix(L, 1, 1, 1, 1);
+      const int check = test_launch ? 0 : k > 0;
+      if (one) {
+        launch_gfix_iter(L, done_iter + 1, check);
+      } else {
+        launch_gfix(L, 0, 0, 1, check, done_iter);
+        launch_gfix(L, 1, 1, 1);
+      }
       ++done_iter;
-      if (test_launch) launch_gfix_finalize(L, 1, done_iter, k == batch - 1);
+      if (test_launch) launch_gfix_finalize(L, 1, done_iter, k == batch - 1, one);
     }
-    if (!test_launch) launch_gfix_finalize(L, 1, done_iter, true);
+    if (!test_launch) launch_gfix_finalize(L, 1, done_iter, true, one);
     int rc = finish_obs(L);
     if (rc) return rc;
     if (o[OBS_GF_DONE] != 0.0) break;
@@ -857,6 +870,8 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
     last = o[OBS_DA];
     batch = next;
   }
+  // the last iteration wrote u_f or, for an even one, the second array
+  if (one && (int)o[OBS_ITER] % 2 == 0) std::swap(L->Uf, L->Ug);
   if (da1) *da1 = o[OBS_DA];
   if (iter_or1) *iter_or1 = (int)o[OBS_ITER];
   if (o[OBS_GF_CAPPED] != 0.0)

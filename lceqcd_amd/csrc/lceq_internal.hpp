@@ -40,6 +40,8 @@ struct lceq_lattice {
   hipStream_t stream;
   // device fields
   double *U, *A, *Uf, *Af, *Vst, *F;
+  double* Ug;        // second link array of landau_gauge, from its first call on
+  double* gf_part;   // da partials of two iterations [2][gfix_tiles]
   double *partials;  // [LCEQ_NSLOT][LCEQ_NQ][pstride]
   int pstride;       // >= number of 64-site blocks (the smallest launch shape)
   double *obs;       // [LCEQ_OBS_N]
@@ -165,13 +167,19 @@ void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double*
 void launch_renorm(lceq_lattice* L, double* U);
 // per-block (unitarity deviation, non-finite count) of U and A into part[2 nb]
 void launch_check_fields(lceq_lattice* L, double* part);
-// One half-iteration of gauge fixing; check = 1 first tests the loop
-// condition for the `iter` iterations already complete (see k_gfix).
-void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check = 0,
-                 int iter = 0);
-void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host);
-// u_f = u, a_f = a, and the loop's observables as before its first iteration
-void launch_gfix_begin(lceq_lattice* L);
+// One half-iteration of gauge fixing (eo = 1 forms da); check = 1 first tests
+// the loop condition for the `iter` iterations already complete (see k_gfix).
+void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check = 0, int iter = 0);
+// Iteration `iter` (from 1) in one launch, from u or the array the iteration
+// before wrote into the other one of u_f and L->Ug
+void launch_gfix_iter(lceq_lattice* L, int iter, int check);
+// one_launch: the iterations were launch_gfix_iter's
+void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch);
+// a_f = a, with `links` u_f = u, and the loop's observables as before its first
+// iteration
+void launch_gfix_begin(lceq_lattice* L, bool links);
+// da partials of an iteration
+int gfix_tiles(const Geom& g);
 // blocks per z slice of the slice sums (the slices buffer holds 14 lz split)
 int corr_split(const Geom& g);
 // the slice sums and correlators of measurement meas (0 correlator, which

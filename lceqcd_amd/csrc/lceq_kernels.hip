@@ -586,22 +586,51 @@ void launch_check_fields(lceq_lattice* L, double* part) {
 
 // ========================================================= gauge fixing
 
+// Tiles of GT_X x GT_Y x GT_Z sites, cut off at the lattice's far faces: the
+// odd half step's blocks, 256 odd sites each
+constexpr int GT_X = 16, GT_Y = 8, GT_Z = 4;
+static int gf_tiles_along(int l, int t) { return (l + t - 1) / t; }
+int gfix_tiles(const Geom& g) {
+  return gf_tiles_along(g.lx, GT_X) * gf_tiles_along(g.ly, GT_Y) * gf_tiles_along(g.lz, GT_Z);
+}
+
+struct TileOrigin {
+  int x, y, z;
+};
+__device__ __forceinline__ TileOrigin tile_origin(int tile, int ntx, int nty) {
+  int nxy = ntx * nty;
+  int tz = div_small(tile, nxy, __builtin_amdgcn_rcpf((float)nxy));
+  int r = tile - tz * nxy;
+  int ty = div_small(r, ntx, __builtin_amdgcn_rcpf((float)ntx));
+  return TileOrigin{GT_X * (r - ty * ntx), GT_Y * ty, GT_Z * tz};
+}
+// odd site i (0..255) of a tile, in tile coordinates
+struct TileSite {
+  int x, y, z;
+};
+__device__ __forceinline__ TileSite tile_odd_site(int i) {
+  int y = (i >> 3) & 7, z = i >> 6;
+  return TileSite{2 * (i & 7) + ((y + z + 1) & 1), y, z};
+}
+
 struct GfArgs {
   int guarded;
+  int lx, ly, lz, ntx, nty;  // extents and tiles (k_gfix<DA>)
   double lambda, alpha;
   double* obs;  // OBS_GF_DONE read when guarded; the convergence test writes
-  double* part;
-  int pstride;
+  double* part;            // da partials this launch writes, one per tile
+  const double* part_old;  // those of the iteration before (check)
+  int ntiles, n;
   // convergence test of the previous iteration at the start of this launch
   // (landau_gauge iterations after the first of a batch): `iter` iterations
-  // are complete, their last da is in `part`
+  // are complete, their last da is in `part_old`
   int check;
   double iter, limit_or, max_iter;
 };
 
 // da1 = (sum of the per-block partials of the eo = 1 half) / N
 // (f/or_gauge_fixing1.f:156-157), summed in a fixed order that does not
-// depend on the caller; every thread of a 256-thread block must call it.
+// depend on the caller; every thread of a block of 256 or more must call it.
 // The order is that of a block: thread t adds partials t, t + 256, ...; the
 // waves' butterflies; the four waves in turn.  Up to 64 partials, one wave's,
 // every wave does that by itself, so that a launch that tests the loop condition
@@ -613,16 +642,21 @@ __device__ __forceinline__ double gfix_da(const double* __restrict__ part, int n
     const int lane = threadIdx.x & 63;
     return wave_sum(lane < nb ? part[lane] : 0.0) / n;
   }
-  double v[1] = {0.0};
-  for (int i0 = threadIdx.x; i0 < nb; i0 += TB * 4) {
-    double y[4];
+  __shared__ double red[4];
+  double v = 0.0;
+  if (threadIdx.x < TB) {
+    for (int i0 = threadIdx.x; i0 < nb; i0 += TB * 4) {
+      double y[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) y[u] = i0 + TB * u < nb ? part[i0 + TB * u] : 0.0;
+      for (int u = 0; u < 4; ++u) y[u] = i0 + TB * u < nb ? part[i0 + TB * u] : 0.0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[0] += y[u];
+      for (int u = 0; u < 4; ++u) v += y[u];
+    }
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   }
-  block_sum<1>(v);
-  return v[0] / n;
+  __syncthreads();
+  return (((red[0] + red[1]) + red[2]) + red[3]) / n;
 }
 
 // The loop condition of f/landau_gauge.f:54-59 after `iter` iterations
@@ -641,16 +675,52 @@ __device__ __forceinline__ bool gfix_stop(double da, double iter, double limit_o
   return stop;
 }
 
+// The weighted sum of three links, f/or_gauge_fixing1.f:97-107, :116-142
+__device__ __forceinline__ su2 gfix_sum(double alpha, const su2 (&u)[3]) {
+  su2 s{c_add(u[0].a, u[1].a), c_add(u[0].b, u[1].b)};
+  s.a = c_add(s.a, c_scale(alpha, u[2].a));
+  s.b = c_add(s.b, c_scale(alpha, u[2].b));
+  return s;
+}
+__device__ __forceinline__ su2 gfix_w(const su2& s1, const su2& s2) {  // :145-146
+  return su2{c_add(s1.a, c_conj(s2.a)), c_sub(s1.b, s2.b)};
+}
+__device__ __forceinline__ double gfix_site_da(const su2& s1, const su2& s2, const su2& w) {
+  double d = c_sub(s1.a, s2.a).im;  // :153-158
+  return d * d + (w.b.re * w.b.re + w.b.im * w.b.im);
+}
+// the overrelaxed gauge transformation of w = s1 + s2^+, :169-242
+__device__ __forceinline__ su2 gfix_rotation(const su2& w, double lambda) {
+  double k = (w.a.re * w.a.re + w.a.im * w.a.im) + (w.b.re * w.b.re + w.b.im * w.b.im);
+  double rk = rsqrt(k);  // w / sqrt(k), :169-183
+  su2 o{c_scale(rk, w.a), c_scale(rk, w.b)};
+  double ra = fmin(1.0, fmax(-1.0, o.a.re));
+  double th = acos(ra);
+  if (th != 0.0) {
+    double tho = lambda * th, sn, cs;
+    sincos(tho, &sn, &cs);
+    // sin(th) for th = acos(ra) in (0, pi] is sqrt((1 - ra)(1 + ra)); the
+    // factored form keeps full relative precision as th -> 0
+    double f = sn * rsqrt((1.0 - ra) * (1.0 + ra));
+    double t2 = f * o.a.im;
+    o.a = c_mk(cs, -t2);
+    o.b = c_mk(-(f * o.b.re), -(f * o.b.im));
+  }
+  return o;
+}
+
 // One parity half of f/or_gauge_fixing1.f:54-328.  Thread x reads and
 // writes only U_mu(x) and U_mu(x-mu) for mu = 1..3 and a_f(x), so the half
-// step has no cross-thread hazards.  With renorm=1 (eo = 1 of a
+// step has no cross-thread hazards.  With RENORM (eo = 1 of a
 // landau_gauge iteration) every link of the lattice is written exactly once
 // and f/u_f_renorm.f is applied on that write.  With check=1 every block
 // first repeats the convergence test of the previous iteration (the same
 // sum in the same order, so all blocks agree) and the launch returns when
 // the loop has ended; the operand loads are issued before the test.
-// DA and RENORM are template arguments: without a branch around each pair, the
-// six normalisations' chains of dependent operations run side by side.
+// DA (eo = 1): da's partial sums, one per tile, the blocks then being tiles; the
+// other half's blocks are index ranges.  DA and RENORM are template arguments:
+// without a branch around each pair, the six normalisations' chains of
+// dependent operations run side by side.
 template <bool DA, bool RENORM>
 __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   const Head h = HEAD_OF;
@@ -658,8 +728,15 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   double *Uf = h.U, *Af = h.A;
   int blk = xcd_block(h.nb);
   int s = blk * TB + threadIdx.x;
+  int eo = DA ? 1 : h.flags & HEAD_EO, oe = eo ^ 1;
   bool act = s < g.n;
-  int eo = h.flags & HEAD_EO, oe = eo ^ 1;
+  if (DA) {
+    TileOrigin o = tile_origin(blk, p.ntx, p.nty);
+    TileSite t = tile_odd_site(threadIdx.x);
+    int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
+    act = x < p.lx && y < p.ly && z < p.lz;
+    s = (x >> 1) + g.h1 * y + g.h2 * z;
+  }
   su2 ux[3], uy[3];
   int sy[3];
   vec3 af;
@@ -677,39 +754,15 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   // its round trip overlaps theirs
   if (p.guarded && p.obs[OBS_GF_DONE] != 0.0) return;
   if (p.check) {
-    double da = gfix_da(p.part, h.nb, (double)g.n);
+    double da = gfix_da(p.part_old, p.ntiles, (double)p.n);
     if (gfix_stop(da, p.iter, p.limit_or, p.max_iter, p.obs, blk == 0 && threadIdx.x == 0))
       return;  // block-uniform
   }
   double red[1] = {0.0};
   if (act) {
-    // :97-107, :116-142
-    su2 s1{c_add(ux[0].a, ux[1].a), c_add(ux[0].b, ux[1].b)};
-    s1.a = c_add(s1.a, c_scale(p.alpha, ux[2].a));
-    s1.b = c_add(s1.b, c_scale(p.alpha, ux[2].b));
-    su2 s2{c_add(uy[0].a, uy[1].a), c_add(uy[0].b, uy[1].b)};
-    s2.a = c_add(s2.a, c_scale(p.alpha, uy[2].a));
-    s2.b = c_add(s2.b, c_scale(p.alpha, uy[2].b));
-    su2 w{c_add(s1.a, c_conj(s2.a)), c_sub(s1.b, s2.b)};  // :145-146
-    if (DA) {                                              // :153-158
-      double d = c_sub(s1.a, s2.a).im;
-      red[0] = d * d + (w.b.re * w.b.re + w.b.im * w.b.im);
-    }
-    double k = (w.a.re * w.a.re + w.a.im * w.a.im) + (w.b.re * w.b.re + w.b.im * w.b.im);
-    double rk = rsqrt(k);  // w / sqrt(k), :169-183
-    su2 o{c_scale(rk, w.a), c_scale(rk, w.b)};
-    double ra = fmin(1.0, fmax(-1.0, o.a.re));
-    double th = acos(ra);
-    if (th != 0.0) {
-      double tho = p.lambda * th, sn, cs;
-      sincos(tho, &sn, &cs);
-      // sin(th) for th = acos(ra) in (0, pi] is sqrt((1 - ra)(1 + ra)); the
-      // factored form keeps full relative precision as th -> 0
-      double f = sn * rsqrt((1.0 - ra) * (1.0 + ra));
-      double t2 = f * o.a.im;
-      o.a = c_mk(cs, -t2);
-      o.b = c_mk(-(f * o.b.re), -(f * o.b.im));
-    }
+    su2 s1 = gfix_sum(p.alpha, ux), s2 = gfix_sum(p.alpha, uy), w = gfix_w(s1, s2);
+    if (DA) red[0] = gfix_site_da(s1, s2, w);
+    su2 o = gfix_rotation(w, p.lambda);
     st_higgs(Af, g, eo, s, adj_rot<false>(o, af));  // g X(a_f) g^+, :243-252
 #pragma unroll
     for (int mu = 0; mu < 3; ++mu) {  // :256-324
@@ -723,7 +776,141 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
       st_link(Uf, g, mu, oe, sy[mu], ny);
     }
   }
-  if (DA) block_sum_store<1>(red, p.part, p.pstride, blk);
+  if (DA) block_sum_store<1>(red, p.part, 0, blk);
+}
+
+// Slot of the even site at tile coordinates (x, y, z), which is in the tile
+// (0..255, in the order of tile_odd_site) or one step out of it along one axis:
+// x = -1 16 slots from 256, x = 16 from 272, y = -1 32 from 288, y = 8 from 320,
+// z = -1 64 from 352, z = 4 from 416
+constexpr int GT_SLOTS = 480, GT_TB = 512;
+__device__ __forceinline__ int tile_slot(int x, int y, int z) {
+  if (x < 0) return 256 + 4 * z + (y >> 1);
+  if (x >= GT_X) return 272 + 4 * z + (y >> 1);
+  if (y < 0) return 288 + 8 * z + (x >> 1);
+  if (y >= GT_Y) return 320 + 8 * z + (x >> 1);
+  if (z < 0) return 352 + 8 * y + (x >> 1);
+  if (z >= GT_Z) return 416 + 8 * y + (x >> 1);
+  return 64 * z + 8 * y + (x >> 1);
+}
+// and the site of slot e
+__device__ __forceinline__ TileSite tile_even_site(int e) {
+  if (e < 256) {
+    int y = (e >> 3) & 7, z = e >> 6;
+    return TileSite{2 * (e & 7) + ((y + z) & 1), y, z};
+  }
+  if (e < 288) {  // x = -1 beside odd sites at x = 0: y + z odd; x = 16: even
+    int f = (e - 256) & 15, far = e >= 272, z = f >> 2;
+    return TileSite{far ? GT_X : -1, 2 * (f & 3) + ((z + 1 + far) & 1), z};
+  }
+  if (e < 352) {
+    int f = (e - 288) & 31, far = e >= 320, z = f >> 3;
+    return TileSite{2 * (f & 7) + ((z + 1 + far) & 1), far ? GT_Y : -1, z};
+  }
+  int f = (e - 352) & 63, far = e >= 416, y = f >> 3;
+  return TileSite{2 * (f & 7) + ((y + 1 + far) & 1), y, far ? GT_Z : -1};
+}
+
+// One landau_gauge iteration, both half steps and u_f_renorm, from the links
+// src to dst.  A block owns a tile's 256 odd sites, whose six links each are
+// every link once.  The even half step's rotations that those links see, of the
+// tile's even sites and the ones a step outside it, are formed first, one per
+// thread, into LDS (480 for 256 sites; the ones outside are another block's
+// too, and come out the same there, since src does not change).  Then each odd
+// site applies them to its links, takes its own rotation, and writes its links
+// normalised.  Both half steps as launches of their own read and write every
+// link: 768 bytes a site of the lattice and iteration, here about 480, and one
+// launch instead of two.  The arithmetic per site and link is k_gfix's.
+// What bounds it is the FP64 issue of 736 rotations for 512 sites on the
+// lattices the Infinity Cache holds, and the launch below 40^3.  An iteration in
+// us, two launches and one: 8^3 8.6 6.4, 16^3 8.6 6.9, 32^3 9.4 7.4, 48^3 12.1
+// 9.1, 64^3 18.5 14.1, 96^3 56 43, 160^3 361 288; 4^3 (16 odd sites) even.
+__global__ __launch_bounds__(GT_TB) void k_gfix_iter(const double* __restrict__ src,
+                                                     double* __restrict__ dst,
+                                                     double* __restrict__ Af, uint64_t h1_ly,
+                                                     uint64_t lz_npad, uint64_t tiles_ntx,
+                                                     uint64_t nty_n, GfArgs p) {
+  __shared__ double2 ga[GT_SLOTS], gb[GT_SLOTS];
+  const int h1 = half0(h1_ly), ly = half1(h1_ly), lz = half0(lz_npad), lx = 2 * h1;
+  Geom g{0, 0, 0, h1, h1 * ly, half1(nty_n), half1(lz_npad), 0.0f, 0.0f, (ly - 1) * h1,
+         (lz - 1) * h1 * ly};
+  const int blk = xcd_block(half0(tiles_ntx)), tid = threadIdx.x;
+  const TileOrigin o = tile_origin(blk, half1(tiles_ntx), half0(nty_n));
+  // the even sites
+  const TileSite te = tile_even_site(min(tid, GT_SLOTS - 1));
+  int ex = o.x + te.x, ey = o.y + te.y, ez = o.z + te.z;
+  const bool eact = tid < GT_SLOTS && ex <= lx && ey <= ly && ez <= lz;
+  const bool own = tid < 256 && ex < lx && ey < ly && ez < lz;
+  ex = ex < 0 ? lx - 1 : ex >= lx ? ex - lx : ex;
+  ey = ey < 0 ? ly - 1 : ey >= ly ? ey - ly : ey;
+  ez = ez < 0 ? lz - 1 : ez >= lz ? ez - lz : ez;
+  const unsigned es = (unsigned)((ex >> 1) + g.h1 * ey + g.h2 * ez);
+  su2 ux[3], uy[3];
+  vec3 ae;
+  if (eact) {
+    Steps st = site_steps(g, Coord{ex >> 1, ey * g.h1, ez * g.h2, (bool)(ex & 1)});
+#pragma unroll
+    for (int mu = 0; mu < 3; ++mu) {
+      ux[mu] = ld_link(src, g, mu, 0, es);
+      uy[mu] = ld_link(src, g, mu, 1, (unsigned)((int)es + st.m[mu]));
+    }
+    if (own) ae = ld_higgs(Af, g, 0, es);
+  }
+  // the loop condition, as in k_gfix
+  if (p.obs[OBS_GF_DONE] != 0.0) return;
+  if (p.check) {
+    double da = gfix_da(p.part_old, p.ntiles, (double)p.n);
+    if (gfix_stop(da, p.iter, p.limit_or, p.max_iter, p.obs, blk == 0 && tid == 0)) return;
+  }
+  su2 w;
+  if (eact) w = gfix_w(gfix_sum(p.alpha, ux), gfix_sum(p.alpha, uy));
+  // the odd site's operands, on their way while the even rotation is formed
+  const TileSite t = tile_odd_site(tid & 255);
+  const int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
+  const bool act = tid < 256 && x < lx && y < ly && z < lz;
+  const int s = (x >> 1) + g.h1 * y + g.h2 * z;
+  int sy[3];
+  vec3 ao;
+  if (act) {
+    Steps st = site_steps(g, Coord{x >> 1, y * g.h1, z * g.h2, (bool)(x & 1)});
+#pragma unroll
+    for (int mu = 0; mu < 3; ++mu) {
+      sy[mu] = s + st.m[mu];
+      ux[mu] = ld_link(src, g, mu, 1, (unsigned)s);
+      uy[mu] = ld_link(src, g, mu, 0, (unsigned)sy[mu]);
+    }
+    ao = ld_higgs(Af, g, 1, (unsigned)s);
+  }
+  if (eact) {
+    su2 r = gfix_rotation(w, p.lambda);
+    ga[tid] = double2{r.a.re, r.a.im};
+    gb[tid] = double2{r.b.re, r.b.im};
+    if (own) st_higgs(Af, g, 0, es, adj_rot<false>(r, ae));
+  }
+  __syncthreads();
+  double red[1] = {0.0};
+  if (act) {
+    auto rot = [&](int dx, int dy, int dz) {
+      int e = tile_slot(t.x + dx, t.y + dy, t.z + dz);
+      return su2{c_mk(ga[e].x, ga[e].y), c_mk(gb[e].x, gb[e].y)};
+    };
+#pragma unroll
+    for (int mu = 0; mu < 3; ++mu) {
+      ux[mu] = m_nd(ux[mu], rot(mu == 0, mu == 1, mu == 2));
+      uy[mu] = m_nn(rot(-(mu == 0), -(mu == 1), -(mu == 2)), uy[mu]);
+    }
+    su2 s1 = gfix_sum(p.alpha, ux), s2 = gfix_sum(p.alpha, uy);
+    w = gfix_w(s1, s2);
+    red[0] = gfix_site_da(s1, s2, w);
+    su2 r = gfix_rotation(w, p.lambda);
+    st_higgs(Af, g, 1, (unsigned)s, adj_rot<false>(r, ao));
+#pragma unroll
+    for (int mu = 0; mu < 3; ++mu) {
+      st_link(dst, g, mu, 1, (unsigned)s, normalized(m_nn(r, ux[mu])));
+      st_link(dst, g, mu, 0, (unsigned)sy[mu], normalized(m_nd(uy[mu], r)));
+    }
+  }
+  block_sum_store<1, GT_TB / 64>(red, p.part, 0, blk);
 }
 
 // da1 after one or_gauge_fixing call (guarded = 0), or the convergence test
@@ -772,47 +959,80 @@ __global__ __launch_bounds__(TB) void k_gfix_begin(const double2* __restrict__ U
   }
 }
 
-void launch_gfix_begin(lceq_lattice* L) {
-  unsigned nu = 12 * (unsigned)L->g.npad, na = 3 * (unsigned)L->g.npad;
+void launch_gfix_begin(lceq_lattice* L, bool links) {
+  unsigned nu = links ? 12 * (unsigned)L->g.npad : 0, na = 3 * (unsigned)L->g.npad;
   hipLaunchKernelGGL(k_gfix_begin, dim3((nu + na + TB - 1) / TB), dim3(TB), 0, L->stream,
                      (const double2*)L->U, (const double2*)L->A, (double2*)L->Uf,
                      (double2*)L->Af, nu, na, L->obs);
 }
 
-void launch_gfix(lceq_lattice* L, int eo, int compute_da, int renorm, int guarded, int check,
-                 int iter) {
+static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
+  const Geom& g = L->g;
   GfArgs a;
   a.guarded = guarded;
+  a.lx = g.lx;
+  a.ly = g.ly;
+  a.lz = g.lz;
+  a.ntx = gf_tiles_along(g.lx, GT_X);
+  a.nty = gf_tiles_along(g.ly, GT_Y);
   a.lambda = L->lambda;
   a.alpha = L->alpha;
   a.obs = L->obs;
-  a.part = L->partials;
-  a.pstride = L->pstride;
+  a.part = L->gf_part;
+  a.part_old = L->gf_part;
+  a.ntiles = gfix_tiles(g);
+  a.n = g.n;
   a.check = check;
   a.iter = (double)iter;
   a.limit_or = L->limit_or;
   a.max_iter = (double)L->max_iter;
+  return a;
+}
+
+void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, int iter) {
+  GfArgs a = gfix_args(L, guarded, check, iter);
   prof_begin(L, KC_GFIX);
   prof_count(L, KC_GFIX);
-  int nb = blocks_for(L->g.n);
+  int nb = eo ? a.ntiles : blocks_for(L->g.n);
   HeadArgs h = head_args(L, L->Uf, L->Af, nb, eo);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A, h.n, h.b, h.h, h.w, h.r,
                        a);
   };
-  if (renorm)
-    launch(k_gfix<true, true>);
-  else if (compute_da)
-    launch(k_gfix<true, false>);
-  else
+  if (!eo)
     launch(k_gfix<false, false>);
+  else if (renorm)
+    launch(k_gfix<true, true>);
+  else
+    launch(k_gfix<true, false>);
   prof_end(L, KC_GFIX);
 }
 
-void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host) {
-  hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream, L->partials,
-                     blocks_for(L->g.n), (double)L->g.n, guarded, (double)iter, L->limit_or,
-                     (double)L->max_iter, L->obs, to_host ? L->pin : nullptr);
+// The link array iteration `iter` (from 1) of the one-launch loop writes: u_f
+// and the second array in turn
+static double* gfix_out(const lceq_lattice* L, int iter) { return iter & 1 ? L->Uf : L->Ug; }
+
+void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
+  GfArgs a = gfix_args(L, 1, check, iter - 1);
+  // the partials too: a block may write its own while another still tests
+  a.part = L->gf_part + (size_t)(iter & 1) * a.ntiles;
+  a.part_old = L->gf_part + (size_t)((iter - 1) & 1) * a.ntiles;
+  const Geom& g = L->g;
+  prof_begin(L, KC_GFIX);
+  prof_count(L, KC_GFIX);
+  hipLaunchKernelGGL(k_gfix_iter, dim3(a.ntiles), dim3(GT_TB), 0, L->stream,
+                     iter == 1 ? L->U : gfix_out(L, iter - 1), gfix_out(L, iter), L->Af,
+                     halves(g.h1, g.ly), halves(g.lz, g.npad), halves(a.ntiles, a.ntx),
+                     halves(a.nty, g.n), a);
+  prof_end(L, KC_GFIX);
+}
+
+void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch) {
+  int nt = gfix_tiles(L->g);
+  hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream,
+                     L->gf_part + (one_launch ? (size_t)(iter & 1) * nt : 0), nt, (double)L->g.n,
+                     guarded, (double)iter, L->limit_or, (double)L->max_iter, L->obs,
+                     to_host ? L->pin : nullptr);
 }
 
 // ========================================================== correlators

@@ -78,3 +78,37 @@ def test_iteration_cap(cap, shape):
     H, _, n = _host_loop(shape, u, a, 1.7, 1.0, 1e-14, cap)
     assert n == cap
     assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
+
+
+@pytest.mark.parametrize("shape,alpha", [((2, 2, 2), 1.0), ((2, 4, 6), 0.8), ((18, 2, 4), 1.0),
+                                         ((16, 8, 4), 1.0), ((14, 10, 6), 1.0), ((34, 18, 10), 0.7),
+                                         ((16, 16, 16), 1.0), ((30, 6, 130), 1.0),
+                                         ((66, 34, 26), 1.0)])
+@pytest.mark.parametrize("cap", [1, 2, 9, 24])
+def test_tiles_equal_the_half_steps(shape, alpha, cap):
+    """An iteration in one launch over tiles of 16 x 8 x 4 sites against the two
+    half steps as launches of their own: tiles cut off at every face, extents of
+    2, one tile, more than 64 tiles (the loop condition by block sums), and an odd
+    and an even number of iterations (the result in either link array)."""
+    import lceqcd_amd
+    print("landau_gauge tiles", shape, cap, flush=True)
+    rng = np.random.default_rng(3)
+    n = shape[0] * shape[1] * shape[2] // 2
+    u = rng.normal(size=(3, 2, n, 4))
+    u /= np.linalg.norm(u, axis=-1, keepdims=True)
+    a = rng.normal(size=(2, n, 3))
+    G = lceqcd_amd.Lattice(*shape)
+    G.put_links(u)
+    G.put_higgs(a)
+    G.set_gauge_fixing(1.7, alpha, 1e-300, cap)
+    H, da, done = _host_loop(shape, u, a, 1.7, alpha, 1e-300, cap)
+    assert done == cap
+    for _ in range(2):  # the second call starts from the other link array
+        with pytest.raises(lceqcd_amd.LceqError, match="da = %g" % da):
+            G.landau_gauge()
+        assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
+        assert np.array_equal(G.get_higgs_fixed(), H.get_higgs_fixed())
+        assert np.array_equal(G.get_links(), u)
+    G.or_gauge_fixing()
+    H.or_gauge_fixing()
+    assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
