@@ -12,7 +12,7 @@ ROOT = os.path.dirname(HERE)
 SRC = [os.path.join(HERE, "csrc", f) for f in ("lceq_kernels.hip", "lceq_api.hip", "lceq_batch.hip",
                                                    "lceq_ranlux.hip", "lceq_conf.hip",
                                                    "lceq_mlp.hip", "lceq_static.hip",
-                                                   "lceq_transfer.hip")]
+                                                   "lceq_transfer.hip", "lceq_link3.hip")]
 OUT = os.path.join(HERE, "liblceq.so")
 # Test-only build of the same sources: every operation rounded as written
 # (no contraction) and 1/sqrt, cos(2 pi r) in the CPU restatement's forms

@@ -88,7 +88,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   alloc(&L->Af, 6 * np);
   alloc(&L->Vst, 24 * np);
   alloc(&L->F, 3 * np);
-  alloc(&L->gf_part, 2 * (size_t)gfix_tiles(g));
+  alloc(&L->gf_part, 2 * (size_t)lattice_tiles(g));
   alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
 
   alloc(&L->obs, LCEQ_OBS_N);
@@ -126,8 +126,8 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
 extern "C" int lceq_destroy(lceq_lattice* L) {
   if (!L) return LCEQ_OK;
   if (L->stream) (void)hipStreamSynchronize(L->stream);
-  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->Ug, L->gf_part, L->partials, L->obs,
-                    L->slices, L->corr, L->hist, L->scratch, L->fed};
+  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->Ug, L->U2, L->gf_part,
+                    L->partials, L->obs, L->slices, L->corr, L->hist, L->scratch, L->fed};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
   if (L->pin) (void)hipHostFree(L->pin);
@@ -658,10 +658,38 @@ extern "C" int lceq_heat_kpi(lceq_lattice* L, int n, const double* b, double* v,
   return LCEQ_OK;
 }
 
+static bool link3_ready(lceq_lattice* L) {
+  if (L->rng_mode != LCEQ_RNG_PHILOX || L->prof_class || L->no_U2 || !link3_tiles(L->g))
+    return false;
+  if (L->U2) return true;
+  const size_t bytes = 24 * (size_t)L->g.npad * sizeof(double);
+  if (hipMalloc((void**)&L->U2, bytes) == hipSuccess) {
+    (void)hipMemsetAsync(L->U2, 0, bytes, L->stream);  // padding lanes hold finite values
+  } else {
+    (void)hipGetLastError();
+    L->U2 = nullptr;
+    L->no_U2 = true;  // the launches per direction need no second array
+  }
+  return L->U2 != nullptr;
+}
+
 // one full link sweep (eo outer, mu inner as in f/agauge.f:53-57); with
 // reduce the six launches leave their plaquette and acceptance partial sums
 // in slots 0-5 for launch_finalize
+//
+// A Philox sweep without sums, all but one of a production sweep's, runs the
+// three directions of a parity in one launch (launch_link3) where link3_tiles
+// says so, from one link array to another; the arrays then change places.
 int link_sweep(lceq_lattice* L, int kp, int measflag, int renorm_on_write, int reduce) {
+  if (!reduce && !measflag && link3_ready(L)) {
+    for (int eo = 0; eo < 2; ++eo) {
+      uint64_t pass = L->pass;
+      L->pass += 3;
+      launch_link3(L, kp, eo, renorm_on_write, L->U, eo ? L->U2 : L->U, L->U2, pass);
+    }
+    std::swap(L->U, L->U2);
+    return check_launch();
+  }
   int64_t per = (kp ? 7 : 1) * (int64_t)L->g.n;
   const double* fed0;
   int rc = take_uniforms(L, 6 * per, &fed0);
@@ -836,7 +864,7 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   // partials costs more than a one-block test launch per iteration (26 us
   // of a 352 us iteration at 160^3), so there each iteration is followed by
   // the finalize instead: the same sum in the same order, the same stop.
-  const bool test_launch = gfix_tiles(L->g) > 2048;
+  const bool test_launch = lattice_tiles(L->g) > 2048;
   // The iterations left are estimated from the decay of da over the last
   // batch, which is close to geometric once the fields are smooth; a batch takes
   // at most 7/8 of them, so that few launches are left over at the end (a
@@ -1014,7 +1042,7 @@ static SlabPlan slab_plan(const lceq_lattice* L) {
   SlabPlan p;
   const Geom& g = L->g;
   // lattices up to this size gain nothing: their launches run at the cache's rate
-  if (240 * (int64_t)g.npad <= (int64_t)288 << 20) return p;
+  if (fields_fit(g)) return p;
   if (L->rng_mode != LCEQ_RNG_PHILOX || L->prof_class) return p;
   const int planes = (int)std::min<int64_t>(SLAB_BYTES / (240 * (int64_t)g.h2), g.lz);
   // two slabs if they do, with the most passes (up to 16) that let both fit

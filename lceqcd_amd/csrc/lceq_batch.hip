@@ -580,9 +580,6 @@ extern "C" int lceq_batch_get_higgs(lceq_batch* B, int r, double* a, int64_t ld)
 #define BATCH_ARGS(c, flags, pass)                                                            \
   (c).heads, halves((c).total_nb, (c).blk_base),                                              \
       halves((flags) | ((c).xcd ? BATCH_XCD : 0), pass), (c).reps, (c).ctr, (c).obs
-static uint64_t halves(int a, int b) {
-  return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
-}
 
 template <bool KP, int TBX>
 static void enqueue_link(lceq_batch* B, const BatchCommon& c, int flags, int mu, int pass) {

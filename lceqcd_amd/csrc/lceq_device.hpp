@@ -256,6 +256,28 @@ __device__ __forceinline__ void unit(int mu, int& dx, int& dy, int& dz) {
   dz = mu == 2;
 }
 
+// Pairs of 32-bit kernel arguments in one 64-bit value
+__host__ __device__ inline uint64_t halves(int a, int b) {
+  return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
+}
+__device__ __forceinline__ int half0(uint64_t v) { return (int)(uint32_t)v; }
+__device__ __forceinline__ int half1(uint64_t v) { return (int)(uint32_t)(v >> 32); }
+
+// Tiles of TX x TY x TZ sites, cut off at the lattice's far faces, numbered x
+// first (ntx, nty: the tiles along x and y)
+inline int tiles_along(int l, int t) { return (l + t - 1) / t; }
+struct TileOrigin {
+  int x, y, z;
+};
+template <int TX, int TY, int TZ>
+__device__ __forceinline__ TileOrigin tile_origin(int tile, int ntx, int nty) {
+  int nxy = ntx * nty;
+  int tz = div_small(tile, nxy, __builtin_amdgcn_rcpf((float)nxy));
+  int r = tile - tz * nxy;
+  int ty = div_small(r, ntx, __builtin_amdgcn_rcpf((float)ntx));
+  return TileOrigin{TX * (r - ty * ntx), TY * ty, TZ * tz};
+}
+
 // ------------------------------------------------------------- storage
 
 // Links: U_mu at parity p, site s as two 16-byte halves

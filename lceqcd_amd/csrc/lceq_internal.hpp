@@ -41,7 +41,9 @@ struct lceq_lattice {
   // device fields
   double *U, *A, *Uf, *Af, *Vst, *F;
   double* Ug;        // second link array of landau_gauge, from its first call on
-  double* gf_part;   // da partials of two iterations [2][gfix_tiles]
+  double* U2;        // second link array of the link sweeps, from the first one on
+  bool no_U2;        // there was no memory for it
+  double* gf_part;   // da partials of two iterations [2][lattice_tiles]
   double *partials;  // [LCEQ_NSLOT][LCEQ_NQ][pstride]
   int pstride;       // >= number of 64-site blocks (the smallest launch shape)
   double *obs;       // [LCEQ_OBS_N]
@@ -100,6 +102,14 @@ inline const char* geom_reject(int lx, int ly, int lz) {
 
 enum KernelClass { KC_NONE = 0, KC_LINK_KP = 1, KC_LINK_OR = 2, KC_HIGGS = 3, KC_GFIX = 4 };
 
+// Tiles of the gauge fixing kernels (256 sites of each parity)
+constexpr int GT_X = 16, GT_Y = 8, GT_Z = 4;
+inline int lattice_tiles(const Geom& g) {
+  return tiles_along(g.lx, GT_X) * tiles_along(g.ly, GT_Y) * tiles_along(g.lz, GT_Z);
+}
+// the fields of a lattice (240 bytes per site of a parity) are at most 288 MiB:
+// about the Infinity Cache
+inline bool fields_fit(const Geom& g) { return 240 * (int64_t)g.npad <= (int64_t)288 << 20; }
 int blocks_for(int n);
 // the strip rows of the update launches' site order (0: index order)
 int strip_rows(const lceq_lattice* L);
@@ -145,6 +155,13 @@ struct SiteRange {
 };
 void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int renorm_on_write,
                  const double* fed, uint64_t pass, int reduce, const SiteRange* range = nullptr);
+// A link sweep without partial sums (Philox), three directions of parity eo in
+// one launch: passes pass .. pass + 2, from the links `src` (of parity eo) and
+// `other` (of the other one) to `dst`, another array than `src`.  link3_tiles:
+// its blocks on lattices where it is the faster way, otherwise 0
+int link3_tiles(const Geom& g);
+void launch_link3(lceq_lattice* L, int kp, int eo, int renorm_on_write, const double* src,
+                  const double* other, double* dst, uint64_t pass);
 // One-block reduction of the partial sums into the observables: link_kind
 // 0 none, 1 KP (agauge), 2 overrelaxation; higgs_kind 0 none, 1-3 ahiggs1-3;
 // with hist_row the observables are also copied into that history row.
@@ -178,8 +195,6 @@ void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, 
 // a_f = a, with `links` u_f = u, and the loop's observables as before its first
 // iteration
 void launch_gfix_begin(lceq_lattice* L, bool links);
-// da partials of an iteration
-int gfix_tiles(const Geom& g);
 // blocks per z slice of the slice sums (the slices buffer holds 14 lz split)
 int corr_split(const Geom& g);
 // the slice sums and correlators of measurement meas (0 correlator, which

@@ -35,8 +35,6 @@ struct Head {
   Geom g;  // without the extents
   int nb, flags;
 };
-__device__ __forceinline__ int half0(uint64_t v) { return (int)(uint32_t)v; }
-__device__ __forceinline__ int half1(uint64_t v) { return (int)(uint32_t)(v >> 32); }
 __device__ __forceinline__ Head head_of(double* U, double* A, uint64_t hn, uint64_t hb,
                                         uint64_t hh, uint64_t hw, uint64_t hr) {
   Geom g{0, 0, 0, half0(hh), half1(hh), half0(hn), half1(hn),
@@ -49,9 +47,6 @@ struct HeadArgs {
   double *U, *A;
   uint64_t n, b, h, w, r;
 };
-static uint64_t halves(int a, int b) {
-  return (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
-}
 // r: the launch covers a range of the sites only; its head then carries the
 // range's length and start in place of n and the number of blocks
 static HeadArgs head_args(const lceq_lattice* L, double* U, double* A, int nb, int eo,
@@ -586,24 +581,6 @@ void launch_check_fields(lceq_lattice* L, double* part) {
 
 // ========================================================= gauge fixing
 
-// Tiles of GT_X x GT_Y x GT_Z sites, cut off at the lattice's far faces: the
-// odd half step's blocks, 256 odd sites each
-constexpr int GT_X = 16, GT_Y = 8, GT_Z = 4;
-static int gf_tiles_along(int l, int t) { return (l + t - 1) / t; }
-int gfix_tiles(const Geom& g) {
-  return gf_tiles_along(g.lx, GT_X) * gf_tiles_along(g.ly, GT_Y) * gf_tiles_along(g.lz, GT_Z);
-}
-
-struct TileOrigin {
-  int x, y, z;
-};
-__device__ __forceinline__ TileOrigin tile_origin(int tile, int ntx, int nty) {
-  int nxy = ntx * nty;
-  int tz = div_small(tile, nxy, __builtin_amdgcn_rcpf((float)nxy));
-  int r = tile - tz * nxy;
-  int ty = div_small(r, ntx, __builtin_amdgcn_rcpf((float)ntx));
-  return TileOrigin{GT_X * (r - ty * ntx), GT_Y * ty, GT_Z * tz};
-}
 // odd site i (0..255) of a tile, in tile coordinates
 struct TileSite {
   int x, y, z;
@@ -731,7 +708,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   int eo = DA ? 1 : h.flags & HEAD_EO, oe = eo ^ 1;
   bool act = s < g.n;
   if (DA) {
-    TileOrigin o = tile_origin(blk, p.ntx, p.nty);
+    TileOrigin o = tile_origin<GT_X, GT_Y, GT_Z>(blk, p.ntx, p.nty);
     TileSite t = tile_odd_site(threadIdx.x);
     int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
     act = x < p.lx && y < p.ly && z < p.lz;
@@ -835,7 +812,7 @@ __global__ __launch_bounds__(GT_TB) void k_gfix_iter(const double* __restrict__ 
   Geom g{0, 0, 0, h1, h1 * ly, half1(nty_n), half1(lz_npad), 0.0f, 0.0f, (ly - 1) * h1,
          (lz - 1) * h1 * ly};
   const int blk = xcd_block(half0(tiles_ntx)), tid = threadIdx.x;
-  const TileOrigin o = tile_origin(blk, half1(tiles_ntx), half0(nty_n));
+  const TileOrigin o = tile_origin<GT_X, GT_Y, GT_Z>(blk, half1(tiles_ntx), half0(nty_n));
   // the even sites
   const TileSite te = tile_even_site(min(tid, GT_SLOTS - 1));
   int ex = o.x + te.x, ey = o.y + te.y, ez = o.z + te.z;
@@ -973,14 +950,14 @@ static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
   a.lx = g.lx;
   a.ly = g.ly;
   a.lz = g.lz;
-  a.ntx = gf_tiles_along(g.lx, GT_X);
-  a.nty = gf_tiles_along(g.ly, GT_Y);
+  a.ntx = tiles_along(g.lx, GT_X);
+  a.nty = tiles_along(g.ly, GT_Y);
   a.lambda = L->lambda;
   a.alpha = L->alpha;
   a.obs = L->obs;
   a.part = L->gf_part;
   a.part_old = L->gf_part;
-  a.ntiles = gfix_tiles(g);
+  a.ntiles = lattice_tiles(g);
   a.n = g.n;
   a.check = check;
   a.iter = (double)iter;
@@ -1028,7 +1005,7 @@ void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
 }
 
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch) {
-  int nt = gfix_tiles(L->g);
+  int nt = lattice_tiles(L->g);
   hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream,
                      L->gf_part + (one_launch ? (size_t)(iter & 1) * nt : 0), nt, (double)L->g.n,
                      guarded, (double)iter, L->limit_or, (double)L->max_iter, L->obs,

@@ -198,11 +198,12 @@ __device__ __forceinline__ void link_prepare(const LinkSite& p, unsigned s, Link
 
 // Update phase of one (eo, mu) class of f/agauge.f:53-193 (KP=true), or the
 // link overrelaxation U -> Vhat^+ U^+ Vhat^+ with the same hopping
-// Metropolis (KP=false).  Partials (added to red): 0 plaquette, 1 KP
-// accepts, 2 Metropolis accepts.
+// Metropolis (KP=false): the link after the update, and whether the Metropolis
+// step took it.  Partials (added to red): 0 plaquette, 1 KP accepts, 2
+// Metropolis accepts.
 template <bool KP>
-__device__ __forceinline__ void link_finish(const LinkSite& p, unsigned s, const LinkOperands& o,
-                                            double (&red)[3]) {
+__device__ __forceinline__ su2 link_value(const LinkSite& p, const LinkOperands& o, bool& taken,
+                                          double (&red)[3]) {
   su2 u = o.u;
   // the old hopping action (f/agauge.f:124-126, 140-147) from the first operands to
   // arrive, ahead of the staple sum; 1.7% off the overrelaxation launch
@@ -239,13 +240,22 @@ __device__ __forceinline__ void link_finish(const LinkSite& p, unsigned s, const
             c_mk(-(d2 * vh.b.re) - u.b.re, -(d2 * vh.b.im) - u.b.im)};
   }
   double sa_n = hop_action(p.beta_a, o.ax, o.axp, hs, h);
-  if (exp(sa_o - sa_n) >= o.racc) {  // f/agauge.f:167-174
+  taken = exp(sa_o - sa_n) >= o.racc;  // f/agauge.f:167-174
+  if (taken) {
     u = p.renorm ? normalized(h) : h;
-    st_link(p.U, p.g, p.mu, p.eo, s, u);
     red[2] += 1.0;
   }
   if (p.measflag == 1) red[0] += m_nn(u, V).a.re;  // f/agauge.f:179-185
+  return u;
 }
+template <bool KP>
+__device__ __forceinline__ void link_finish(const LinkSite& p, unsigned s, const LinkOperands& o,
+                                            double (&red)[3]) {
+  bool taken;
+  su2 u = link_value<KP>(p, o, taken, red);
+  if (taken) st_link(p.U, p.g, p.mu, p.eo, s, u);
+}
+
 
 // One site: all operand loads are issued before any arithmetic, so that one
 // memory latency covers the site; the uniform phase runs under it.
