@@ -51,6 +51,21 @@ extern "C" const char* lceq_last_error(void) { return g_err.c_str(); }
 
 // ------------------------------------------------------------ lifecycle
 
+// The second link array; without memory for it the callers take their launches
+// in place
+static bool spare_links(lceq_lattice* L) {
+  if (L->spare) return true;
+  const size_t bytes = 24 * (size_t)L->g.npad * sizeof(double);
+  if (hipMalloc((void**)&L->spare, bytes) == hipSuccess) {
+    // padding lanes hold finite values
+    (void)hipMemsetAsync(L->spare, 0, bytes, L->stream);
+  } else {
+    (void)hipGetLastError();
+    L->spare = nullptr;
+  }
+  return L->spare != nullptr;
+}
+
 extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   if (!out) return fail(LCEQ_ERR_ARG, "null output pointer");
   *out = nullptr;
@@ -111,6 +126,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
     (void)hipMemsetAsync(L->partials, 0, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride * sizeof(double),
                    L->stream);
     (void)hipMemsetAsync(L->obs, 0, LCEQ_OBS_N * sizeof(double), L->stream);
+    if (link3_tiles(L->g)) (void)spare_links(L);
 
     if (hipStreamSynchronize(L->stream) != hipSuccess) rc = fail(LCEQ_ERR_HIP, "init sync failed");
   }
@@ -126,7 +142,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
 extern "C" int lceq_destroy(lceq_lattice* L) {
   if (!L) return LCEQ_OK;
   if (L->stream) (void)hipStreamSynchronize(L->stream);
-  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->Ug, L->U2, L->gf_part,
+  double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->spare, L->gf_part,
                     L->partials, L->obs, L->slices, L->corr, L->hist, L->scratch, L->fed};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
@@ -658,21 +674,6 @@ extern "C" int lceq_heat_kpi(lceq_lattice* L, int n, const double* b, double* v,
   return LCEQ_OK;
 }
 
-static bool link3_ready(lceq_lattice* L) {
-  if (L->rng_mode != LCEQ_RNG_PHILOX || L->prof_class || L->no_U2 || !link3_tiles(L->g))
-    return false;
-  if (L->U2) return true;
-  const size_t bytes = 24 * (size_t)L->g.npad * sizeof(double);
-  if (hipMalloc((void**)&L->U2, bytes) == hipSuccess) {
-    (void)hipMemsetAsync(L->U2, 0, bytes, L->stream);  // padding lanes hold finite values
-  } else {
-    (void)hipGetLastError();
-    L->U2 = nullptr;
-    L->no_U2 = true;  // the launches per direction need no second array
-  }
-  return L->U2 != nullptr;
-}
-
 // one full link sweep (eo outer, mu inner as in f/agauge.f:53-57); with
 // reduce the six launches leave their plaquette and acceptance partial sums
 // in slots 0-5 for launch_finalize
@@ -681,13 +682,15 @@ static bool link3_ready(lceq_lattice* L) {
 // three directions of a parity in one launch (launch_link3) where link3_tiles
 // says so, from one link array to another; the arrays then change places.
 int link_sweep(lceq_lattice* L, int kp, int measflag, int renorm_on_write, int reduce) {
-  if (!reduce && !measflag && link3_ready(L)) {
+  if (!reduce && !measflag && L->rng_mode == LCEQ_RNG_PHILOX && !L->prof_class &&
+      link3_tiles(L->g) && L->spare) {
     for (int eo = 0; eo < 2; ++eo) {
       uint64_t pass = L->pass;
       L->pass += 3;
-      launch_link3(L, kp, eo, renorm_on_write, L->U, eo ? L->U2 : L->U, L->U2, pass);
+      launch_link3(L, kp, eo, renorm_on_write, L->U, eo ? L->spare : L->U, L->spare,
+                   pass);
     }
-    std::swap(L->U, L->U2);
+    std::swap(L->U, L->spare);
     return check_launch();
   }
   int64_t per = (kp ? 7 : 1) * (int64_t)L->g.n;
@@ -850,11 +853,7 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   NEEDL(L);
   // one launch per iteration between two link arrays; without memory for the
   // second, two launches in place
-  if (!L->Ug && hipMalloc((void**)&L->Ug, 24 * (size_t)L->g.npad * sizeof(double)) != hipSuccess) {
-    (void)hipGetLastError();
-    L->Ug = nullptr;
-  }
-  const bool one = L->Ug != nullptr;
+  const bool one = spare_links(L);
   launch_gfix_begin(L, !one);
   // Batches of guarded iterations; after convergence (or the cap) the
   // remaining launches of a batch return at once.  Inside a batch the loop
@@ -899,7 +898,7 @@ extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
     batch = next;
   }
   // the last iteration wrote u_f or, for an even one, the second array
-  if (one && (int)o[OBS_ITER] % 2 == 0) std::swap(L->Uf, L->Ug);
+  if (one && (int)o[OBS_ITER] % 2 == 0) std::swap(L->Uf, L->spare);
   if (da1) *da1 = o[OBS_DA];
   if (iter_or1) *iter_or1 = (int)o[OBS_ITER];
   if (o[OBS_GF_CAPPED] != 0.0)

@@ -40,9 +40,11 @@ struct lceq_lattice {
   hipStream_t stream;
   // device fields
   double *U, *A, *Uf, *Af, *Vst, *F;
-  double* Ug;        // second link array of landau_gauge, from its first call on
-  double* U2;        // second link array of the link sweeps, from the first one on
-  bool no_U2;        // there was no memory for it
+  // A second link array (spare_links): link sweeps and landau_gauge read one
+  // array and write the other, which then change places.  Between calls it
+  // holds nothing.  Lattices whose link sweeps use it have it from creation on,
+  // so that a sweep allocates nothing, the others from their first landau_gauge.
+  double* spare;
   double* gf_part;   // da partials of two iterations [2][lattice_tiles]
   double *partials;  // [LCEQ_NSLOT][LCEQ_NQ][pstride]
   int pstride;       // >= number of 64-site blocks (the smallest launch shape)
@@ -188,7 +190,7 @@ void launch_check_fields(lceq_lattice* L, double* part);
 // the loop condition for the `iter` iterations already complete (see k_gfix).
 void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check = 0, int iter = 0);
 // Iteration `iter` (from 1) in one launch, from u or the array the iteration
-// before wrote into the other one of u_f and L->Ug
+// before wrote into the other one of u_f and the second array
 void launch_gfix_iter(lceq_lattice* L, int iter, int check);
 // one_launch: the iterations were launch_gfix_iter's
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch);

@@ -987,7 +987,7 @@ void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, in
 
 // The link array iteration `iter` (from 1) of the one-launch loop writes: u_f
 // and the second array in turn
-static double* gfix_out(const lceq_lattice* L, int iter) { return iter & 1 ? L->Uf : L->Ug; }
+static double* gfix_out(const lceq_lattice* L, int iter) { return iter & 1 ? L->Uf : L->spare; }
 
 void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
   GfArgs a = gfix_args(L, 1, check, iter - 1);
