@@ -207,11 +207,14 @@ __global__ __launch_bounds__(L3_TB) void k_link3(const double* __restrict__ src,
 //   64x64x80 (1280) 233 239, 80x80x64 (1600) 334 304, 96^3 (3456) 608 572,
 //   112x112x96 (4704) 820 757; tiles cut off: 72x72x96 (2160) 371 386,
 //   100^3 (4375) 684 758
-// Above the Infinity Cache the second array would be extra traffic.
+// The second array counts against the Infinity Cache: 128x128x72 (0.25 GB of
+// fields and second array) 786 755, 128x128x80 (0.28) 864 869, 128^3 (0.45)
+// 1362 1643.
 int link3_tiles(const Geom& g) {
   const int nt = tiles_along(g.lx, L3_X) * tiles_along(g.ly, L3_Y) * tiles_along(g.lz, L3_Z);
   const bool whole = g.lx % L3_X == 0 && g.ly % L3_Y == 0 && g.lz % L3_Z == 0;
-  return fields_fit(g) && (nt <= 512 || (nt >= 1600 && whole)) ? nt : 0;
+  const bool cached = (240 + 192) * (int64_t)g.npad <= (int64_t)256 << 20;
+  return cached && (nt <= 512 || (nt >= 1600 && whole)) ? nt : 0;
 }
 
 void launch_link3(lceq_lattice* L, int kp, int eo, int renorm_on_write, const double* src,
