@@ -851,9 +851,14 @@ extern "C" int lceq_or_gauge_fixing(lceq_lattice* L, double* da1) {
 
 extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   NEEDL(L);
-  // one launch per iteration between two link arrays; without memory for the
-  // second, two launches in place
-  const bool one = spare_links(L);
+  // One launch per iteration between two link arrays; two launches in place
+  // without memory for the second, and where the Infinity Cache holds (nearly)
+  // one array and a_f but not two.  us an iteration, in place and in one launch:
+  // 112^3 (303 MB with two arrays) 93 93, 128x128x100 (354) 110 115, 128^3 (453)
+  // 140 168, 132^3 (276 with one) 171 195, 140^3 (329) 230 222, 160^3 361 276
+  const int64_t one_array = 240 * (int64_t)L->g.npad, two_arrays = 432 * (int64_t)L->g.npad;
+  const bool one =
+      (two_arrays <= (int64_t)288 << 20 || one_array > (int64_t)280 << 20) && spare_links(L);
   launch_gfix_begin(L, !one);
   // Batches of guarded iterations; after convergence (or the cap) the
   // remaining launches of a batch return at once.  Inside a batch the loop
@@ -1041,7 +1046,7 @@ static SlabPlan slab_plan(const lceq_lattice* L) {
   SlabPlan p;
   const Geom& g = L->g;
   // lattices up to this size gain nothing: their launches run at the cache's rate
-  if (fields_fit(g)) return p;
+  if (240 * (int64_t)g.npad <= (int64_t)288 << 20) return p;
   if (L->rng_mode != LCEQ_RNG_PHILOX || L->prof_class) return p;
   const int planes = (int)std::min<int64_t>(SLAB_BYTES / (240 * (int64_t)g.h2), g.lz);
   // two slabs if they do, with the most passes (up to 16) that let both fit

@@ -318,15 +318,17 @@ constexpr int CPOL_WRITE_THROUGH = 16;  // sc1
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);
 }
+// WT = false: by way of the L2's write-back (k_gfix_iter)
+template <bool WT = true>
 __device__ __forceinline__ void st_link(double* __restrict__ U, const Geom& g, int mu, int p,
                                         unsigned s, su2 u) {
   double2* q = reinterpret_cast<double2*>(U + (size_t)((mu * 2 + p) * 4) * (size_t)g.npad);
   __builtin_amdgcn_raw_buffer_store_b128(
       __builtin_bit_cast(lceq_v4i, make_double2(u.a.re, u.a.im)), raw_rsrc(q), s * 16u, 0,
-      CPOL_WRITE_THROUGH);
+      WT ? CPOL_WRITE_THROUGH : 0);
   __builtin_amdgcn_raw_buffer_store_b128(
       __builtin_bit_cast(lceq_v4i, make_double2(u.b.re, u.b.im)), raw_rsrc(q + g.npad), s * 16u,
-      0, CPOL_WRITE_THROUGH);
+      0, WT ? CPOL_WRITE_THROUGH : 0);
 }
 __device__ __forceinline__ vec3 ld_higgs(const double* __restrict__ A, const Geom& g, int p,
                                          unsigned s) {

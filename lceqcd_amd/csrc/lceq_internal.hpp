@@ -109,9 +109,6 @@ constexpr int GT_X = 16, GT_Y = 8, GT_Z = 4;
 inline int lattice_tiles(const Geom& g) {
   return tiles_along(g.lx, GT_X) * tiles_along(g.ly, GT_Y) * tiles_along(g.lz, GT_Z);
 }
-// the fields of a lattice (240 bytes per site of a parity) are at most 288 MiB:
-// about the Infinity Cache
-inline bool fields_fit(const Geom& g) { return 240 * (int64_t)g.npad <= (int64_t)288 << 20; }
 int blocks_for(int n);
 // the strip rows of the update launches' site order (0: index order)
 int strip_rows(const lceq_lattice* L);
@@ -192,6 +189,10 @@ void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check = 0
 // Iteration `iter` (from 1) in one launch, from u or the array the iteration
 // before wrote into the other one of u_f and the second array
 void launch_gfix_iter(lceq_lattice* L, int iter, int check);
+// u_f and a_f are within the Infinity Cache
+inline bool gfix_links_cached(const Geom& g) {
+  return (192 + 48) * (int64_t)g.npad <= (int64_t)256 << 20;
+}
 // one_launch: the iterations were launch_gfix_iter's
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch);
 // a_f = a, with `links` u_f = u, and the loop's observables as before its first

@@ -698,7 +698,10 @@ __device__ __forceinline__ su2 gfix_rotation(const su2& w, double lambda) {
 // other half's blocks are index ranges.  DA and RENORM are template arguments:
 // without a branch around each pair, the six normalisations' chains of
 // dependent operations run side by side.
-template <bool DA, bool RENORM>
+// TILES: the blocks of DA are tiles; beyond the Infinity Cache, where the ends of
+// a tile's rows cost more than its order gives, index ranges (us a call of
+// or_gauge_fixing, tiles and index ranges: 132^3 241 190, 160^3 385 372).
+template <bool DA, bool RENORM, bool TILES>
 __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   const Head h = HEAD_OF;
   const Geom& g = h.g;
@@ -707,7 +710,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   int s = blk * TB + threadIdx.x;
   int eo = DA ? 1 : h.flags & HEAD_EO, oe = eo ^ 1;
   bool act = s < g.n;
-  if (DA) {
+  if (DA && TILES) {
     TileOrigin o = tile_origin<GT_X, GT_Y, GT_Z>(blk, p.ntx, p.nty);
     TileSite t = tile_odd_site(threadIdx.x);
     int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
@@ -801,7 +804,13 @@ __device__ __forceinline__ TileSite tile_even_site(int e) {
 // What bounds it is the FP64 issue of 736 rotations for 512 sites on the
 // lattices the Infinity Cache holds, and the launch below 40^3.  An iteration in
 // us, two launches and one: 8^3 8.6 6.4, 16^3 8.6 6.9, 32^3 9.4 7.4, 48^3 12.1
-// 9.1, 64^3 18.5 14.1, 96^3 56 43, 160^3 361 288; 4^3 (16 odd sites) even.
+// 9.1, 64^3 18.5 14.1, 96^3 56 43, 160^3 361 276; 4^3 (16 odd sites) even.
+// WT: links stored through the L2.  Beyond the Infinity Cache they are not: a
+// tile's rows are 128-byte pieces, which end inside lines where lx is not a
+// multiple of 16, and memory then takes the lines whole, not piece by piece: us
+// an iteration, through and not, 140^3 254 223, 180x150x150 393 341, 160^3 288
+// 276; in the cache 64^3 13.9 15.4.
+template <bool WT>
 __global__ __launch_bounds__(GT_TB) void k_gfix_iter(const double* __restrict__ src,
                                                      double* __restrict__ dst,
                                                      double* __restrict__ Af, uint64_t h1_ly,
@@ -883,8 +892,8 @@ __global__ __launch_bounds__(GT_TB) void k_gfix_iter(const double* __restrict__ 
     st_higgs(Af, g, 1, (unsigned)s, adj_rot<false>(r, ao));
 #pragma unroll
     for (int mu = 0; mu < 3; ++mu) {
-      st_link(dst, g, mu, 1, (unsigned)s, normalized(m_nn(r, ux[mu])));
-      st_link(dst, g, mu, 0, (unsigned)sy[mu], normalized(m_nd(uy[mu], r)));
+      st_link<WT>(dst, g, mu, 1, (unsigned)s, normalized(m_nn(r, ux[mu])));
+      st_link<WT>(dst, g, mu, 0, (unsigned)sy[mu], normalized(m_nd(uy[mu], r)));
     }
   }
   block_sum_store<1, GT_TB / 64>(red, p.part, 0, blk);
@@ -943,7 +952,12 @@ void launch_gfix_begin(lceq_lattice* L, bool links) {
                      (double2*)L->Af, nu, na, L->obs);
 }
 
-static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
+// da's partial sums: one per tile or, of half steps over index ranges, per block
+static int gfix_sums(const Geom& g, bool one_launch) {
+  return one_launch || gfix_links_cached(g) ? lattice_tiles(g) : blocks_for(g.n);
+}
+
+static GfArgs gfix_args(lceq_lattice* L, bool one_launch, int guarded, int check, int iter) {
   const Geom& g = L->g;
   GfArgs a;
   a.guarded = guarded;
@@ -957,7 +971,7 @@ static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
   a.obs = L->obs;
   a.part = L->gf_part;
   a.part_old = L->gf_part;
-  a.ntiles = lattice_tiles(g);
+  a.ntiles = gfix_sums(g, one_launch);
   a.n = g.n;
   a.check = check;
   a.iter = (double)iter;
@@ -967,7 +981,7 @@ static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
 }
 
 void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, int iter) {
-  GfArgs a = gfix_args(L, guarded, check, iter);
+  GfArgs a = gfix_args(L, false, guarded, check, iter);
   prof_begin(L, KC_GFIX);
   prof_count(L, KC_GFIX);
   int nb = eo ? a.ntiles : blocks_for(L->g.n);
@@ -976,12 +990,13 @@ void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, in
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A, h.n, h.b, h.h, h.w, h.r,
                        a);
   };
+  const bool tiles = gfix_links_cached(L->g);
   if (!eo)
-    launch(k_gfix<false, false>);
+    launch(k_gfix<false, false, false>);
   else if (renorm)
-    launch(k_gfix<true, true>);
+    tiles ? launch(k_gfix<true, true, true>) : launch(k_gfix<true, true, false>);
   else
-    launch(k_gfix<true, false>);
+    tiles ? launch(k_gfix<true, false, true>) : launch(k_gfix<true, false, false>);
   prof_end(L, KC_GFIX);
 }
 
@@ -990,22 +1005,28 @@ void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, in
 static double* gfix_out(const lceq_lattice* L, int iter) { return iter & 1 ? L->Uf : L->spare; }
 
 void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
-  GfArgs a = gfix_args(L, 1, check, iter - 1);
+  GfArgs a = gfix_args(L, true, 1, check, iter - 1);
   // the partials too: a block may write its own while another still tests
   a.part = L->gf_part + (size_t)(iter & 1) * a.ntiles;
   a.part_old = L->gf_part + (size_t)((iter - 1) & 1) * a.ntiles;
   const Geom& g = L->g;
   prof_begin(L, KC_GFIX);
   prof_count(L, KC_GFIX);
-  hipLaunchKernelGGL(k_gfix_iter, dim3(a.ntiles), dim3(GT_TB), 0, L->stream,
-                     iter == 1 ? L->U : gfix_out(L, iter - 1), gfix_out(L, iter), L->Af,
-                     halves(g.h1, g.ly), halves(g.lz, g.npad), halves(a.ntiles, a.ntx),
-                     halves(a.nty, g.n), a);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.ntiles), dim3(GT_TB), 0, L->stream,
+                       iter == 1 ? L->U : gfix_out(L, iter - 1), gfix_out(L, iter), L->Af,
+                       halves(g.h1, g.ly), halves(g.lz, g.npad), halves(a.ntiles, a.ntx),
+                       halves(a.nty, g.n), a);
+  };
+  if (gfix_links_cached(g))
+    launch(k_gfix_iter<true>);
+  else
+    launch(k_gfix_iter<false>);
   prof_end(L, KC_GFIX);
 }
 
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch) {
-  int nt = lattice_tiles(L->g);
+  int nt = gfix_sums(L->g, one_launch);
   hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream,
                      L->gf_part + (one_launch ? (size_t)(iter & 1) * nt : 0), nt, (double)L->g.n,
                      guarded, (double)iter, L->limit_or, (double)L->max_iter, L->obs,

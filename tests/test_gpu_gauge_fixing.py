@@ -112,3 +112,10 @@ def test_tiles_equal_the_half_steps(shape, alpha, cap):
     G.or_gauge_fixing()
     H.or_gauge_fixing()
     assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
+
+
+@pytest.mark.parametrize("shape", [(128, 128, 100), (140, 140, 140)])
+def test_lattices_beyond_the_cache(shape):
+    """Two link arrays that the Infinity Cache does not hold (half steps in place),
+    and one that it does not (one launch, the links stored without write-through)."""
+    test_tiles_equal_the_half_steps(shape, 1.0, 9)
