@@ -79,8 +79,9 @@ int lceq_set_imode(lceq_lattice *L, int imode);
 /* launch shape of the link and Higgs updates (no counterpart in the
  * reference): threads (= sites) per block 64, 128, 256 or 512, XCD-aware
  * block order (1) or launch order (0).  Fields do not depend on the shape;
- * plaquette and Higgs sums are added in a shape-dependent order.  Default
- * 256, XCD order. */
+ * plaquette and Higgs sums are added in a shape-dependent order.  Launches of
+ * three link directions at once have a shape of their own.  Default 256, XCD
+ * order. */
 int lceq_set_shape(lceq_lattice *L, int threads_per_block, int xcd_order);
 int lceq_get_shape(lceq_lattice *L, int *threads_per_block, int *xcd_order);
 /* autotuner: time `trials` production sweeps (lceq_sweep schedule 0 with
@@ -232,7 +233,10 @@ int lceq_history(lceq_lattice *L, double *out, int n);
  * returns their summed duration and count.  One event pair brackets each run
  * of consecutive launches of the class (e.g. the 6 * n_or overrelaxation
  * launches of a schedule-0 sweep), so no event sits between them; the
- * duration of a run includes the dispatch gaps inside it. */
+ * duration of a run includes the dispatch gaps inside it.  Until then a sweep
+ * takes its launches per class over the whole lattice, also where it would take
+ * three directions in one or go by slabs (same fields); a landau_gauge
+ * iteration is one launch of LCEQ_KC_GFIX where it is one, otherwise two. */
 int lceq_profile_begin(lceq_lattice *L, int kernel_class, int max_launches);
 int lceq_profile_end(lceq_lattice *L, double *total_ms, int *launches);
 
