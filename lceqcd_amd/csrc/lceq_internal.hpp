@@ -25,7 +25,7 @@ enum {
   OBS_DELTA = 11,  // ahiggs1 Metropolis step (device-resident in sweeps)
   OBS_NACCH = 12,  // raw counts of the last link call
   OBS_NACC1 = 13,
-  OBS_GF_DONE = 14,  // landau_gauge convergence flag (1.0 = converged)
+  OBS_GF_DONE = 14,  // landau_gauge: iterations after which the loop ended, 0 before
   OBS_GF_CAPPED = 15,
   LCEQ_OBS_N = 16
 };
@@ -183,6 +183,15 @@ void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double*
 void launch_renorm(lceq_lattice* L, double* U);
 // per-block (unitarity deviation, non-finite count) of U and A into part[2 nb]
 void launch_check_fields(lceq_lattice* L, double* part);
+// Whether the gauge-fixing loop ended ahead of a launch: `done` is OBS_GF_DONE,
+// `testing` the iterations after which the launch itself tests the loop
+// condition (0: it does not).  The launch that finds the loop ended writes the
+// flag while other waves of it still read it; its own entry counts as none, so
+// that all waves take the same way whichever value they see, on to the test,
+// whose block sums need every wave of the block.
+__host__ __device__ inline bool gfix_ended(double done, double testing) {
+  return done != 0.0 && done != testing;
+}
 // One half-iteration of gauge fixing (eo = 1 forms da); check = 1 first tests
 // the loop condition for the `iter` iterations already complete (see k_gfix).
 void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check = 0, int iter = 0);

@@ -646,7 +646,7 @@ __device__ __forceinline__ bool gfix_stop(double da, double iter, double limit_o
   if (writer) {
     obs[OBS_DA] = da;
     obs[OBS_ITER] = iter;
-    if (stop) obs[OBS_GF_DONE] = 1.0;
+    if (stop) obs[OBS_GF_DONE] = iter;
     if (stop && !conv) obs[OBS_GF_CAPPED] = 1.0;
   }
   return stop;
@@ -732,7 +732,7 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   }
   // uniform over the grid; tested after the operand loads are issued, so that
   // its round trip overlaps theirs
-  if (p.guarded && p.obs[OBS_GF_DONE] != 0.0) return;
+  if (p.guarded && gfix_ended(p.obs[OBS_GF_DONE], p.check ? p.iter : 0.0)) return;
   if (p.check) {
     double da = gfix_da(p.part_old, p.ntiles, (double)p.n);
     if (gfix_stop(da, p.iter, p.limit_or, p.max_iter, p.obs, blk == 0 && threadIdx.x == 0))
@@ -843,7 +843,7 @@ __global__ __launch_bounds__(GT_TB) void k_gfix_iter(const double* __restrict__ 
     if (own) ae = ld_higgs(Af, g, 0, es);
   }
   // the loop condition, as in k_gfix
-  if (p.obs[OBS_GF_DONE] != 0.0) return;
+  if (gfix_ended(p.obs[OBS_GF_DONE], p.check ? p.iter : 0.0)) return;
   if (p.check) {
     double da = gfix_da(p.part_old, p.ntiles, (double)p.n);
     if (gfix_stop(da, p.iter, p.limit_or, p.max_iter, p.obs, blk == 0 && tid == 0)) return;

@@ -119,3 +119,11 @@ def test_lattices_beyond_the_cache(shape):
     """Two link arrays that the Infinity Cache does not hold (half steps in place),
     and one that it does not (one launch, the links stored without write-through)."""
     test_tiles_equal_the_half_steps(shape, 1.0, 9)
+
+
+@pytest.mark.parametrize("shape,limit", [((96, 96, 64), 1e-4), ((104, 104, 104), 1e-4)])
+def test_device_loop_of_many_tiles(shape, limit):
+    """1152 tiles, whose sum over block sums tests the loop condition inside the
+    next iteration's launch, and 2366 within the Infinity Cache, with a launch of
+    its own for the test; the loop ends inside a batch of iterations."""
+    test_device_loop_equals_host_loop(shape, 1.0, limit)
