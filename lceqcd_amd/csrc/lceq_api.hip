@@ -851,14 +851,8 @@ extern "C" int lceq_or_gauge_fixing(lceq_lattice* L, double* da1) {
 
 extern "C" int lceq_landau_gauge(lceq_lattice* L, double* da1, int* iter_or1) {
   NEEDL(L);
-  // One launch per iteration between two link arrays; two launches in place
-  // without memory for the second, and where the Infinity Cache holds (nearly)
-  // one array and a_f but not two.  us an iteration, in place and in one launch:
-  // 112^3 (303 MB with two arrays) 93 93, 128x128x100 (354) 110 115, 128^3 (453)
-  // 140 168, 132^3 (276 with one) 171 195, 140^3 (329) 230 222, 160^3 361 276
-  const int64_t one_array = 240 * (int64_t)L->g.npad, two_arrays = 432 * (int64_t)L->g.npad;
-  const bool one =
-      (two_arrays <= (int64_t)288 << 20 || one_array > (int64_t)280 << 20) && spare_links(L);
+  // two launches in place without memory for the second link array
+  const bool one = gfix_one_launch(L->g) && spare_links(L);
   launch_gfix_begin(L, !one);
   // Batches of guarded iterations; after convergence (or the cap) the
   // remaining launches of a batch return at once.  Inside a batch the loop

@@ -202,6 +202,22 @@ void launch_gfix_iter(lceq_lattice* L, int iter, int check);
 inline bool gfix_links_cached(const Geom& g) {
   return (192 + 48) * (int64_t)g.npad <= (int64_t)256 << 20;
 }
+// Whether a landau_gauge iteration is one launch over tiles between two link
+// arrays, or two launches in place.  In place where the Infinity Cache holds
+// (nearly) one array and a_f but not two; us an iteration, in place and in one
+// launch: 112^3 (303 MB with two arrays) 93 93, 128x128x100 (354) 110 115, 128^3
+// (453) 140 168, 132^3 (276 with one) 171 195, 140^3 (329) 230 222, 160^3 361 276.
+// And where the tiles are mostly empty, whose blocks cost as much as full ones:
+// up to an eighth filled (2x16x16 7.1 9.4, 2x128x64 7.8 8.5, 2x512x64 12.7 17.5,
+// 4x4x2048 9.0 10.6; a quarter 4x64x64 7.8 6.8, 4x128x128 9.3 9.1), and up to half
+// beyond two blocks per CU (4x128x256 12.4 15.8, 6x256x128 15.2 16.4, 6x256x256
+// 27.0 30.2; half 8x256x256 33.9 31.9).
+inline bool gfix_one_launch(const Geom& g) {
+  const int64_t one_array = 240 * (int64_t)g.npad, two_arrays = 432 * (int64_t)g.npad;
+  if (two_arrays > (int64_t)288 << 20 && one_array <= (int64_t)280 << 20) return false;
+  const int64_t tiles = lattice_tiles(g), room = 512 * tiles, sites = 2 * (int64_t)g.n;
+  return 8 * sites > room && (tiles <= 512 || 2 * sites >= room);
+}
 // one_launch: the iterations were launch_gfix_iter's
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch);
 // a_f = a, with `links` u_f = u, and the loop's observables as before its first

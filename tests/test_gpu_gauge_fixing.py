@@ -127,3 +127,25 @@ def test_device_loop_of_many_tiles(shape, limit):
     next iteration's launch, and 2366 within the Infinity Cache, with a launch of
     its own for the test; the loop ends inside a batch of iterations."""
     test_device_loop_equals_host_loop(shape, 1.0, limit)
+
+
+@pytest.mark.parametrize("shape,launches", [((2, 16, 16), 2), ((4, 4, 4), 2), ((4, 128, 256), 2),
+                                            ((6, 256, 128), 2), ((6, 4, 8), 1), ((4, 32, 64), 1),
+                                            ((8, 256, 128), 1), ((16, 16, 16), 1)])
+def test_mostly_empty_tiles_take_the_half_steps(shape, launches):
+    """An iteration is two launches in place where one launch's tiles would hold
+    few sites each, and one otherwise; the same fields as the host loop."""
+    import lceqcd_amd
+    print("landau_gauge launches", shape, flush=True)
+    u, a = _thermalised(shape, 47)
+    G = lceqcd_amd.Lattice(*shape)
+    G.put_links(u)
+    G.put_higgs(a)
+    G.set_gauge_fixing(1.7, 1.0, 1e-300, 8)
+    G.profile_begin(lceqcd_amd.KC_GFIX, 100)
+    with pytest.raises(lceqcd_amd.LceqError, match="max_iter"):
+        G.landau_gauge()
+    assert G.profile_end()[1] == 8 * launches
+    H, _, _ = _host_loop(shape, u, a, 1.7, 1.0, 1e-300, 8)
+    assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
+    assert np.array_equal(G.get_higgs_fixed(), H.get_higgs_fixed())
