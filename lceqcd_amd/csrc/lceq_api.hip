@@ -103,7 +103,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   alloc(&L->Af, 6 * np);
   alloc(&L->Vst, 24 * np);
   alloc(&L->F, 3 * np);
-  alloc(&L->gf_part, 2 * (size_t)lattice_tiles(g));
+  alloc(&L->gf_part, 2 * (size_t)lattice_tiles(g) + (gfix_site_sums(g) ? (size_t)g.n : 0));
   alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
 
   alloc(&L->obs, LCEQ_OBS_N);

@@ -45,7 +45,9 @@ struct lceq_lattice {
   // holds nothing.  Lattices whose link sweeps use it have it from creation on,
   // so that a sweep allocates nothing, the others from their first landau_gauge.
   double* spare;
-  double* gf_part;   // da partials of two iterations [2][lattice_tiles]
+  // da partials of two iterations [2][lattice_tiles], then, where gfix_site_sums,
+  // one da per odd site [n]
+  double* gf_part;
   double *partials;  // [LCEQ_NSLOT][LCEQ_NQ][pstride]
   int pstride;       // >= number of 64-site blocks (the smallest launch shape)
   double *obs;       // [LCEQ_OBS_N]
@@ -217,6 +219,21 @@ inline bool gfix_one_launch(const Geom& g) {
   if (two_arrays > (int64_t)288 << 20 && one_array <= (int64_t)280 << 20) return false;
   const int64_t tiles = lattice_tiles(g), room = 512 * tiles, sites = 2 * (int64_t)g.n;
   return 8 * sites > room && (tiles <= 512 || 2 * sites >= room);
+}
+// The order of da's sum, one for each lattice, so that landau_gauge and a host
+// loop over or_gauge_fixing form the same da and stop after the same iteration: by
+// tiles where landau_gauge's iterations are launches over tiles, otherwise by the
+// half step's blocks of site indices
+inline bool gfix_tile_order(const Geom& g) { return gfix_one_launch(g); }
+// The odd half step of an order by tiles runs over tiles itself, or over site
+// indices where cut-off tiles cost more (and beyond the Infinity Cache), with one
+// da stored per site and added by tiles in a launch of its own.  us a call of
+// or_gauge_fixing, by tiles and by indices (without that launch, 3 us): 34x64x64
+// (384 tiles) 27.5 25.5, 50x64x64 (512) 31.4 28.0, 66x64x64 (640) 39.6 34.5, 100^3
+// 88.4 76.1, 18x256x256 112.6 88.0; whole tiles 64^3 32.1 31.2.
+inline bool gfix_site_sums(const Geom& g) {
+  const bool whole = g.lx % GT_X == 0 && g.ly % GT_Y == 0 && g.lz % GT_Z == 0;
+  return gfix_tile_order(g) && !(gfix_links_cached(g) && (whole || lattice_tiles(g) <= 512));
 }
 // one_launch: the iterations were launch_gfix_iter's
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch);

@@ -595,7 +595,8 @@ struct GfArgs {
   int lx, ly, lz, ntx, nty;  // extents and tiles (k_gfix<DA>)
   double lambda, alpha;
   double* obs;  // OBS_GF_DONE read when guarded; the convergence test writes
-  double* part;            // da partials this launch writes, one per tile
+  double* part;            // da partials this launch writes, one per tile or block
+  double* sites;           // or da itself, one per site (DA_SITES)
   const double* part_old;  // those of the iteration before (check)
   int ntiles, n;
   // convergence test of the previous iteration at the start of this launch
@@ -694,23 +695,22 @@ __device__ __forceinline__ su2 gfix_rotation(const su2& w, double lambda) {
 // first repeats the convergence test of the previous iteration (the same
 // sum in the same order, so all blocks agree) and the launch returns when
 // the loop has ended; the operand loads are issued before the test.
-// DA (eo = 1): da's partial sums, one per tile, the blocks then being tiles; the
-// other half's blocks are index ranges.  DA and RENORM are template arguments:
-// without a branch around each pair, the six normalisations' chains of
-// dependent operations run side by side.
-// TILES: the blocks of DA are tiles; beyond the Infinity Cache, where the ends of
-// a tile's rows cost more than its order gives, index ranges (us a call of
-// or_gauge_fixing, tiles and index ranges: 132^3 241 190, 160^3 385 372).
-template <bool DA, bool RENORM, bool TILES>
+// DA (eo = 1): da's partial sums, one per block, the blocks being tiles or index
+// ranges, or da per site (gfix_site_sums says which); the other half's blocks are
+// index ranges.  DA and RENORM are template arguments: without a branch around
+// each pair, the six normalisations' chains of dependent operations run side by
+// side.
+enum { DA_NONE, DA_TILES, DA_BLOCKS, DA_SITES };
+template <int DA, bool RENORM>
 __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   const Head h = HEAD_OF;
   const Geom& g = h.g;
   double *Uf = h.U, *Af = h.A;
   int blk = xcd_block(h.nb);
   int s = blk * TB + threadIdx.x;
-  int eo = DA ? 1 : h.flags & HEAD_EO, oe = eo ^ 1;
+  int eo = DA != DA_NONE ? 1 : h.flags & HEAD_EO, oe = eo ^ 1;
   bool act = s < g.n;
-  if (DA && TILES) {
+  if (DA == DA_TILES) {
     TileOrigin o = tile_origin<GT_X, GT_Y, GT_Z>(blk, p.ntx, p.nty);
     TileSite t = tile_odd_site(threadIdx.x);
     int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
@@ -741,7 +741,8 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
   double red[1] = {0.0};
   if (act) {
     su2 s1 = gfix_sum(p.alpha, ux), s2 = gfix_sum(p.alpha, uy), w = gfix_w(s1, s2);
-    if (DA) red[0] = gfix_site_da(s1, s2, w);
+    if (DA != DA_NONE) red[0] = gfix_site_da(s1, s2, w);
+    if (DA == DA_SITES) p.sites[s] = red[0];
     su2 o = gfix_rotation(w, p.lambda);
     st_higgs(Af, g, eo, s, adj_rot<false>(o, af));  // g X(a_f) g^+, :243-252
 #pragma unroll
@@ -756,7 +757,20 @@ __global__ __launch_bounds__(256) void k_gfix(HEAD_PARAMS, GfArgs p) {
       st_link(Uf, g, mu, oe, sy[mu], ny);
     }
   }
-  if (DA) block_sum_store<1>(red, p.part, 0, blk);
+  if (DA == DA_TILES || DA == DA_BLOCKS) block_sum_store<1>(red, p.part, 0, blk);
+}
+
+// da of the odd sites, added by tiles as k_gfix<DA_TILES> and k_gfix_iter do
+__global__ __launch_bounds__(256) void k_gfix_site_sums(const double* __restrict__ sites, Geom g,
+                                                        int ntx, int nty,
+                                                        double* __restrict__ part) {
+  const int blk = blockIdx.x;
+  const TileOrigin o = tile_origin<GT_X, GT_Y, GT_Z>(blk, ntx, nty);
+  const TileSite t = tile_odd_site(threadIdx.x);
+  const int x = o.x + t.x, y = o.y + t.y, z = o.z + t.z;
+  double red[1] = {0.0};
+  if (x < g.lx && y < g.ly && z < g.lz) red[0] = sites[(x >> 1) + g.h1 * y + g.h2 * z];
+  block_sum_store<1>(red, part, 0, blk);
 }
 
 // Slot of the even site at tile coordinates (x, y, z), which is in the tile
@@ -952,12 +966,12 @@ void launch_gfix_begin(lceq_lattice* L, bool links) {
                      (double2*)L->Af, nu, na, L->obs);
 }
 
-// da's partial sums: one per tile or, of half steps over index ranges, per block
-static int gfix_sums(const Geom& g, bool one_launch) {
-  return one_launch || gfix_links_cached(g) ? lattice_tiles(g) : blocks_for(g.n);
+// da's partial sums: one per tile or per block of site indices
+static int gfix_sums(const Geom& g) {
+  return gfix_tile_order(g) ? lattice_tiles(g) : blocks_for(g.n);
 }
 
-static GfArgs gfix_args(lceq_lattice* L, bool one_launch, int guarded, int check, int iter) {
+static GfArgs gfix_args(lceq_lattice* L, int guarded, int check, int iter) {
   const Geom& g = L->g;
   GfArgs a;
   a.guarded = guarded;
@@ -971,7 +985,8 @@ static GfArgs gfix_args(lceq_lattice* L, bool one_launch, int guarded, int check
   a.obs = L->obs;
   a.part = L->gf_part;
   a.part_old = L->gf_part;
-  a.ntiles = gfix_sums(g, one_launch);
+  a.sites = L->gf_part + 2 * (size_t)lattice_tiles(g);
+  a.ntiles = gfix_sums(g);
   a.n = g.n;
   a.check = check;
   a.iter = (double)iter;
@@ -981,23 +996,31 @@ static GfArgs gfix_args(lceq_lattice* L, bool one_launch, int guarded, int check
 }
 
 void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, int iter) {
-  GfArgs a = gfix_args(L, false, guarded, check, iter);
+  GfArgs a = gfix_args(L, guarded, check, iter);
   prof_begin(L, KC_GFIX);
   prof_count(L, KC_GFIX);
-  int nb = eo ? a.ntiles : blocks_for(L->g.n);
+  const Geom& g = L->g;
+  const bool tiles = gfix_tile_order(g), sites = gfix_site_sums(g);
+  int nb = eo && tiles && !sites ? a.ntiles : blocks_for(g.n);
   HeadArgs h = head_args(L, L->Uf, L->Af, nb, eo);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(TB), 0, L->stream, h.U, h.A, h.n, h.b, h.h, h.w, h.r,
                        a);
   };
-  const bool tiles = gfix_links_cached(L->g);
   if (!eo)
-    launch(k_gfix<false, false, false>);
-  else if (renorm)
-    tiles ? launch(k_gfix<true, true, true>) : launch(k_gfix<true, true, false>);
+    launch(k_gfix<DA_NONE, false>);
+  else if (sites)
+    renorm ? launch(k_gfix<DA_SITES, true>) : launch(k_gfix<DA_SITES, false>);
+  else if (tiles)
+    renorm ? launch(k_gfix<DA_TILES, true>) : launch(k_gfix<DA_TILES, false>);
   else
-    tiles ? launch(k_gfix<true, false, true>) : launch(k_gfix<true, false, false>);
+    renorm ? launch(k_gfix<DA_BLOCKS, true>) : launch(k_gfix<DA_BLOCKS, false>);
   prof_end(L, KC_GFIX);
+  // after the loop's end the sites hold the last iteration's da, whose sums these
+  // are again
+  if (eo && sites)
+    hipLaunchKernelGGL(k_gfix_site_sums, dim3(a.ntiles), dim3(TB), 0, L->stream, a.sites, g, a.ntx,
+                       a.nty, a.part);
 }
 
 // The link array iteration `iter` (from 1) of the one-launch loop writes: u_f
@@ -1005,7 +1028,7 @@ void launch_gfix(lceq_lattice* L, int eo, int renorm, int guarded, int check, in
 static double* gfix_out(const lceq_lattice* L, int iter) { return iter & 1 ? L->Uf : L->spare; }
 
 void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
-  GfArgs a = gfix_args(L, true, 1, check, iter - 1);
+  GfArgs a = gfix_args(L, 1, check, iter - 1);
   // the partials too: a block may write its own while another still tests
   a.part = L->gf_part + (size_t)(iter & 1) * a.ntiles;
   a.part_old = L->gf_part + (size_t)((iter - 1) & 1) * a.ntiles;
@@ -1026,7 +1049,7 @@ void launch_gfix_iter(lceq_lattice* L, int iter, int check) {
 }
 
 void launch_gfix_finalize(lceq_lattice* L, int guarded, int iter, bool to_host, bool one_launch) {
-  int nt = gfix_sums(L->g, one_launch);
+  int nt = gfix_sums(L->g);
   hipLaunchKernelGGL(k_gfix_finalize, dim3(1), dim3(TB), 0, L->stream,
                      L->gf_part + (one_launch ? (size_t)(iter & 1) * nt : 0), nt, (double)L->g.n,
                      guarded, (double)iter, L->limit_or, (double)L->max_iter, L->obs,

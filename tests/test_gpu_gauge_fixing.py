@@ -149,3 +149,14 @@ def test_mostly_empty_tiles_take_the_half_steps(shape, launches):
     H, _, _ = _host_loop(shape, u, a, 1.7, 1.0, 1e-300, 8)
     assert np.array_equal(G.get_links_fixed(), H.get_links_fixed())
     assert np.array_equal(G.get_higgs_fixed(), H.get_higgs_fixed())
+
+
+@pytest.mark.parametrize("shape,limit", [((140, 140, 140), 1e-3), ((132, 132, 132), 1e-3),
+                                         ((18, 128, 128), 1e-4), ((66, 66, 66), 1e-4),
+                                         ((4, 256, 128), 1e-4), ((50, 64, 64), 1e-4)])
+def test_one_da_for_both_loops(shape, limit):
+    """The device loop and the host loop add da in the same order on every lattice:
+    beyond the Infinity Cache in one launch per iteration and in place, and
+    within it on tiles that are cut off (above and below 512 of them) and mostly
+    empty."""
+    test_device_loop_equals_host_loop(shape, 1.0, limit)
