@@ -205,20 +205,33 @@ inline bool gfix_links_cached(const Geom& g) {
   return (192 + 48) * (int64_t)g.npad <= (int64_t)256 << 20;
 }
 // Whether a landau_gauge iteration is one launch over tiles between two link
-// arrays, or two launches in place.  In place where the Infinity Cache holds
-// (nearly) one array and a_f but not two; us an iteration, in place and in one
-// launch: 112^3 (303 MB with two arrays) 93 93, 128x128x100 (354) 110 115, 128^3
-// (453) 140 168, 132^3 (276 with one) 171 195, 140^3 (329) 230 222, 160^3 361 276.
-// And where the tiles are mostly empty, whose blocks cost as much as full ones:
-// up to an eighth filled (2x16x16 7.1 9.4, 2x128x64 7.8 8.5, 2x512x64 12.7 17.5,
-// 4x4x2048 9.0 10.6; a quarter 4x64x64 7.8 6.8, 4x128x128 9.3 9.1), and up to half
-// beyond two blocks per CU (4x128x256 12.4 15.8, 6x256x128 15.2 16.4, 6x256x256
-// 27.0 30.2; half 8x256x256 33.9 31.9).
+// arrays, or two launches in place.  In place:
+// - Where the tiles are mostly empty, whose blocks cost as much as full ones, up to
+//   an eighth filled (us an iteration in place and in one launch: 2x16x16 7.1 9.4,
+//   2x128x64 7.8 8.5, 4x4x2048 9.0 10.6; a quarter 4x64x64 7.8 6.8, 4x128x128 9.3
+//   9.1), and up to half beyond two blocks per CU (4x128x256 12.4 15.8, 6x256x128
+//   15.2 16.4, 6x256x256 27.0 30.2; half 8x256x256 33.9 31.9).
+// - Where the Infinity Cache holds (nearly) one array and a_f but not two.  A row of
+//   a tile is 128 bytes; where rows end inside lines (lx no multiple of 16) the
+//   stores of neighbouring tiles meet there, and two arrays cost more well before
+//   they fill the cache (MiB of two arrays): 102^3 (218) 76 63, 66x128x128 (222) 77
+//   68, 104^3 (231, half lines) 78 56, 34x256x128 (229) 74 70-111, 18x256x256 (243)
+//   77 73-125, 108^3 (259) 82 110, 110^3 (274) 92 122; whole rows 96x96x128 (243) 79
+//   53-74, 128x128x80 (270) 84 82, 112^3 (289) 91 91, 128^3 (453) 140 168.
+// - Beyond it, until one array is out of it as well: 132^3 (497) 171 195, 144x130x130
+//   (501) 183 187, whole rows from there on: 128x142x142 (531) 180 180, 144^3 (615)
+//   236 196, 160^3 361 276; others much later: 136^3 (518) 185 196, 140^3 (565) 197
+//   222, 146^3 (641) 264 273, 148^3 (667) 277 271, 150^3 (695) 298 283, 170^3 (1012)
+//   454 405; and where a lone site ends rows of few tiles, later still: 50x256x224
+//   (590) 220 298, 50x512x512 (2700) 1178 1351, 34x512x400 (1434) 640 640.
 inline bool gfix_one_launch(const Geom& g) {
-  const int64_t one_array = 240 * (int64_t)g.npad, two_arrays = 432 * (int64_t)g.npad;
-  if (two_arrays > (int64_t)288 << 20 && one_array <= (int64_t)280 << 20) return false;
   const int64_t tiles = lattice_tiles(g), room = 512 * tiles, sites = 2 * (int64_t)g.n;
-  return 8 * sites > room && (tiles <= 512 || 2 * sites >= room);
+  if (8 * sites <= room || (tiles > 512 && 2 * sites < room)) return false;
+  const int64_t one_array = 240 * (int64_t)g.npad >> 20, two_arrays = 432 * (int64_t)g.npad >> 20;
+  const int end = g.lx % GT_X;  // sites in the last tile of a row, 0: all
+  if (two_arrays < (end == 0 ? 288 : end == 8 ? 232 : 224)) return true;
+  if (one_array < 280) return false;
+  return end == 0 || (two_arrays >= 650 && !(end == 2 && g.lx < 64));
 }
 // The order of da's sum, one for each lattice, so that landau_gauge and a host
 // loop over or_gauge_fixing form the same da and stop after the same iteration: by

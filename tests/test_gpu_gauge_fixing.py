@@ -160,3 +160,14 @@ def test_one_da_for_both_loops(shape, limit):
     within it on tiles that are cut off (above and below 512 of them) and mostly
     empty."""
     test_device_loop_equals_host_loop(shape, 1.0, limit)
+
+
+@pytest.mark.parametrize("shape,launches", [((96, 96, 96), 1), ((104, 104, 104), 1),
+                                            ((108, 108, 108), 2), ((34, 256, 128), 2),
+                                            ((128, 128, 100), 2), ((140, 140, 140), 2),
+                                            ((50, 256, 400), 2), ((160, 160, 112), 1),
+                                            ((148, 148, 148), 1)])
+def test_launches_where_the_cache_ends(shape, launches):
+    """Rows of whole tiles and others on either side of the Infinity Cache, with
+    one and with two launches an iteration."""
+    test_mostly_empty_tiles_take_the_half_steps(shape, launches)
