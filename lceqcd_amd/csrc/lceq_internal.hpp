@@ -159,8 +159,33 @@ void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int reno
 // A link sweep without partial sums (Philox), three directions of parity eo in
 // one launch: passes pass .. pass + 2, from the links `src` (of parity eo) and
 // `other` (of the other one) to `dst`, another array than `src`.  link3_tiles:
-// its blocks on lattices where it is the faster way, otherwise 0
-int link3_tiles(const Geom& g);
+// its blocks on lattices where it is the faster way, otherwise 0.
+// The launch runs as long as its fullest CU: a CU holds three blocks, and half
+// as many link updates again as the launches per direction have.  Those cost a
+// launch each, so that up to two blocks per CU are the faster way whatever the
+// tiles hold, and many rounds of whole tiles save their passes over memory; in
+// between, and where tiles are cut off, the extra updates cost more.  us per
+// production sweep of n_or = 4 (one of the five link sweeps is a measured one),
+// launches per direction and this one:
+//   16^3 (16 tiles) 114-127 89, 32^3 (128) 114-128 91, 44^3 (363) 129 123,
+//   64x64x32 (512) 132 118, 50^3 (676) 131 162, 64^3 (1024) 159 188,
+//   64x64x80 (1280) 233 239, 80x80x64 (1600) 334 304, 96^3 (3456) 608 572,
+//   112x112x96 (4704) 820 757; tiles cut off: 72x72x96 (2160) 371 386,
+//   100^3 (4375) 684 758
+// The second array counts against the Infinity Cache: 128x128x72 (0.25 GB of
+// fields and second array) 786 755, 128x128x80 (0.28) 864 869, 128^3 (0.45)
+// 1362 1643.
+// A tile of two columns stores lone 16-byte pieces; where they are half the tiles
+// or more, up to one block per CU: 18x34x50 (234) 136 102, 18x32x64 (256) 127 101,
+// 18x34x66 (306) 137 138, 18x48x64 (384) 128 133, 18x64x64 (512) 122 131.
+constexpr int L3_X = 16, L3_Y = 4, L3_Z = 4;
+inline int link3_tiles(const Geom& g) {
+  const int nt = tiles_along(g.lx, L3_X) * tiles_along(g.ly, L3_Y) * tiles_along(g.lz, L3_Z);
+  const bool whole = g.lx % L3_X == 0 && g.ly % L3_Y == 0 && g.lz % L3_Z == 0;
+  const bool cached = (240 + 192) * (int64_t)g.npad <= (int64_t)256 << 20;
+  const bool narrow = g.lx % L3_X == 2 && g.lx < 2 * L3_X;
+  return cached && (nt <= (narrow ? 256 : 512) || (nt >= 1600 && whole)) ? nt : 0;
+}
 void launch_link3(lceq_lattice* L, int kp, int eo, int renorm_on_write, const double* src,
                   const double* other, double* dst, uint64_t pass);
 // One-block reduction of the partial sums into the observables: link_kind

@@ -23,7 +23,6 @@ namespace lceq {
 namespace {
 
 constexpr int L3_TB = 256;
-constexpr int L3_X = 16, L3_Y = 4, L3_Z = 4;
 constexpr int L3_PASS2 = 128, L3_PASS1 = 184, L3_PASS0 = 239;  // sites of the passes
 
 struct TileSite {
@@ -194,28 +193,6 @@ __global__ __launch_bounds__(L3_TB) void k_link3(const double* __restrict__ src,
 }
 
 }  // namespace
-
-// The launch runs as long as its fullest CU: a CU holds three blocks, and half
-// as many link updates again as the launches per direction have.  Those cost a
-// launch each, so that up to two blocks per CU are the faster way whatever the
-// tiles hold, and many rounds of whole tiles save their passes over memory; in
-// between, and where tiles are cut off, the extra updates cost more.  us per
-// production sweep of n_or = 4 (one of the five link sweeps is a measured one),
-// launches per direction and this one:
-//   16^3 (16 tiles) 114-127 89, 32^3 (128) 114-128 91, 44^3 (363) 129 123,
-//   64x64x32 (512) 132 118, 50^3 (676) 131 162, 64^3 (1024) 159 188,
-//   64x64x80 (1280) 233 239, 80x80x64 (1600) 334 304, 96^3 (3456) 608 572,
-//   112x112x96 (4704) 820 757; tiles cut off: 72x72x96 (2160) 371 386,
-//   100^3 (4375) 684 758
-// The second array counts against the Infinity Cache: 128x128x72 (0.25 GB of
-// fields and second array) 786 755, 128x128x80 (0.28) 864 869, 128^3 (0.45)
-// 1362 1643.
-int link3_tiles(const Geom& g) {
-  const int nt = tiles_along(g.lx, L3_X) * tiles_along(g.ly, L3_Y) * tiles_along(g.lz, L3_Z);
-  const bool whole = g.lx % L3_X == 0 && g.ly % L3_Y == 0 && g.lz % L3_Z == 0;
-  const bool cached = (240 + 192) * (int64_t)g.npad <= (int64_t)256 << 20;
-  return cached && (nt <= 512 || (nt >= 1600 && whole)) ? nt : 0;
-}
 
 void launch_link3(lceq_lattice* L, int kp, int eo, int renorm_on_write, const double* src,
                   const double* other, double* dst, uint64_t pass) {
