@@ -235,8 +235,8 @@ int lceq_history(lceq_lattice *L, double *out, int n);
  * launches of a schedule-0 sweep), so no event sits between them; the
  * duration of a run includes the dispatch gaps inside it.  Until then a sweep
  * takes its launches per class over the whole lattice, also where it would take
- * three directions in one or go by slabs (same fields); a landau_gauge
- * iteration is one launch of LCEQ_KC_GFIX where it is one, otherwise two. */
+ * three directions in one, go by slabs or carry renorm in a Higgs launch (same
+ * fields); a landau_gauge iteration is one launch of LCEQ_KC_GFIX where it is one, otherwise two. */
 int lceq_profile_begin(lceq_lattice *L, int kernel_class, int max_launches);
 int lceq_profile_end(lceq_lattice *L, double *total_ms, int *launches);
 

@@ -1153,7 +1153,7 @@ extern "C" int lceq_sweep(lceq_lattice* L, int schedule, int nsweep, int n_or, d
       // ahiggs2's averages are ahiggs3's a launch later, so it sums nothing.
       // renorm is carried by the next sweep's first launch, which loads every
       // link once (64^3: a renorm launch 12.2 us, carried 1.6)
-      const bool carry = L->rng_mode == LCEQ_RNG_PHILOX;
+      const bool carry = carries_renorm(L);
       if ((rc = higgs_sweep(L, 2, 0, 0, carry && it > 0))) return rc;
       if ((rc = higgs_sweep(L, 3, measflag, measflag))) return rc;
       if ((rc = link_sweep(L, 1, measflag, 0, measflag))) return rc;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/lceq.h"
 #include "lceq_device.hpp"
 
 // number of per-block partial quantities a reduction slot holds
@@ -208,6 +209,11 @@ void launch_higgs(lceq_lattice* L, int kind, int eo, int measflag, const double*
                   uint64_t pass, int reduce, bool renorm = false,
                   const SiteRange* range = nullptr);
 void launch_renorm(lceq_lattice* L, double* U);
+// Whether a reference sweep's renorm goes into the next sweep's first launch;
+// not while a kernel class is timed, whose launches are then its own alone
+inline bool carries_renorm(const lceq_lattice* L) {
+  return L->rng_mode == LCEQ_RNG_PHILOX && L->prof_class == KC_NONE;
+}
 // per-block (unitarity deviation, non-finite count) of U and A into part[2 nb]
 void launch_check_fields(lceq_lattice* L, double* part);
 // Whether the gauge-fixing loop ended ahead of a launch: `done` is OBS_GF_DONE,

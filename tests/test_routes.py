@@ -48,3 +48,13 @@ def test_three_directions_in_one_launch(rule, shape, tiles):
     """Link sweeps of lattices whose tiles are mostly two columns wide take the
     launches per direction beyond 256 tiles."""
     assert rule("link3_tiles(g)", shape) == tiles
+
+
+@pytest.mark.parametrize("state,carried", [("", 1), ("L.prof_class = KC_HIGGS;", 0),
+                                           ("L.prof_class = KC_GFIX;", 0),
+                                           ("L.rng_mode = LCEQ_RNG_FED;", 0)])
+def test_renorm_within_a_higgs_launch(rule, state, carried):
+    """Timed Higgs launches do not do renorm's work (nor do fed ones)."""
+    made = "[] { lceq_lattice L{}; L.rng_mode = LCEQ_RNG_PHILOX; %s return L; }" % state
+    assert rule("([&] { lceq_lattice L = %s(); return carries_renorm(&L); })()" % made,
+                (4, 4, 4)) == carried
