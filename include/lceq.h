@@ -85,7 +85,9 @@ int lceq_set_imode(lceq_lattice *L, int imode);
 int lceq_set_shape(lceq_lattice *L, int threads_per_block, int xcd_order);
 int lceq_get_shape(lceq_lattice *L, int *threads_per_block, int *xcd_order);
 /* autotuner: time `trials` production sweeps (lceq_sweep schedule 0 with
- * n_or) at every shape and keep the fastest; fields, observables, the pass
+ * n_or) at every shape and keep the fastest, with launches per direction, which
+ * are what a shape applies to, also on lattices whose sweeps take three
+ * directions in one; fields, observables, the pass
  * counter and the history are restored.  ms (or NULL) receives 8 times per
  * sweep, shapes (64,128,256,512) x (launch order, XCD order).  Philox only. */
 int lceq_autotune(lceq_lattice *L, int n_or, int trials, double *ms);
@@ -100,8 +102,8 @@ int lceq_autotune(lceq_lattice *L, int n_or, int trials, double *ms);
 int lceq_set_site_order(lceq_lattice *L, int strip_rows);
 int lceq_get_site_order(lceq_lattice *L, int *strip_rows);
 /* time `trials` production sweeps with site orders 0, 4, 8, 16 (those that
- * divide ly) at the current launch shape, keep the fastest; fields,
- * observables, the pass counter and the history are restored.  ms (or NULL)
+ * divide ly) at the current launch shape, with launches per direction as
+ * lceq_autotune, keep the fastest; fields, observables, the pass counter and the history are restored.  ms (or NULL)
  * receives 4 times per sweep (-1 where an order does not fit). */
 int lceq_autotune_site_order(lceq_lattice *L, int n_or, int trials, double *ms);
 /* Measurement aid with no counterpart in the reference: a plain device copy

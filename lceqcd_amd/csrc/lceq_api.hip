@@ -344,6 +344,7 @@ extern "C" int lceq_autotune(lceq_lattice* L, int n_or, int trials, double* ms) 
   const int shapes[4] = {64, 128, 256, 512};
   double best = 1e300, delta = o[OBS_DELTA];
   int best_tb = L->tb, best_x = L->xcd, rc = LCEQ_OK;
+  L->tuning = 1;
   for (int i = 0; i < 8 && rc == LCEQ_OK; ++i) {
     L->tb = shapes[i / 2];
     L->xcd = i % 2;
@@ -366,6 +367,7 @@ extern "C" int lceq_autotune(lceq_lattice* L, int n_or, int trials, double* ms) 
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  L->tuning = 0;
   L->tb = best_tb;
   L->xcd = best_x;
   L->pass = pass0;
@@ -426,6 +428,7 @@ extern "C" int lceq_autotune_site_order(lceq_lattice* L, int n_or, int trials, d
   const int orders[4] = {0, 4, 8, 16};
   double best = 1e300, delta = o[OBS_DELTA];
   int best_sy = L->strip, rc = LCEQ_OK;
+  L->tuning = 1;
   for (int i = 0; i < 4 && rc == LCEQ_OK; ++i) {
     int sy = orders[i];
     if (sy && (L->g.ly % sy || (int64_t)L->g.ly * L->g.lz >= ((int64_t)1 << 22))) {
@@ -451,6 +454,7 @@ extern "C" int lceq_autotune_site_order(lceq_lattice* L, int n_or, int trials, d
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  L->tuning = 0;
   L->strip = best_sy;
   L->pass = pass0;
   L->hist_rows = rows0;
@@ -679,11 +683,10 @@ extern "C" int lceq_heat_kpi(lceq_lattice* L, int n, const double* b, double* v,
 // in slots 0-5 for launch_finalize
 //
 // A Philox sweep without sums, all but one of a production sweep's, runs the
-// three directions of a parity in one launch (launch_link3) where link3_tiles
+// three directions of a parity in one launch (launch_link3) where takes_link3
 // says so, from one link array to another; the arrays then change places.
 int link_sweep(lceq_lattice* L, int kp, int measflag, int renorm_on_write, int reduce) {
-  if (!reduce && !measflag && L->rng_mode == LCEQ_RNG_PHILOX && !L->prof_class &&
-      link3_tiles(L->g) && L->spare) {
+  if (!reduce && !measflag && takes_link3(L)) {
     for (int eo = 0; eo < 2; ++eo) {
       uint64_t pass = L->pass;
       L->pass += 3;

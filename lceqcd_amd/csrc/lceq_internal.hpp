@@ -75,6 +75,7 @@ struct lceq_lattice {
   // site order of those launches: strips of `strip` y rows (0: by the
   // lattice's shape, strip_rows)
   int strip;
+  int tuning;  // an autotuner times these: sweeps take launches that they apply to
   uint64_t seed, pass;
   // timing of one kernel class (bench instrumentation): one event pair per
   // run of consecutive launches of that class, launches counted inside runs
@@ -186,6 +187,13 @@ inline int link3_tiles(const Geom& g) {
   const bool cached = (240 + 192) * (int64_t)g.npad <= (int64_t)256 << 20;
   const bool narrow = g.lx % L3_X == 2 && g.lx < 2 * L3_X;
   return cached && (nt <= (narrow ? 256 : 512) || (nt >= 1600 && whole)) ? nt : 0;
+}
+// whether a link sweep without sums takes them: not while a kernel class is timed
+// or a launch shape or site order is tuned, which are those of the launches per
+// direction (measured and fed sweeps, agauge, link_or)
+inline bool takes_link3(const lceq_lattice* L) {
+  return L->rng_mode == LCEQ_RNG_PHILOX && L->prof_class == KC_NONE && !L->tuning && L->spare &&
+         link3_tiles(L->g);
 }
 void launch_link3(lceq_lattice* L, int kp, int eo, int renorm_on_write, const double* src,
                   const double* other, double* dst, uint64_t pass);

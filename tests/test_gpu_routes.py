@@ -1,0 +1,82 @@
+"""The kernels that calls launch, from a device trace (torch.profiler) of one
+child process, which loads torch ahead of the library so that both use one HIP
+runtime.  Tests of one way of launching against another compare results only;
+that the two ways are two is checked here."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+CHILD = r"""
+import json, re, sys
+import torch
+from torch.profiler import ProfilerActivity, profile
+import lceqcd_amd
+from lceqcd_amd import KC_GFIX
+
+def lattice(*shape):
+    L = lceqcd_amd.Lattice(*shape)
+    L.set_couplings(9.0, 0.175, -0.45, 0.025)
+    L.hotstart(5, 0.5)
+    L.rng_philox(5, 0)
+    return L
+
+def traced(L, call):
+    call()
+    L.sync()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        L.sync()
+        torch.cuda.synchronize()
+    counts = {}
+    for e in p.events():
+        k = re.search(r"\b(k_\w+)", e.name)
+        if k and "CUDA" in str(e.device_type):
+            counts[k.group(1)] = counts.get(k.group(1), 0) + 1
+    return counts
+
+def timed(L, call):
+    L.profile_begin(KC_GFIX, 1)
+    call()
+    L.profile_end()
+
+torch.zeros(1, device="cuda")
+out = {}
+for shape in ((16, 16, 16), (44, 44, 44)):
+    print("tracing", shape, file=sys.stderr, flush=True)
+    L = lattice(*shape)
+    out["tune %d" % shape[0]] = traced(L, lambda: L.autotune(n_or=2, trials=1))
+    out["order tune %d" % shape[0]] = traced(L, lambda: L.autotune_site_order(n_or=2, trials=1))
+    out["sweep %d" % shape[0]] = traced(L, lambda: L.sweep(0, 3, n_or=2, delta=0.4, measflag=0))
+    L.close()
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def launches():
+    print("device traces of launches", flush=True)
+    r = subprocess.run([sys.executable, "-c", CHILD], cwd=ROOT, capture_output=True, text=True,
+                       timeout=110)
+    assert r.returncode == 0, r.stderr[-2000:]
+    out = json.loads(r.stdout.splitlines()[-1])
+    print(out, flush=True)
+    if not any(out.values()):
+        pytest.skip("no device trace to be had")
+    return out
+
+
+@pytest.mark.parametrize("extent", [16, 44])
+def test_tuners_time_what_they_set(launches, extent):
+    """A launch shape and a site order are those of the launches per direction, so
+    the tuners time these where sweeps take three directions in one launch."""
+    assert launches["sweep %d" % extent] == {"k_link3": 18, "k_higgs": 6, "k_finalize": 3,
+                                             "k_set_obs": 1}
+    for name in ("tune %d", "order tune %d"):
+        got = launches[name % extent]
+        assert "k_link3" not in got and got["k_link"] == 9 * got["k_higgs"]
