@@ -927,11 +927,11 @@ def learned_batch(args, log=None):
     return res
 
 
-def hbm_resident_or(shape, n_or, tb_x, sweeps=10, order=0):
+def hbm_resident_or(shape, n_or, tb_x, sweeps=10, order=None):
     """The overrelaxation launch on a lattice too large for the 256 MB
     Infinity Cache (160^3: 490 MB of fields, 557 MB moved per launch), timed
     with HIP events as the 64^3 launch is, at the same launch shape and site
-    order `order` (-1: the one the site-order tuner picks)."""
+    order `order` (-1: the one the site-order tuner picks, None: the library's)."""
     import lceqcd_amd
     V = shape[0] * shape[1] * shape[2]
     L = lceqcd_amd.Lattice(*shape)
@@ -940,11 +940,11 @@ def hbm_resident_or(shape, n_or, tb_x, sweeps=10, order=0):
     L.rng_philox(12345, 0)
     L.set_shape(*tb_x)
     d = L.sweep(lceqcd_amd.SWEEP_KP_OR_METRO, 2, n_or=n_or, delta=0.4, measflag=0)
-    if order < 0:
+    orders = {}
+    if order is not None and order < 0:
         orders = L.autotune_site_order(n_or=n_or, trials=3)
-    else:
+    elif order is not None:
         L.set_site_order(order)
-        orders = {}
     L.profile_begin(lceqcd_amd.KC_LINK_OR, 6 * n_or * sweeps)
     L.sweep(lceqcd_amd.SWEEP_KP_OR_METRO, sweeps, n_or=n_or, delta=d, measflag=1)
     ms, n = L.profile_end()
@@ -975,7 +975,7 @@ def kernels(args):
     L.rng_philox(314159, 0)
     if args.shape:
         L.set_shape(*(int(v) for v in args.shape.split(",")))
-    if args.order > 0:
+    if args.order is not None and args.order >= 0:
         L.set_site_order(args.order)
     L.sweep(lceqcd_amd.SWEEP_REFERENCE, 2, measflag=1)
     L.history(2)
@@ -1154,11 +1154,12 @@ def main():
                     help="replicas96: replica group size in MiB of fields (0: one group; "
                          "default: the library's)")
     ap.add_argument("--scan-lattice", default="24,24,24")
-    ap.add_argument("--order", type=int, default=0,
+    ap.add_argument("--order", type=int, default=None,
                     help="site order (strip rows, 0 = index order, -1 = the site-order "
-                         "tuner's choice) of the measured lattice")
-    ap.add_argument("--big-order", type=int, default=0,
-                    help="site order of the 160^3 HBM-resident launch (-1: tuned)")
+                         "tuner's choice; default: the library's) of the measured lattice")
+    ap.add_argument("--big-order", type=int, default=None,
+                    help="site order of the 160^3 HBM-resident launch (-1: tuned; "
+                         "default: the library's)")
     ap.add_argument("--grid", default="literal", choices=["literal", "straddle"],
                     help="replicas96: the configuration's beta_2 grid (broken phase "
                          "throughout) or one that straddles the transition")
@@ -1224,11 +1225,11 @@ def main():
         tuned = {}
     else:
         tuned = L.autotune(n_or=args.n_or, trials=10)
-    if args.order < 0:
+    tuned_order = {}
+    if args.order is not None and args.order < 0:
         tuned_order = L.autotune_site_order(n_or=args.n_or, trials=10)
-    else:
+    elif args.order is not None:
         L.set_site_order(args.order)
-        tuned_order = {}
     L.sync()
 
     # timed region: K sweeps, synchronised on both sides

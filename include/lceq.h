@@ -95,15 +95,17 @@ int lceq_autotune(lceq_lattice *L, int n_or, int trials, double *ms);
  * reference): a power of two >= 2 dividing ly (with ly * lz < 2^22) takes the
  * rows (y, z) of a parity in strips of that many y rows, each strip advancing
  * through z, so that the z neighbours of the sites in flight stay in the L2;
- * strip_rows = 0 leaves the order to the library: index order, and strips
- * where a z plane is large (8192 sites of a parity or more).
+ * strip_rows = 0 takes the sites in index order.  Until it is called the order
+ * is the library's: index order, and strips where a z plane is large (8192
+ * sites of a parity or more).  lceq_get_site_order answers the rows in use.
  * Fields do not depend on the order; plaquette and Higgs sums are added in an
- * order-dependent way.  Default 0. */
+ * order-dependent way. */
 int lceq_set_site_order(lceq_lattice *L, int strip_rows);
 int lceq_get_site_order(lceq_lattice *L, int *strip_rows);
 /* time `trials` production sweeps with site orders 0, 4, 8, 16 (those that
  * divide ly) at the current launch shape, with launches per direction as
- * lceq_autotune, keep the fastest; fields, observables, the pass counter and the history are restored.  ms (or NULL)
+ * lceq_autotune, and with the library's own order where that is another one;
+ * keep the fastest; fields, observables, the pass counter and the history are restored.  ms (or NULL)
  * receives 4 times per sweep (-1 where an order does not fit). */
 int lceq_autotune_site_order(lceq_lattice *L, int n_or, int trials, double *ms);
 /* Measurement aid with no counterpart in the reference: a plain device copy

@@ -78,6 +78,7 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   L->vol = lx * ly * lz;
   L->tb = 256;
   L->xcd = 1;
+  L->strip = -1;
   L->pstride = (g.n + 63) / 64 + 8;  // block partials of the smallest launch shape
   L->beta = 9.0;
   L->lambda = 1.0;
@@ -385,7 +386,7 @@ extern "C" int lceq_set_site_order(lceq_lattice* L, int strip_rows) {
   if (sy != 0 && (sy < 2 || (sy & (sy - 1)) || L->g.ly % sy))
     return fail(LCEQ_ERR_ARG, "strip rows must be 0 or a power of two >= 2 dividing ly = %d",
                 L->g.ly);
-  // order_site divides a launch position by lx/2 to get its row; the
+  // strip_site divides a launch position by lx/2 to get its row; the
   // reciprocal division is exact for quotients below 2^22, so the rows
   // ly * lz of a parity must stay below that
   if (sy != 0 && (int64_t)L->g.ly * L->g.lz >= ((int64_t)1 << 22))
@@ -398,13 +399,13 @@ extern "C" int lceq_set_site_order(lceq_lattice* L, int strip_rows) {
 
 extern "C" int lceq_get_site_order(lceq_lattice* L, int* strip_rows) {
   NEEDL(L);
-  if (strip_rows) *strip_rows = L->strip;
+  if (strip_rows) *strip_rows = lceq::strip_rows(L);
   return LCEQ_OK;
 }
 
 // Time `trials` production sweeps with each site order of 0, 4, 8 and 16
-// strip rows (those dividing ly) at the current launch shape and keep the
-// fastest; the fields, the observables, the pass counter and the history are
+// strip rows (those dividing ly), and with the library's own order where that is
+// another one, at the current launch shape and keep the fastest; the fields, the observables, the pass counter and the history are
 // restored.  ms (or NULL) receives 4 times per sweep, -1 for an order that
 // does not fit the lattice.
 extern "C" int lceq_autotune_site_order(lceq_lattice* L, int n_or, int trials, double* ms) {
@@ -425,12 +426,15 @@ extern "C" int lceq_autotune_site_order(lceq_lattice* L, int n_or, int trials, d
     (void)hipEventDestroy(e0);
     return fail(LCEQ_ERR_HIP, "hipEventCreate failed");
   }
-  const int orders[4] = {0, 4, 8, 16};
+  const int before = strip_rows(L);
+  L->strip = -1;
+  const int orders[5] = {0, 4, 8, 16, strip_rows(L)};
   double best = 1e300, delta = o[OBS_DELTA];
-  int best_sy = L->strip, rc = LCEQ_OK;
+  int best_sy = before, rc = LCEQ_OK;
   L->tuning = 1;
-  for (int i = 0; i < 4 && rc == LCEQ_OK; ++i) {
+  for (int i = 0; i < 5 && rc == LCEQ_OK; ++i) {
     int sy = orders[i];
+    if (i == 4 && std::find(orders, orders + 4, sy) != orders + 4) break;
     if (sy && (L->g.ly % sy || (int64_t)L->g.ly * L->g.lz >= ((int64_t)1 << 22))) {
       if (ms) ms[i] = -1.0;  // the order does not fit (lceq_set_site_order's limits)
       continue;
@@ -446,7 +450,7 @@ extern "C" int lceq_autotune_site_order(lceq_lattice* L, int n_or, int trials, d
       break;
     }
     double per = (double)el / trials;
-    if (ms) ms[i] = per;
+    if (ms && i < 4) ms[i] = per;
     if (per < best) {
       best = per;
       best_sy = sy;

@@ -72,8 +72,8 @@ struct lceq_lattice {
   // launch shape of the link and Higgs updates: threads (= sites) per block
   // 64/128/256/512 and the XCD-aware block order (partials sized for 64)
   int tb, xcd;
-  // site order of those launches: strips of `strip` y rows (0: by the
-  // lattice's shape, strip_rows)
+  // site order of those launches: strips of `strip` y rows, 0 index order, -1 by
+  // the lattice's shape (strip_rows)
   int strip;
   int tuning;  // an autotuner times these: sweeps take launches that they apply to
   uint64_t seed, pass;

@@ -94,7 +94,7 @@ static bool early_schedule(const lceq_lattice* L) {
 // 12800 sites a plane on (200x200x40 0.890 0.677).
 int strip_rows(const lceq_lattice* L) {
   const Geom& g = L->g;
-  if (L->strip) return L->strip;
+  if (L->strip >= 0) return L->strip;
   if (g.h2 < 8192 || (int64_t)g.ly * g.lz >= (int64_t)1 << 22) return 0;
   int sy = 2;
   while ((int64_t)sy * g.h1 < 1024) sy *= 2;

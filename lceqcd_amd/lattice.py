@@ -138,9 +138,9 @@ class Lattice:
 
     # -------------------------------------------------------------- uniforms
     def set_site_order(self, strip_rows=0):
-        """Site order of the link and Higgs updates: 0 (the library's: index
-        order, strips on lattices with large planes) or strips of
-        ``strip_rows`` y rows advancing through z (same fields)."""
+        """Site order of the link and Higgs updates: index order (0) or strips
+        of ``strip_rows`` y rows advancing through z (same fields).  Until set it
+        is the library's: index order, strips on lattices with large planes."""
         self._check(self._L.lceq_set_site_order(self.h, int(strip_rows)))
 
     def get_site_order(self):

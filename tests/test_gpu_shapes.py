@@ -128,3 +128,35 @@ def test_stream_bandwidth_probe():
     rate = 31 * n * 16 / (us.value * 1e-6) / 1e9
     print("stream probe GB/s", rate, flush=True)
     assert np.isfinite(us.value) and 0.0 < rate < 20000.0
+
+
+@pytest.mark.parametrize("lat,own", [((160, 160, 6), 16), ((200, 200, 8), 2), ((64, 64, 16), 0)])
+def test_index_order_can_be_set(lat, own):
+    """The library's order on large planes is strips, and what is set replaces it:
+    0 is the index order.  The tuner times the library's order too where it is
+    none of the four."""
+    import lceqcd_amd
+    print("site order", lat, own, flush=True)
+    out = []
+    for order in (None, 0, 2):
+        L = lceqcd_amd.Lattice(*lat)
+        L.set_couplings(*COUP)
+        L.hotstart(6, 0.5)
+        L.rng_philox(6, 0)
+        assert L.get_site_order() == own
+        if order is not None:
+            L.set_site_order(order)
+            assert L.get_site_order() == order
+        L.sweep(0, 2, n_or=1, delta=0.4, measflag=1)
+        out.append((L.get_links(), L.get_higgs(), L.history(2)))
+        if order is None:
+            ms = L.autotune_site_order(n_or=1, trials=1)
+            got = L.get_site_order()
+            assert got in set(ms) | {own} and set(ms) <= {0, 4, 8, 16}
+            assert np.array_equal(L.get_links(), out[0][0])
+        L.close()
+    for got in out[1:]:
+        assert np.array_equal(got[0], out[0][0]) and np.array_equal(got[1], out[0][1])
+        np.testing.assert_allclose(got[2], out[0][2], rtol=1e-12, atol=1e-14)
+    if own:  # the orders add their sums differently, so they are not one order
+        assert not np.array_equal(out[1][2], out[0][2])
