@@ -108,10 +108,9 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
 
   alloc(&L->obs, LCEQ_OBS_N);
-  if (rc == LCEQ_OK &&
-      hipHostMalloc((void**)&L->pin, (LCEQ_OBS_N + LCEQ_PIN_DOUBLES) * sizeof(double),
-                    hipHostMallocDefault) != hipSuccess)
+  if (rc == LCEQ_OK && !(L->pin_block = pinned_take(L->device, PINNED_RESULTS)))
     rc = fail(LCEQ_ERR_HIP, "hipHostMalloc failed");
+  if (L->pin_block) L->pin = static_cast<double*>(pinned_host(L->pin_block));
   alloc(&L->slices, 14 * (size_t)lz * corr_split(L->g));
   alloc(&L->corr, 5 * (size_t)lz + 8);
   L->hist_cap = 4096;
@@ -147,7 +146,7 @@ extern "C" int lceq_destroy(lceq_lattice* L) {
                     L->partials, L->obs, L->slices, L->corr, L->hist, L->scratch, L->fed};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
-  if (L->pin) (void)hipHostFree(L->pin);
+  if (L->pin_block) pinned_give(L->pin_block);
   if (L->prof_ev) {
     for (int i = 0; i < L->prof_cap; ++i) (void)hipEventDestroy(L->prof_ev[i]);
     delete[] L->prof_ev;

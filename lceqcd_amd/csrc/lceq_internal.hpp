@@ -34,6 +34,10 @@ enum {
 // doubles of lceq_lattice::pin after the observables (64 KiB in all)
 #define LCEQ_PIN_DOUBLES (8192 - LCEQ_OBS_N)
 
+namespace lceq {
+struct Pinned;
+}
+
 struct lceq_lattice {
   lceq::Geom g;
   int vol;
@@ -55,6 +59,7 @@ struct lceq_lattice {
   // pinned host memory that kernels write results to: the observables, then
   // PIN_DOUBLES values of any other small result
   double *pin;
+  lceq::Pinned* pin_block;
   double *hist;      // [hist_cap][LCEQ_OBS_N] per-sweep records
   int hist_cap;
   int hist_rows;     // rows recorded since the last lceq_history
@@ -147,6 +152,14 @@ int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, d
                    int64_t ld, int ncomp, int nclass, bool get);
 // a lattice or batch that transfers fields exists (+1) or is gone (-1)
 void transfer_user(int change);
+// Pinned host memory of a device, from and to a pool (lceq_transfer.hip); null
+// without memory.  A block goes back when no kernel uses it any more.
+enum { PINNED_RESULTS, PINNED_SMALL, PINNED_LARGE, PINNED_KINDS };
+constexpr size_t PINNED_RESULTS_BYTES = (LCEQ_OBS_N + LCEQ_PIN_DOUBLES) * sizeof(double);
+struct Pinned;
+Pinned* pinned_take(int device, int kind);
+void pinned_give(Pinned* block);
+void* pinned_host(Pinned* block);
 
 // launchers (lceq_kernels.hip); all enqueue on L->stream, no host sync.
 // Link launches use reduction slots 0-5 ((eo, mu) order), Higgs launches

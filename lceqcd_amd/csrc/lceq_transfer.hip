@@ -12,10 +12,10 @@
 #include <string.h>
 
 #include <algorithm>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
-#include <vector>
 
 #include "../../include/lceq.h"
 #include "lceq_internal.hpp"
@@ -62,60 +62,82 @@ constexpr int SLOTS = 2 * MAX_WORKERS;
 constexpr size_t SLOT_BYTES = 1536 << 10;  // whole rows of 32 and of 24 bytes
 constexpr size_t MIN_CHUNK = SLOT_BYTES / 2;
 
-struct Stage {
-  int device;
+}  // namespace
+
+// Pinned blocks not in use stay allocated for the next lattice, batch or transfer
+// on their device, up to KEEP of each kind (121 MiB) while a lattice or batch
+// exists and LEFT (one of each, 26 MiB) when none does, so that a program that
+// makes lattices one after the other does not allocate them each time: the driver
+// unmaps a freed block behind the call, and the next lattice's allocations wait for
+// it.  A life with the links read and written, in us, with pageable copies, with
+// blocks freed with the last lattice, and as here: 8^3 154-246 213-291 193-227,
+// 16^3 202-260 225-343 244-261, 24^3 411-752 1530-2400 1080-1290, 40^3 2700-2910
+// 915-980 800-885.
+struct Pinned {
+  int device, kind;
   char* host;
-  hipEvent_t ev[SLOTS];
+  hipEvent_t ev[SLOTS];  // EVENTS of them
 };
 
-// Stages not in use: at most KEEP of them stay allocated (24 MiB of pinned
-// memory each) for the next transfer of any lattice or batch on their device,
-// and none once the last lattice and batch are destroyed.
-constexpr size_t KEEP = 2;
+namespace {
+
+constexpr size_t PINNED_BYTES[PINNED_KINDS] = {PINNED_RESULTS_BYTES, 2 * MIN_CHUNK,
+                                               SLOTS * SLOT_BYTES};
+constexpr int EVENTS[PINNED_KINDS] = {0, 2, SLOTS};
+constexpr int KEEP[PINNED_KINDS] = {16, 16, 4}, LEFT[PINNED_KINDS] = {1, 1, 1}, KEEP_MOST = 16;
 std::mutex g_mu;
-std::vector<Stage*> g_idle;
+Pinned* g_idle[PINNED_KINDS][KEEP_MOST];
+int g_nidle[PINNED_KINDS];
 int g_users = 0;
 
-void stage_free(Stage* S) {
-  for (hipEvent_t e : S->ev)
+void pinned_free(Pinned* P) {
+  for (hipEvent_t e : P->ev)
     if (e) (void)hipEventDestroy(e);
-  if (S->host) (void)hipHostFree(S->host);
-  delete S;
+  if (P->host) (void)hipHostFree(P->host);
+  delete P;
 }
 
-Stage* stage_take(int device) {
+}  // namespace
+
+Pinned* pinned_take(int device, int kind) {
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    for (size_t i = 0; i < g_idle.size(); ++i)
-      if (g_idle[i]->device == device) {
-        Stage* S = g_idle[i];
-        g_idle.erase(g_idle.begin() + i);
-        return S;
+    for (int i = g_nidle[kind] - 1; i >= 0; --i)
+      if (g_idle[kind][i]->device == device) {
+        Pinned* P = g_idle[kind][i];
+        g_idle[kind][i] = g_idle[kind][--g_nidle[kind]];
+        return P;
       }
   }
-  Stage* S = new Stage();
-  memset(S, 0, sizeof(*S));
-  S->device = device;
-  bool ok = hipHostMalloc((void**)&S->host, SLOTS * SLOT_BYTES, hipHostMallocDefault) == hipSuccess;
-  for (int i = 0; ok && i < SLOTS; ++i)
-    ok = hipEventCreateWithFlags(&S->ev[i], hipEventDisableTiming) == hipSuccess;
+  Pinned* P = new (std::nothrow) Pinned();
+  if (!P) return nullptr;
+  P->device = device;
+  P->kind = kind;
+  bool ok = hipHostMalloc((void**)&P->host, PINNED_BYTES[kind], hipHostMallocDefault) == hipSuccess;
+  for (int i = 0; ok && i < EVENTS[kind]; ++i)
+    ok = hipEventCreateWithFlags(&P->ev[i], hipEventDisableTiming) == hipSuccess;
   if (!ok) {
-    stage_free(S);
+    (void)hipGetLastError();  // reported here, not by the next launch
+    pinned_free(P);
     return nullptr;
   }
-  return S;
+  return P;
 }
 
-void stage_give(Stage* S) {
+void pinned_give(Pinned* P) {
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_users > 0 && g_idle.size() < KEEP) {
-      g_idle.push_back(S);
+    if (g_nidle[P->kind] < (g_users > 0 ? KEEP : LEFT)[P->kind]) {
+      g_idle[P->kind][g_nidle[P->kind]++] = P;
       return;
     }
   }
-  stage_free(S);
+  pinned_free(P);
 }
+
+void* pinned_host(Pinned* P) { return P->host; }
+
+namespace {
 
 struct Transfer {
   hipStream_t stream;
@@ -126,8 +148,9 @@ struct Transfer {
   int ncomp;
   bool get;
   unsigned rows, rows_per_slot;
+  size_t slot_bytes;
   int chunks, workers;
-  Stage* stage;
+  Pinned* stage;
 };
 
 // copy between the slot and the caller's array: row r of the field is at
@@ -181,7 +204,7 @@ hipError_t run_worker(const Transfer& t, int w) {
   };
   for (int c = w; c < t.chunks && e == hipSuccess; c += t.workers) {
     int k = slot_of(c);
-    char* slot = t.stage->host + (size_t)k * SLOT_BYTES;
+    char* slot = t.stage->host + (size_t)k * t.slot_bytes;
     unsigned row0 = (unsigned)c * t.rows_per_slot;
     if (!t.get) {
       int before = c - 2 * t.workers;  // the slot's previous chunk
@@ -194,14 +217,14 @@ hipError_t run_worker(const Transfer& t, int w) {
     if (t.chunks > 1 && (e = hipEventRecord(t.stage->ev[k], t.stream)) != hipSuccess) break;
     if (t.get && prev >= 0) {
       if ((e = finish(prev)) != hipSuccess) break;
-      host_copy(t, t.stage->host + (size_t)slot_of(prev) * SLOT_BYTES,
+      host_copy(t, t.stage->host + (size_t)slot_of(prev) * t.slot_bytes,
                 (unsigned)prev * t.rows_per_slot, rows_of(prev));
     }
     prev = c;
   }
   if (t.get && prev >= 0 && e == hipSuccess) {
     if ((e = finish(prev)) != hipSuccess) return e;
-    host_copy(t, t.stage->host + (size_t)slot_of(prev) * SLOT_BYTES,
+    host_copy(t, t.stage->host + (size_t)slot_of(prev) * t.slot_bytes,
               (unsigned)prev * t.rows_per_slot, rows_of(prev));
   }
   return e;
@@ -210,13 +233,15 @@ hipError_t run_worker(const Transfer& t, int w) {
 }  // namespace
 
 void transfer_user(int change) {
-  std::vector<Stage*> drop;
+  Pinned* drop[PINNED_KINDS * KEEP_MOST];
+  int ndrop = 0;
   {
     std::lock_guard<std::mutex> lock(g_mu);
     g_users += change;
-    if (g_users == 0) drop.swap(g_idle);
+    for (int k = 0; g_users == 0 && k < PINNED_KINDS; ++k)
+      while (g_nidle[k] > LEFT[k]) drop[ndrop++] = g_idle[k][--g_nidle[k]];
   }
-  for (Stage* S : drop) stage_free(S);
+  while (ndrop) pinned_free(drop[--ndrop]);
 }
 
 int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, double* host,
@@ -240,11 +265,13 @@ int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, d
   const size_t rb = (size_t)ncomp * sizeof(double);
   unsigned share = (t.rows + MAX_WORKERS - 1) / MAX_WORKERS;
   t.rows_per_slot = std::min((unsigned)(SLOT_BYTES / rb), std::max((unsigned)(MIN_CHUNK / rb), share));
+  t.slot_bytes = t.rows_per_slot * rb;
   t.chunks = (int)((t.rows + t.rows_per_slot - 1) / t.rows_per_slot);
   t.workers = std::min(MAX_WORKERS, std::max(1, t.chunks / 2));
   int current = device;
   if (hipGetDevice(&current) == hipSuccess && current != device) (void)hipSetDevice(device);
-  t.stage = stage_take(device);
+  // one worker's chunks are MIN_CHUNK, and it has two slots
+  t.stage = pinned_take(device, t.workers > 1 ? PINNED_LARGE : PINNED_SMALL);
   if (!t.stage) {
     if (current != device) (void)hipSetDevice(current);
     return set_error(LCEQ_ERR_HIP, "no pinned memory for a field transfer");
@@ -257,7 +284,7 @@ int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, d
         err[w] = hipSetDevice(t.device);
         if (err[w] == hipSuccess) err[w] = run_worker(t, w);
       });
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {
       err[w] = run_worker(t, w);  // no thread to be had: its chunks here
     }
   }
@@ -274,7 +301,7 @@ int transfer_field(hipStream_t stream, int device, const Geom& g, double* dev, d
     if (e == hipSuccess) e = es;
   }
   if (current != device) (void)hipSetDevice(current);
-  stage_give(t.stage);
+  pinned_give(t.stage);
   if (e != hipSuccess)
     return set_error(LCEQ_ERR_HIP, "field transfer failed: %s", hipGetErrorString(e));
   return LCEQ_OK;

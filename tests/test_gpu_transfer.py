@@ -108,3 +108,42 @@ def test_history_ring_of_a_batch():
     assert np.array_equal(B.history(600)[:500], rows[0][500:])
     assert np.array_equal(B.observables(), rows[1][-1])
     B.close()
+
+
+def test_pinned_blocks_are_used_again():
+    """A pinned block that was given back is the next one taken, also when no
+    lattice exists, and never by two at a time; the pool keeps a bounded number
+    (csrc/lceq_transfer.hip KEEP and LEFT: 16 and 1 of the first kind)."""
+    import gc
+    import lceqcd_amd
+    from lceqcd_amd import _lib
+    lib = C.CDLL(_lib.load()._name)  # prototypes of its own
+    take, give = lib._ZN4lceq11pinned_takeEii, lib._ZN4lceq11pinned_giveEPNS_6PinnedE
+    host = lib._ZN4lceq11pinned_hostEPNS_6PinnedE
+    take.restype, take.argtypes = C.c_void_p, [C.c_int, C.c_int]
+    give.restype, give.argtypes = None, [C.c_void_p]
+    host.restype, host.argtypes = C.c_void_p, [C.c_void_p]
+    print("pinned blocks", flush=True)
+    gc.collect()  # lattices of other tests
+    L = lceqcd_amd.Lattice(4, 4, 4)
+    for kind in range(3):
+        blocks = [take(0, kind) for _ in range(3)]
+        assert all(blocks) and len({host(b) for b in blocks}) == 3
+        give(blocks[1])
+        assert take(0, kind) == blocks[1]
+        for b in blocks:
+            give(b)
+        again = [take(0, kind) for _ in range(3)]
+        assert set(again) == set(blocks)
+        for b in again:
+            give(b)
+    many = [take(0, 0) for _ in range(20)]
+    for b in many:
+        give(b)
+    L.close()
+    b = take(0, 0)
+    assert b and host(b)
+    C.memset(host(b), 0, 65536)
+    give(b)
+    assert take(0, 0) == b
+    give(b)
