@@ -66,6 +66,65 @@ static bool spare_links(lceq_lattice* L) {
   return L->spare != nullptr;
 }
 
+// The device arrays of a lattice, zeroed, so that padding lanes hold finite values.
+// Up to ARENA_MAX in all (to 52^3) they share one allocation and one fill: 13 of
+// each, and what the driver does behind them, cost more than the rest of a small
+// lattice's life.  A life with the links read and written, in us, with arrays of
+// their own and as here: 8^3 193-227 126-135, 16^3 244-261 185-195, 24^3 1080-1290
+// 284-292, 32^3 638-645 445-459, 48^3 1165 879-897.  The updates run alike.
+constexpr size_t ARENA_MAX = (size_t)64 << 20;
+
+static int create_arrays(lceq_lattice* L) {
+  const Geom& g = L->g;
+  const size_t np = (size_t)g.npad, lz = (size_t)g.lz;
+  const struct {
+    double** p;
+    size_t count;
+  } arrays[] = {{&L->U, 24 * np},
+                {&L->A, 6 * np},
+                {&L->Uf, 24 * np},
+                {&L->Af, 6 * np},
+                {&L->Vst, 24 * np},
+                {&L->F, 3 * np},
+                {&L->gf_part, 2 * (size_t)lattice_tiles(g) + (gfix_site_sums(g) ? (size_t)g.n : 0)},
+                {&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride},
+                {&L->obs, LCEQ_OBS_N},
+                {&L->slices, 14 * lz * corr_split(g)},
+                {&L->corr, 5 * lz + 8},
+                {&L->hist, (size_t)L->hist_cap * LCEQ_OBS_N},
+                // last: without memory for it a lattice of its own arrays goes without
+                {&L->spare, link3_tiles(g) ? 24 * np : 0}};
+  auto room = [](size_t count) { return (count * sizeof(double) + 4095) / 4096 * 4096; };
+  size_t total = 0;
+  for (const auto& a : arrays) total += room(a.count);
+  if (total <= ARENA_MAX && hipMalloc((void**)&L->arena, total) == hipSuccess) {
+    L->arena_bytes = total;
+    char* at = L->arena;
+    for (const auto& a : arrays) {
+      if (a.count) *a.p = reinterpret_cast<double*>(at);
+      at += room(a.count);
+    }
+    HIPCHK(hipMemsetAsync(L->arena, 0, total, L->stream));
+    return LCEQ_OK;
+  }
+  (void)hipGetLastError();
+  L->arena = nullptr;
+  for (const auto& a : arrays) {
+    if (!a.count) continue;
+    if (a.p == &L->spare) {
+      (void)spare_links(L);
+      continue;
+    }
+    hipError_t e = hipMalloc((void**)a.p, a.count * sizeof(double));
+    if (e != hipSuccess) {
+      *a.p = nullptr;
+      return fail(LCEQ_ERR_HIP, "hipMalloc(%zu doubles): %s", a.count, hipGetErrorString(e));
+    }
+    HIPCHK(hipMemsetAsync(*a.p, 0, a.count * sizeof(double), L->stream));
+  }
+  return LCEQ_OK;
+}
+
 extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   if (!out) return fail(LCEQ_ERR_ARG, "null output pointer");
   *out = nullptr;
@@ -88,48 +147,17 @@ extern "C" int lceq_create(int lx, int ly, int lz, lceq_lattice** out) {
   L->rng_mode = LCEQ_RNG_PHILOX;
   L->seed = 12345;
   int rc = LCEQ_OK;
-  auto alloc = [&](double** p, size_t count) {
-    if (rc != LCEQ_OK) return;
-    hipError_t e = hipMalloc((void**)p, count * sizeof(double));
-    if (e != hipSuccess) rc = fail(LCEQ_ERR_HIP, "hipMalloc(%zu doubles): %s", count, hipGetErrorString(e));
-  };
-  size_t np = (size_t)g.npad;
   if (hipGetDevice(&L->device) != hipSuccess) rc = fail(LCEQ_ERR_HIP, "no HIP device");
   if (rc == LCEQ_OK && hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking) != hipSuccess)
     rc = fail(LCEQ_ERR_HIP, "hipStreamCreate failed");
 
-  alloc(&L->U, 24 * np);
-  alloc(&L->A, 6 * np);
-  alloc(&L->Uf, 24 * np);
-  alloc(&L->Af, 6 * np);
-  alloc(&L->Vst, 24 * np);
-  alloc(&L->F, 3 * np);
-  alloc(&L->gf_part, 2 * (size_t)lattice_tiles(g) + (gfix_site_sums(g) ? (size_t)g.n : 0));
-  alloc(&L->partials, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride);
-
-  alloc(&L->obs, LCEQ_OBS_N);
   if (rc == LCEQ_OK && !(L->pin_block = pinned_take(L->device, PINNED_RESULTS)))
     rc = fail(LCEQ_ERR_HIP, "hipHostMalloc failed");
   if (L->pin_block) L->pin = static_cast<double*>(pinned_host(L->pin_block));
-  alloc(&L->slices, 14 * (size_t)lz * corr_split(L->g));
-  alloc(&L->corr, 5 * (size_t)lz + 8);
   L->hist_cap = 4096;
-  alloc(&L->hist, (size_t)L->hist_cap * LCEQ_OBS_N);
-  if (rc == LCEQ_OK) {
-    // zero every field so padding lanes hold finite values
-    (void)hipMemsetAsync(L->U, 0, 24 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->A, 0, 6 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->Uf, 0, 24 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->Af, 0, 6 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->Vst, 0, 24 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->F, 0, 3 * np * sizeof(double), L->stream);
-    (void)hipMemsetAsync(L->partials, 0, (size_t)LCEQ_NSLOT * LCEQ_NQ * L->pstride * sizeof(double),
-                   L->stream);
-    (void)hipMemsetAsync(L->obs, 0, LCEQ_OBS_N * sizeof(double), L->stream);
-    if (link3_tiles(L->g)) (void)spare_links(L);
-
-    if (hipStreamSynchronize(L->stream) != hipSuccess) rc = fail(LCEQ_ERR_HIP, "init sync failed");
-  }
+  if (rc == LCEQ_OK) rc = create_arrays(L);
+  if (rc == LCEQ_OK && hipStreamSynchronize(L->stream) != hipSuccess)
+    rc = fail(LCEQ_ERR_HIP, "init sync failed");
   transfer_user(1);
   if (rc != LCEQ_OK) {
     lceq_destroy(L);
@@ -144,8 +172,11 @@ extern "C" int lceq_destroy(lceq_lattice* L) {
   if (L->stream) (void)hipStreamSynchronize(L->stream);
   double* bufs[] = {L->U, L->A, L->Uf, L->Af, L->Vst, L->F, L->spare, L->gf_part,
                     L->partials, L->obs, L->slices, L->corr, L->hist, L->scratch, L->fed};
-  for (double* b : bufs)
-    if (b) (void)hipFree(b);
+  for (double* b : bufs) {
+    const char* p = reinterpret_cast<char*>(b);
+    if (p && !(L->arena && p >= L->arena && p < L->arena + L->arena_bytes)) (void)hipFree(b);
+  }
+  if (L->arena) (void)hipFree(L->arena);
   if (L->pin_block) pinned_give(L->pin_block);
   if (L->prof_ev) {
     for (int i = 0; i < L->prof_cap; ++i) (void)hipEventDestroy(L->prof_ev[i]);

@@ -43,6 +43,9 @@ struct lceq_lattice {
   int vol;
   int device;
   hipStream_t stream;
+  // One allocation for the arrays of a small lattice (create_arrays), or null
+  char* arena;
+  size_t arena_bytes;
   // device fields
   double *U, *A, *Uf, *Af, *Vst, *F;
   // A second link array (spare_links): link sweeps and landau_gauge read one

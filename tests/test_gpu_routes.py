@@ -54,6 +54,23 @@ for shape in ((16, 16, 16), (44, 44, 44)):
     out["order tune %d" % shape[0]] = traced(L, lambda: L.autotune_site_order(n_or=2, trials=1))
     out["sweep %d" % shape[0]] = traced(L, lambda: L.sweep(0, 3, n_or=2, delta=0.4, measflag=0))
     L.close()
+def life():
+    L = lceqcd_amd.Lattice(8, 8, 8)
+    u = L.get_links()
+    L.put_links(u)
+    L.put_higgs(L.get_higgs())
+    L.close()
+
+print("tracing allocations", file=sys.stderr, flush=True)
+keep = lattice(4, 4, 4)
+life()
+with profile(activities=[ProfilerActivity.CUDA]) as p:
+    for _ in range(3):
+        life()
+    torch.cuda.synchronize()
+out["life"] = {}
+for e in p.events():
+    out["life"][e.name] = out["life"].get(e.name, 0) + 1
 print(json.dumps(out))
 """
 
@@ -80,3 +97,10 @@ def test_tuners_time_what_they_set(launches, extent):
     for name in ("tune %d", "order tune %d"):
         got = launches[name % extent]
         assert "k_link3" not in got and got["k_link"] == 9 * got["k_higgs"]
+
+
+def test_a_small_lattice_is_one_allocation(launches):
+    """Three lattices made, filled, read and closed one after the other."""
+    life = launches["life"]
+    assert life["hipMalloc"] == 3 and life["hipFree"] == 3
+    assert sum(n for name, n in life.items() if "_host<" in name) == 12

@@ -147,3 +147,33 @@ def test_pinned_blocks_are_used_again():
     give(b)
     assert take(0, 0) == b
     give(b)
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2), (16, 16, 16), (52, 52, 52), (54, 54, 54)])
+def test_arrays_of_a_lattice_are_apart(shape):
+    """Up to 64 MiB a lattice's arrays share one allocation: what is written to
+    each by its own calls leaves the others as they are, also when the link
+    arrays have changed places."""
+    import lceqcd_amd
+    print("arrays of", shape, flush=True)
+    n = shape[0] * shape[1] * shape[2] // 2
+    rng = np.random.default_rng(2)
+    fields = {"links": rng.normal(size=(3, 2, n, 4)), "higgs": rng.normal(size=(2, n, 3)),
+              "links_fixed": rng.normal(size=(3, 2, n, 4)), "higgs_fixed": rng.normal(size=(2, n, 3))}
+    L = lceqcd_amd.Lattice(*shape)
+    L.set_couplings(9.0, 0.175, -0.45, 0.025)
+    L.hotstart(3, 0.5)
+    L.rng_philox(3, 0)
+    L.sweep(0, 3, n_or=1, delta=0.4, measflag=1)
+    rows = L.history(2)
+    assert np.isfinite(rows).all()
+    L.set_gauge_fixing(1.7, 1.0, 1e-300, 9)
+    with pytest.raises(lceqcd_amd.LceqError, match="max_iter"):
+        L.landau_gauge()
+    for name, field in fields.items():
+        getattr(L, "put_" + name)(field)
+    L.correlator()
+    L.polyakov()
+    for name, field in fields.items():
+        assert np.array_equal(getattr(L, "get_" + name)(), field)
+    L.close()
