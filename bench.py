@@ -467,8 +467,12 @@ def scan(args):
                       "beta_a": res}), flush=True)
 
 
-REF_SWEEP_BYTES_PER_SITE = 2 * 2 * HIGGS_PASS_BYTES_PER_SITE + 6 * LINK_PASS_BYTES_PER_SITE + 192
-GFIX_PASS_BYTES_PER_SITE = 216   # all links read + written, a_f of one parity read + written
+# renorm is carried by the next sweep's first Higgs launch, which reads every link
+# anyway: its writes are what it adds
+REF_SWEEP_BYTES_PER_SITE = 2 * 2 * HIGGS_PASS_BYTES_PER_SITE + 6 * LINK_PASS_BYTES_PER_SITE + 96
+# one landau_gauge iteration by its launches: one reads and writes every link and
+# a_f once, two (one per parity) every link each and a_f of their parity
+GFIX_BYTES_PER_SITE = {1: 192 + 48, 2: 2 * (192 + 24)}
 SLICES_BYTES_PER_SITE = 144      # u_f 96 + a_f 24 + a 24
 
 
@@ -624,6 +628,18 @@ def reference_schedule_summary(seconds, procs=16):
     return rec
 
 
+def gfix_launches(L):
+    """Launches of one landau_gauge iteration on this lattice (its u_f changes)."""
+    import lceqcd_amd
+    L.set_gauge_fixing(1.7, 1.0, 1e-300, 8)
+    L.profile_begin(lceqcd_amd.KC_GFIX, 64)
+    try:
+        L.landau_gauge()
+    except lceqcd_amd.LceqError:
+        pass  # stops at its eight iterations
+    return L.profile_end()[1] // 8
+
+
 def refsched64(args):
     """The reference schedule, gauge fixing and correlators at 64^3."""
     import lceqcd_amd
@@ -672,9 +688,10 @@ def refsched64(args):
     corr_ms = (time.perf_counter() - t0) * 1e3 / ncorr
     kp_us = kp_ms * 1e3 / max(kp_n, 1)
     kp_bytes = LINK_PASS_BYTES_PER_SITE * V
-    # one iteration = two k_gfix launches (one per parity)
+    gf_launches = gfix_launches(L)
+    gf_bytes = GFIX_BYTES_PER_SITE[gf_launches] * V
     gf_us = gf_ms * 1e3 / max(iters, 1)
-    gf_gbps = 2 * GFIX_PASS_BYTES_PER_SITE * V / (gf_us * 1e-6) / 1e9
+    gf_gbps = gf_bytes / (gf_us * 1e-6) / 1e9
     rec = {
         "metric": METRIC,
         "value": V / (ms * 1e-3),
@@ -700,7 +717,8 @@ def refsched64(args):
             "higgs_launch_us": hg_ms * 1e3 / max(hg_n, 1),
             "landau_gauge": {"iterations": iters, "da": da, "ms": gf_ms,
                              "us_per_iteration": gf_us,
-                             "bytes_per_iteration": 2 * GFIX_PASS_BYTES_PER_SITE * V,
+                             "launches_per_iteration": gf_launches,
+                             "bytes_per_iteration": gf_bytes,
                              "algorithmic_GBps": gf_gbps,
                              "frac_of_hbm": gf_gbps / HBM_PEAK_GBPS},
             "correlators_ms": corr_ms,
@@ -929,7 +947,8 @@ def learned_batch(args, log=None):
 
 def hbm_resident_or(shape, n_or, tb_x, sweeps=10, order=None):
     """The overrelaxation launch on a lattice too large for the 256 MB
-    Infinity Cache (160^3: 490 MB of fields, 557 MB moved per launch), timed
+    Infinity Cache (160^3: 490 MB of fields, 557 MB moved per launch), over the
+    whole lattice (sweeps of it go by slabs that the cache holds), timed
     with HIP events as the 64^3 launch is, at the same launch shape and site
     order `order` (-1: the one the site-order tuner picks, None: the library's)."""
     import lceqcd_amd
@@ -1077,7 +1096,10 @@ def sizes(args):
     configurations, and on 128^3 and 160^3 (whose fields no cache holds):
     autotuned launch shape, then args.steps timed sweeps (scaled down to
     about 1.2e9 site-updates at the larger sizes) and the OR launch from HIP
-    events.  One JSON line."""
+    events.  The OR launch is the one per direction and whole lattice, which is
+    what a timed class runs; the sweeps of some sizes take three directions in
+    one launch, which moves less, or go by slabs, so a sweep's rate is given as
+    that of launches per direction in the same time.  One JSON line."""
     import lceqcd_amd
     out = []
     for shape in SIZES:
@@ -1100,7 +1122,8 @@ def sizes(args):
         or_us = 1e3 * or_ms / max(or_n, 1)
         rec = {"lattice": list(shape), "sites": V, "fields_MB": 120 * V / 1e6, "steps": steps,
                "ms_per_sweep": ms, "site_updates_per_s": V / (ms * 1e-3),
-               "sweep_algorithmic_GBps": SWEEP_BYTES_PER_SITE * V / (ms * 1e-3) / 1e9,
+               "per_direction_equivalent_GBps":
+                   SWEEP_BYTES_PER_SITE * V / (ms * 1e-3) / 1e9,
                "or_launch_us": or_us,
                "or_launch_GBps": LINK_PASS_BYTES_PER_SITE * V / (or_us * 1e-6) / 1e9,
                "launch_shape": list(L.get_shape())}

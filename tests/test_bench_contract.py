@@ -23,3 +23,15 @@ def test_help_lists_the_driver_flags():
     assert r.returncode == 0
     for flag in ("--gpus", "--steps", "--warmup", "--workload"):
         assert flag in r.stdout
+
+
+def test_bytes_follow_the_launches():
+    """What the record's rates are made of: a gauge-fixing iteration reads and
+    writes every link once in one launch and twice in two, and a_f once either
+    way; renorm adds its writes to a launch that reads the links anyway."""
+    sys.path.insert(0, ROOT)
+    import bench
+    links, higgs = 3 * 32, 24  # bytes a site
+    assert bench.GFIX_BYTES_PER_SITE == {1: 2 * links + 2 * higgs, 2: 4 * links + 2 * higgs}
+    assert bench.REF_SWEEP_BYTES_PER_SITE == 4 * bench.HIGGS_PASS_BYTES_PER_SITE \
+        + 6 * bench.LINK_PASS_BYTES_PER_SITE + links
