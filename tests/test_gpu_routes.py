@@ -54,6 +54,17 @@ for shape in ((16, 16, 16), (44, 44, 44)):
     out["order tune %d" % shape[0]] = traced(L, lambda: L.autotune_site_order(n_or=2, trials=1))
     out["sweep %d" % shape[0]] = traced(L, lambda: L.sweep(0, 3, n_or=2, delta=0.4, measflag=0))
     L.close()
+for name, shape in (("link3", (16, 16, 16)), ("slabs", (128, 128, 160))):
+    print("tracing", name, file=sys.stderr, flush=True)
+    L = lattice(*shape)
+    production = lambda: L.sweep(0, 3, n_or=1, delta=0.4, measflag=0)
+    reference = lambda: L.sweep(1, 3, measflag=0)
+    out[name] = traced(L, production)
+    out[name + " timed"] = traced(L, lambda: timed(L, production))
+    out[name + " reference"] = traced(L, reference)
+    out[name + " reference timed"] = traced(L, lambda: timed(L, reference))
+    L.close()
+
 def life():
     L = lceqcd_amd.Lattice(8, 8, 8)
     u = L.get_links()
@@ -104,3 +115,19 @@ def test_a_small_lattice_is_one_allocation(launches):
     life = launches["life"]
     assert life["hipMalloc"] == 3 and life["hipFree"] == 3
     assert sum(n for name, n in life.items() if "_host<" in name) == 12
+
+
+def test_timed_sweeps_take_the_launches_per_direction(launches):
+    """What tests compare three directions in one launch, slabs and the carried
+    renorm with: 6 link launches of the whole lattice per link sweep, 2 per Higgs
+    update and a renorm per reference sweep while a class is timed."""
+    assert launches["link3"]["k_link3"] == 12 and "k_link" not in launches["link3"]
+    slabs = launches["slabs"]
+    assert "k_link3" not in slabs and slabs["k_link"] == 2 * 36 and slabs["k_higgs"] == 2 * 6
+    for name in ("link3", "slabs"):
+        timed = launches[name + " timed"]
+        assert "k_link3" not in timed and timed["k_link"] == 36 and timed["k_higgs"] == 6
+        assert launches[name + " reference"]["k_renorm"] == 1
+        timed = launches[name + " reference timed"]
+        assert "k_link3" not in timed
+        assert timed["k_link"] == 18 and timed["k_higgs"] == 12 and timed["k_renorm"] == 3

@@ -80,3 +80,34 @@ def test_library_order_on_large_planes(shape, order):
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][2], out[1][2])
     _same_sums(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("shape", [(144, 144, 128), (174, 150, 130), (256, 256, 44)])
+def test_slabs_in_the_librarys_order(shape):
+    """Slabs and the library's site order together (strips of 16 and of 2 rows),
+    against whole-lattice launches in index order and against a batch of one
+    replica, whose launches are whole and in index order."""
+    import lceqcd_amd
+    print("slabs in the library's order", shape, flush=True)
+    coup = (9.0, 0.175, -0.45, 0.025)
+    out = []
+    for whole in (False, True):
+        L = _lattice(shape, 5)
+        if whole:
+            assert L.get_site_order() > 0
+            L.set_site_order(0)
+            L.profile_begin(lceqcd_amd.KC_GFIX, 1)
+        L.sweep(0, 2, n_or=2, delta=0.4, measflag=1)
+        out.append((L.get_links(), L.get_higgs(), L.history(2)))
+        L.close()
+    B = lceqcd_amd.Batch([shape])
+    B.set_couplings([coup])
+    B.hotstart([5], 0.5)
+    B.rng_philox([5])
+    B.sweep(2, n_or=2, delta=0.4, measflag=1)
+    out.append((B.get_links(0), B.get_higgs(0), B.history(2)[:, 0]))
+    B.close()
+    for got in out[1:]:
+        assert np.array_equal(got[0], out[0][0])
+        assert np.array_equal(got[1], out[0][1])
+        _same_sums(got[2], out[0][2])

@@ -60,3 +60,25 @@ def test_losses_of_more_steps_than_one_download():
     a = np.concatenate([mlp.train(512, batch=512, lr=2e-3, seed=1), ])
     assert np.array_equal(a.astype(np.float32), got["loss"][:512])
     assert np.isfinite(got["loss"]).all() and (got["loss"] != 0).all()
+
+
+def test_each_loss_is_that_of_its_step():
+    """Losses at the end of the first download (512 steps), in the second and at its
+    end: with batches of all records a step's loss is the mean over the records at
+    the parameters before it, so that a call of one step from these parameters
+    gives it again, up to the order of 512 single-precision terms in blocks of 32
+    (32 x 2^-24 of their size, which 2e-5 of 1 + |loss| covers tenfold)."""
+    from perf import cases
+    print("losses of their steps", flush=True)
+    case = {"kind": "train", "lx": 8, "ly": 8, "lz": 8, "stride": 1, "steps": 600, "batch": 512}
+    state = cases.prepare(case, 4)
+    loss = cases.run(state)["loss"]
+    mlp = state["mlp"]
+    for step in (0, 1, 511, 512, 513, 555, 599):
+        mlp.set_state(state["weights"])
+        first = mlp.train(step, batch=512, lr=2e-3, seed=1)
+        assert np.array_equal(first.astype(np.float32), loss[:step])
+        again = mlp.train(1, batch=512, lr=2e-3, seed=1)[0]
+        assert abs(again - loss[step]) <= 2e-5 * (1.0 + abs(again)), step
+    # a loss of the first download in the place of one of the second would not pass
+    assert np.abs(loss[512:] - loss[:88]).min() > 1e-3
