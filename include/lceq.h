@@ -57,7 +57,15 @@ typedef struct lceq_lattice lceq_lattice;
 /* ---- lifecycle -------------------------------------------------------- */
 /* Whole lattice lx*ly*lz on the current HIP device; extents even and >= 2
  * (f/topology.f:124-142).  Replaces initialize/topology/adresses
- * (f/initialize.f:35-45, f/adresses.f:18) for one device. */
+ * (f/initialize.f:35-45, f/adresses.f:18) for one device.
+ * Device memory: 348 bytes a site (links, their gauge-fixed copy and the staples
+ * 96 each, Higgs fields 24 each, force 12), and 96 more, a second link array,
+ * where link sweeps run three directions in one launch (up to about 44^3, and
+ * larger cached lattices of whole 16 x 4 x 4 tiles) and on other lattices from
+ * their first lceq_landau_gauge (without memory for it both run as they do without
+ * it).  Pinned host memory: 64 KiB a lattice, and up to 24 MiB for each field
+ * transfer under way, from a pool that keeps at most 121 MiB idle, and 26 MiB once
+ * no lattice or batch exists. */
 int lceq_create(int lx, int ly, int lz, lceq_lattice **out);
 int lceq_destroy(lceq_lattice *L);
 /* the extents lx, ly, lz of the lattice */
@@ -203,7 +211,9 @@ int lceq_u_f_renorm(lceq_lattice *L);
 int lceq_or_gauge_fixing(lceq_lattice *L, double *da1);
 /* landau_gauge(da1,iter_or1), f/landau_gauge.f:6 (called at f/main.f:62,74):
  * copies u->u_f, a->a_f and iterates or_gauge_fixing + u_f_renorm while
- * da1 > limit_or.  Returns LCEQ_ERR_NOT_CONVERGED if max_iter is reached. */
+ * da1 > limit_or.  Returns LCEQ_ERR_NOT_CONVERGED if max_iter is reached.
+ * or_gauge_fixing adds da1 in the same order, so that a loop over the two
+ * routines stops after the same iteration. */
 int lceq_landau_gauge(lceq_lattice *L, double *da1, int *iter_or1);
 /* correlator(meas,mstart), f/correlator.f:11 (called at f/meas2a.f:35):
  * the three z-correlators the reference writes (arrays of length lz); also

@@ -402,11 +402,6 @@ __device__ __forceinline__ void philox_pair(const Philox& key, uint32_t idx, uin
 
 // ------------------------------------------------------------ reductions
 
-// Deterministic in-block sum of NQ doubles (blockDim = 256 = 4 waves of 64):
-// xor-butterfly inside each wave, then the four wave totals in fixed order.
-// Every thread of the block receives the NQ totals.
-// Deterministic block sum over NW waves (fixed butterfly and combine order);
-// the result is left in every thread.
 // Sum of one value over a wave's 64 lanes, in every lane: partners 32, 16, 8,
 // 4, 2 and 1 lanes away in turn, the additions of a xor butterfly.  The partner's
 // value comes by lane swaps and row moves inside the vector unit (4 cycles)
@@ -441,27 +436,9 @@ __device__ __forceinline__ double wave_sum(double t) {
   return t;
 }
 
-template <int NQ, int NW = 4>
-__device__ __forceinline__ void block_sum(double (&v)[NQ]) {
-  __shared__ double red[NW][NQ];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) v[q] = wave_sum(v[q]);
-  int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) red[wv][q] = v[q];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    double t = red[0][q];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) t += red[w][q];
-    v[q] = t;
-  }
-  __syncthreads();
-}
-// the block's totals to out[q * stride + blk], one thread per quantity
+// Sums of NQ values over a block of NW waves, in a fixed order (each wave's
+// butterfly, then the waves in turn), to out[q * stride + blk]; one thread per
+// quantity stores.  Every thread of the block must call it.
 template <int NQ, int NW = 4>
 __device__ __forceinline__ void block_sum_store(double (&v)[NQ], double* __restrict__ out,
                                                 int stride, int blk) {

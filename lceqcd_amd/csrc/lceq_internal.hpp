@@ -178,11 +178,14 @@ void launch_link(lceq_lattice* L, int kp, int eo, int mu, int measflag, int reno
 // one launch: passes pass .. pass + 2, from the links `src` (of parity eo) and
 // `other` (of the other one) to `dst`, another array than `src`.  link3_tiles:
 // its blocks on lattices where it is the faster way, otherwise 0.
-// The launch runs as long as its fullest CU: a CU holds three blocks, and half
-// as many link updates again as the launches per direction have.  Those cost a
-// launch each, so that up to two blocks per CU are the faster way whatever the
-// tiles hold, and many rounds of whole tiles save their passes over memory; in
-// between, and where tiles are cut off, the extra updates cost more.  us per
+// Half as many link updates again as the launches per direction have, in a third of
+// the launches and with 168 bytes a site in place of 408.  Launches per direction
+// cost a launch each, so that up to two blocks per CU (512) this one is the faster
+// way whatever the tiles hold.  Then the sites count: it takes 0.72-0.74 ns a site
+// and sweep from 64^3 to 80x80x64 alike, launches per direction 0.61 as long as the
+// fields (31 MB at 64^3) are about the size of the L2s (32 MB), 0.71 at 39 MB
+// (64x64x80) and 0.82 at 49 MB (80x80x64, 1600 whole tiles), from where it stays the
+// faster way.  With tiles cut off, whose extra sites are more, it does not.  us per
 // production sweep of n_or = 4 (one of the five link sweeps is a measured one),
 // launches per direction and this one:
 //   16^3 (16 tiles) 114-127 89, 32^3 (128) 114-128 91, 44^3 (363) 129 123,

@@ -813,10 +813,16 @@ __device__ __forceinline__ TileSite tile_even_site(int e) {
 // too, and come out the same there, since src does not change).  Then each odd
 // site applies them to its links, takes its own rotation, and writes its links
 // normalised.  Both half steps as launches of their own read and write every
-// link: 768 bytes a site of the lattice and iteration, here about 480, and one
-// launch instead of two.  The arithmetic per site and link is k_gfix's.
-// What bounds it is the FP64 issue of 736 rotations for 512 sites on the
-// lattices the Infinity Cache holds, and the launch below 40^3.  An iteration in
+// link (432 bytes a site of the lattice and iteration with a_f), here once (240, and
+// the faces), and one launch instead of two.  The arithmetic per site and link is
+// k_gfix's.
+// What bounds it on lattices the Infinity Cache holds is the chain of a block: two
+// rounds of dependent gathers, the loop condition's flag and partials ahead of the
+// first, a barrier in each, with half the waves idle after the second.  Counters at
+// 64^3 (14.3 us): waves wait 43% of their cycles, the vector unit issues for 37% of
+// the launch (763 instructions a wave, half of them FP64), and 71 MB pass the L2s,
+// 5.0 TB/s (63 MB without the faces).  Beyond the cache HBM: 160^3 1.26 GB in 266 us,
+// 4.7 TB/s.  Below 40^3 the launch.  An iteration in
 // us, two launches and one: 8^3 8.6 6.4, 16^3 8.6 6.9, 32^3 9.4 7.4, 48^3 12.1
 // 9.1, 64^3 18.5 14.1, 96^3 56 43, 160^3 361 276; 4^3 (16 odd sites) even.
 // WT: links stored through the L2.  Beyond the Infinity Cache they are not: a

@@ -73,9 +73,12 @@ struct Link3Args {
   int n, nty, renorm;
 };
 
-// Bound by the vector unit and the L1 at nine wave-passes a tile (six without
-// the extra sites) and, below two blocks per CU, by one block's chain of three
-// passes: 5.8 us a launch at 16^3 against three launches of 3.8.  16 x 8 x 4
+// Below two blocks per CU what bounds it is one block's chain of three passes (5.8
+// us a launch at 16^3 against three launches of 3.8).  Counters at 96^3, nine
+// wave-passes a tile (six without the extra sites): the heatbath's launch (73.7 us)
+// issues vector instructions for 65% of its time; the overrelaxation's (49.0 us) for
+// 41%, and its waves, two per SIMD on average, wait for 40% of theirs; 200 MB pass the
+// L2s, 4.1 TB/s, where three launches per direction move 361 in 55.9 us.  16 x 8 x 4
 // tiles (8.3 extra wave-passes for 12) took 8.3 there and lost from 48^3 on;
 // four waves per SIMD (the operands not loaded ahead of the draws) is 4% slower
 // than three from 64^3 on.  The operands of a pass that the one before it does
