@@ -26,18 +26,31 @@ def lattice(*shape):
     L.rng_philox(5, 0)
     return L
 
+out = {}
+
+def trace(call):
+    # events of one call by name; of two calls, which whole traces show alike
+    seen = []
+    for _ in range(2):
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            call()
+            torch.cuda.synchronize()
+        counts = {}
+        for e in p.events():
+            counts[e.name] = counts.get(e.name, 0) + 1
+        seen.append(counts)
+    if seen[0] != seen[1]:
+        out["incomplete"] = True
+    return seen[0]
+
 def traced(L, call):
     call()
     L.sync()
-    with profile(activities=[ProfilerActivity.CUDA]) as p:
-        call()
-        L.sync()
-        torch.cuda.synchronize()
     counts = {}
-    for e in p.events():
-        k = re.search(r"\b(k_\w+)", e.name)
-        if k and "CUDA" in str(e.device_type):
-            counts[k.group(1)] = counts.get(k.group(1), 0) + 1
+    for name, n in trace(lambda: (call(), L.sync())).items():
+        k = re.search(r"\b(k_\w+)", name)
+        if k:
+            counts[k.group(1)] = counts.get(k.group(1), 0) + n
     return counts
 
 def timed(L, call):
@@ -46,7 +59,6 @@ def timed(L, call):
     L.profile_end()
 
 torch.zeros(1, device="cuda")
-out = {}
 for shape in ((16, 16, 16), (44, 44, 44)):
     print("tracing", shape, file=sys.stderr, flush=True)
     L = lattice(*shape)
@@ -75,13 +87,7 @@ def life():
 print("tracing allocations", file=sys.stderr, flush=True)
 keep = lattice(4, 4, 4)
 life()
-with profile(activities=[ProfilerActivity.CUDA]) as p:
-    for _ in range(3):
-        life()
-    torch.cuda.synchronize()
-out["life"] = {}
-for e in p.events():
-    out["life"][e.name] = out["life"].get(e.name, 0) + 1
+out["life"] = trace(lambda: [life() for _ in range(3)])
 print(json.dumps(out))
 """
 
@@ -90,12 +96,12 @@ print(json.dumps(out))
 def launches():
     print("device traces of launches", flush=True)
     r = subprocess.run([sys.executable, "-c", CHILD], cwd=ROOT, capture_output=True, text=True,
-                       timeout=110)
+                       timeout=170)
     assert r.returncode == 0, r.stderr[-2000:]
     out = json.loads(r.stdout.splitlines()[-1])
     print(out, flush=True)
-    if not any(out.values()):
-        pytest.skip("no device trace to be had")
+    if out.get("incomplete") or not any(out.values()):
+        pytest.skip("no whole device trace to be had")
     return out
 
 
